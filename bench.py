@@ -373,15 +373,15 @@ def main():
         head.set_guess(M.GUESS_LEARNED)
 
     def fresh(precision, guess=M.GUESS_PREVIOUS, prime=False, lds_fp64=False, with_net=False, tol=TOL):
-        # MOBYDIFF_LDS_SOR is read when a handle is created: 2 puts the FP64 batches on the
-        # LDS-resident kernel too
+        # MOBYDIFF_LDS_SOR is read when a handle is created: 2 (the default) runs the FP64 batches on
+        # the LDS-resident kernel, 1 on the streaming sweeps, the reference's kernel structure
         saved = os.environ.get("MOBYDIFF_LDS_SOR")
-        if lds_fp64:
-            os.environ["MOBYDIFF_LDS_SOR"] = "2"
+        if precision == M.PREC_FP64:
+            os.environ["MOBYDIFF_LDS_SOR"] = "2" if lds_fp64 else "1"
         try:
             ch = make_channel(M, precision, args.check_every, args.inner, tol)
         finally:
-            if lds_fp64:
+            if precision == M.PREC_FP64:
                 if saved is None:
                     del os.environ["MOBYDIFF_LDS_SOR"]
                 else:

@@ -765,6 +765,8 @@ extern "C" int mdx_apply_bc_redblack(mdx_handle *h) {
 // gave up.  The batch drained, but its iterate and residual are not trustworthy; the SOR solve that
 // saw it restarts on the streaming sweeps.
 static constexpr int MDX_LDS_TIMEOUT = 100;
+// Internal: a batch to be queued ahead of its input check could not run on the LDS-resident solver.
+static constexpr int MDX_LDS_REFUSED = 101;
 // restarts after which the LDS-resident solver stays off for the handle
 static constexpr int LDS_TIMEOUT_MAX = 3;
 
@@ -798,8 +800,34 @@ static int read_norm(mdx_handle *h, double *out) {
     return rc == MDX_LDS_TIMEOUT ? MDX_OK : rc;
 }
 
-// Plan and allocate the LDS-resident solver once the IBM state is known (uniform grid, z-invariant
-// or absent IBM coefficients); rb_state = -1 leaves the streaming sweeps in charge.
+// The LDS-resident solver's workgroups wait for each other, so two of its batches that share the
+// device's CUs could hold each other up until their waits give up.  A device has one turn: a solve
+// (or an mdx_step_batch call, for all of its handles, whose plans share the CUs out) that finds it
+// taken by another thread runs on the streaming sweeps, which give the same bits.  When a turn
+// ends no batch of it still waits: the last check has been read, and a batch queued behind it
+// finds it converged and returns.
+static constexpr int LDS_MAX_DEVICES = 64;
+static std::atomic<bool> g_lds_turn[LDS_MAX_DEVICES];
+
+class LdsTurn {
+    int dev_ = -1;
+
+public:
+    LdsTurn() = default;
+    LdsTurn(const LdsTurn &) = delete;
+    LdsTurn &operator=(const LdsTurn &) = delete;
+    bool take(int dev) {
+        if (dev < 0 || dev >= LDS_MAX_DEVICES || g_lds_turn[dev].exchange(true, std::memory_order_acquire)) return false;
+        dev_ = dev;
+        return true;
+    }
+    ~LdsTurn() {
+        if (dev_ >= 0) g_lds_turn[dev_].store(false, std::memory_order_release);
+    }
+};
+
+// Plan and allocate the LDS-resident solver once the IBM state is known (z-invariant or absent IBM
+// coefficients); rb_state = -1 leaves the streaming sweeps in charge.
 static int rb_prepare(mdx_handle *h) {
     if (h->rb_state != 0) return MDX_OK;
     h->rb_state = -1;
@@ -809,7 +837,6 @@ static int rb_prepare(mdx_handle *h) {
         if (h->sweep_fused) h->rb_note = "fused red+black iterations: 32x8x8 tiles with a two-cell halo in LDS";
         return MDX_OK;
     }
-    if (h->stretched) { h->rb_note = "streaming sweeps: stretched grid"; return MDX_OK; }
     if (h->ibm_on && !h->coef_plane) { h->rb_note = "streaming sweeps: IBM coefficients vary in z"; return MDX_OK; }
     RbPlanOut p64{}, p32{};
     std::string why;
@@ -976,6 +1003,8 @@ static int sweep_batch(mdx_handle *h, bool fp32, int m, const RbDefect *df = nul
             h->rb_state = -1;
             h->rb_note = std::string("streaming sweeps: LDS-resident launch refused (") + hipGetErrorString(e) + ")";
             if (fp32) MDX_HIP(launch_zero32(h, h->e32, h->ni));   // the streaming sweeps start from e = 0
+            // the streaming FP64 sweeps change Phi whatever the pending check says
+            else if (df && df->skip) return MDX_LDS_REFUSED;
         }
     }
     if (lds_for(h, fp32)) {
@@ -1001,10 +1030,12 @@ static int sweep_batch(mdx_handle *h, bool fp32, int m, const RbDefect *df = nul
         MDX_HIP(sweep_launches(h, fp32, m));
     }
     if (!launches) launches = (h->sweep_fused ? 1 : 2) * m;   // streaming: one launch per colour
-    // a batch that should have ended with the LDS defect epilogue but ran on the streaming sweeps
-    // (launch refused): the separate defect kernel forms the same check
-    if (df && !lds_for(h, fp32))
-        MDX_HIP(launch_defect64(h, df->phi_in, h->e32, df->phi_out, h->r32, df->host_slot, df->seq));
+    // a batch that should have ended with the LDS check epilogue but ran on the streaming sweeps
+    // (launch refused): the separate kernel forms the same check
+    if (df && !lds_for(h, fp32)) {
+        if (fp32) MDX_HIP(launch_defect64(h, df->phi_in, h->e32, df->phi_out, h->r32, df->host_slot, df->seq));
+        else MDX_HIP(launch_sor_residual64(h, h->phi, df->host_slot, df->seq));
+    }
     h->sw_last = qs;
     if (qs >= 0) {
         MDX_HIP(hipEventRecord(h->ev_sw[qs][1], h->stream));
@@ -1015,38 +1046,7 @@ static int sweep_batch(mdx_handle *h, bool fp32, int m, const RbDefect *df = nul
     return MDX_OK;
 }
 
-// Plain FP64 red-black SOR to ||div||_inf < tol; Phi starts at zero (the previous-step pressure).
-// r_first >= 0: the residual of the initial iterate is already known (learned-guess selection).
-static int sor_solve64(mdx_handle *h, mdx_solve_stats *st, double r_first) {
-    const mdx_config &c = h->cfg;
-    double r = 0.0;
-    int it = 0, checks = 0;
-    for (;;) {
-        int rc;
-        if (checks == 0 && r_first >= 0.0) {
-            r = r_first;
-        } else {
-            MDX_HIP(launch_reset_max(h));
-            MDX_HIP(launch_sor_residual64(h, h->phi));
-            if ((rc = read_max(h, &r))) return rc;
-        }
-        sweep_account(h);
-        if (checks == 0) st->div0_inf = r;
-        ++checks;
-        if (!(r >= c.tol) || it >= c.max_iter) break;   // NaN stops too and is reported below
-        const int m = std::min(c.check_every, c.max_iter - it);
-        if ((rc = sweep_batch(h, false, m))) return rc;
-        it += m;
-    }
-    st->iterations = it;
-    st->checks = checks;
-    st->div_inf = r;
-    st->converged = r < c.tol;
-    st->lds_sweeps = lds_for(h, false);
-    return MDX_OK;
-}
-
-// pinned words of the mixed solve's two check slots: [CHECK_PIN + 4 * slot] = max, error word, seq
+// pinned words of a solve's two check slots: [CHECK_PIN + 4 * slot] = max, error word, seq
 static constexpr int CHECK_PIN = 16;
 // pinned words of the learned start's comparison, each [max, error word, seq]: the residual of
 // Phi_0 (RP), max |rhs| (RZ: the residual of Phi = 0) and the learned start's first check (SEL)
@@ -1079,6 +1079,76 @@ static int wait_check(mdx_handle *h, int w, unsigned long long seq, double *r) {
     int err;
     std::memcpy(&err, &h->h_pinned[w + 1], sizeof err);
     if (err) return lds_timeout_seen(h);
+    return MDX_OK;
+}
+
+// Plain FP64 red-black SOR to ||div||_inf < tol; Phi starts at zero (the previous-step pressure).
+// r_first >= 0: the residual of the initial iterate is already known (learned-guess selection).
+static int sor_solve64(mdx_handle *h, mdx_solve_stats *st, double r_first) {
+    const mdx_config &c = h->cfg;
+    double r = 0.0;
+    int it = 0, checks = 0;
+    // On the LDS-resident solver a batch forms the check that follows it, and the next batch is
+    // queued before that check is read: it reads the maximum on the GPU and leaves Phi as it is when
+    // the solve has converged, so the GPU never waits for the host inside a solve.
+    const bool lds = lds_for(h, false);
+    int slot = 0;
+    unsigned long long seq[2] = {0, 0};
+    auto enqueue = [&](int m, int sl, int skip) -> int {
+        seq[sl] = ++h->chk_seq;
+        const RbDefect df{nullptr, h->phi, h->d_pinned + CHECK_PIN + 4 * sl, seq[sl], skip, c.tol};
+        return sweep_batch(h, false, m, &df);
+    };
+    for (;;) {
+        int rc;
+        if (lds) {
+            const int m = std::min(c.check_every, c.max_iter - it);
+            bool ahead = m > 0 && lds_for(h, false);
+            if (checks == 0 && r_first >= 0.0) {
+                r = r_first;
+                ahead = false;   // this maximum is not the one the device holds
+            } else {
+                if (checks == 0) {
+                    seq[slot] = ++h->chk_seq;
+                    MDX_HIP(launch_sor_residual64(h, h->phi, h->d_pinned + CHECK_PIN + 4 * slot, seq[slot]));
+                }
+                if (ahead && (rc = enqueue(m, slot ^ 1, 1))) {
+                    if (rc != MDX_LDS_REFUSED) return rc;
+                    ahead = false;
+                }
+                if ((rc = wait_check(h, CHECK_PIN + 4 * slot, seq[slot], &r))) return rc;
+            }
+            const bool done = !(r >= c.tol) || it >= c.max_iter;
+            if (done && ahead && lds_for(h, false) && h->sw_last >= 0) h->sw_void[h->sw_last] = true;
+            sweep_account(h);
+            if (checks == 0) st->div0_inf = r;
+            ++checks;
+            if (done) break;
+            if (!ahead && (rc = enqueue(m, slot ^ 1, 0))) return rc;
+            it += m;
+            slot ^= 1;
+            continue;
+        }
+        if (checks == 0 && r_first >= 0.0) {
+            r = r_first;
+        } else {
+            MDX_HIP(launch_reset_max(h));
+            MDX_HIP(launch_sor_residual64(h, h->phi));
+            if ((rc = read_max(h, &r))) return rc;
+        }
+        sweep_account(h);
+        if (checks == 0) st->div0_inf = r;
+        ++checks;
+        if (!(r >= c.tol) || it >= c.max_iter) break;   // NaN stops too and is reported below
+        const int m = std::min(c.check_every, c.max_iter - it);
+        if ((rc = sweep_batch(h, false, m))) return rc;
+        it += m;
+    }
+    st->iterations = it;
+    st->checks = checks;
+    st->div_inf = r;
+    st->converged = r < c.tol;
+    st->lds_sweeps = lds_for(h, false);
     return MDX_OK;
 }
 
@@ -1522,6 +1592,8 @@ extern "C" int mdx_pressure_projection(mdx_handle *h, double dtg, mdx_solve_stat
         int rc = ensure_mu(h, dtg);
         if (rc) return rc;
         if ((rc = rb_prepare(h))) return rc;
+        LdsTurn turn;   // held until this solve has read its last check
+        h->lds_suspended = h->rb_state == 1 && (h->in_batch ? !h->batch_lds : !turn.take(h->device));
         double r_first = -1.0;
         const int stage = (int)(h->proj_count % 3);
         const auto t_plan = std::chrono::steady_clock::now();
@@ -1774,7 +1846,8 @@ extern "C" int mdx_set_step_report(mdx_handle *h, int32_t bulk_velocity) {
 // seeds) stepped concurrently: one host thread per handle drives that handle's own stream, so the
 // GPU overlaps the instances' kernels and each instance's residual checks wait only on its own
 // work.  Each instance computes exactly what mdx_step computes for it alone.  The LDS-resident
-// sweeps need every CU for one launch and are switched off for batched handles.
+// sweeps of a batched handle are planned on an equal share of the CUs, so the batches of all
+// instances are resident together; a grid too large for its share runs on the streaming sweeps.
 extern "C" int mdx_step_batch(mdx_handle *const *hs, int32_t n, double dt, mdx_step_stats *stats) {
     MDX_CHECK(hs && n > 0, MDX_ERR_ARG, "mdx_step_batch: need n > 0 handles");
     for (int q = 0; q < n; ++q) {
@@ -1786,13 +1859,24 @@ extern "C" int mdx_step_batch(mdx_handle *const *hs, int32_t n, double dt, mdx_s
                       "mdx_step_batch: two handles share one attached network");
         }
     }
+    std::vector<LdsTurn> turns(n);
     for (int q = 0; q < n; ++q) {
         mdx_handle *h = hs[q];
-        if (h->lds_sor_mode != 0) {
-            h->lds_sor_mode = 0;
-            h->rb_state = -1;
-            h->rb_note = "streaming sweeps: concurrent batch";
+        int cus = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) {
+            (void)hipGetLastError();
+            cus = 0;   // no share: the streaming sweeps
         }
+        const int share = cus / n;
+        if (h->rb_cus == 0 || h->rb_cus > std::max(1, share)) {
+            h->rb_cus = std::max(1, share);
+            h->rb_state = 0;   // planned again on its share
+        }
+        int first = q;   // the handle that took (or failed to take) the turn of this device
+        for (int r = 0; r < q; ++r)
+            if (hs[r]->device == h->device) { first = r; break; }
+        h->in_batch = true;
+        h->batch_lds = share > 0 && (first < q ? hs[first]->batch_lds : turns[q].take(h->device));
     }
     std::vector<int> rc(n, MDX_OK);
     std::vector<std::string> err(n);
@@ -1809,6 +1893,7 @@ extern "C" int mdx_step_batch(mdx_handle *const *hs, int32_t n, double dt, mdx_s
             if (rc[q]) err[q] = mdx_last_error();
         });
     for (auto &t : th) t.join();
+    for (int q = 0; q < n; ++q) hs[q]->in_batch = false;
     for (int q = 0; q < n; ++q)
         if (rc[q]) {
             mdx_set_error("mdx_step_batch: instance " + std::to_string(q) + ": " + err[q]);

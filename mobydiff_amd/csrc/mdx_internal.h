@@ -221,9 +221,10 @@ struct mdx_handle {
     // one launch per red+black iteration (halo-recomputing tiles) instead of one per colour
     bool sweep_fused = false;
 
-    // LDS-resident red-black solver (MOBYDIFF_LDS_SOR): 0 off, 1 FP32 sweep batches (the default),
-    // 2 FP32 and FP64 batches; plans per precision and the tagged face buffers
-    int lds_sor_mode = 1;
+    // LDS-resident red-black solver (MOBYDIFF_LDS_SOR): 0 off, 1 FP32 sweep batches, 2 FP32 and FP64
+    // batches (the default); plans per precision and the tagged face buffers
+    int lds_sor_mode = 2;
+    int rb_cus = 0;                // CUs the plan may hold (0: all of the device's)
     // launch the LDS-resident kernel through hipLaunchCooperativeKernel (MOBYDIFF_LDS_COOP=1)
     // instead of an ordinary launch of a grid that the plan already sized to be co-resident
     bool rb_coop = false;
@@ -253,6 +254,9 @@ struct mdx_handle {
     int rb_spin_limit = 1 << 20;
     int lds_timeouts = 0;
     bool lds_suspended = false;
+    // the handle is being stepped by mdx_step_batch, which holds the device's LDS turn for all of
+    // its handles (or, with batch_lds false, could not take it)
+    bool in_batch = false, batch_lds = false;
     mdx::RbPlanOut rb_plan64{}, rb_plan32{};
     void *rb_faces = nullptr;      // tagged face words of the LDS-resident sweeps
     int *rb_xl32 = nullptr, *rb_xl64 = nullptr;   // exchange lists of the two plans
@@ -350,7 +354,8 @@ hipError_t launch_sor_prepare(mdx_handle *h, double *rhs_max_slot = nullptr, uns
 hipError_t launch_sor_start(mdx_handle *h, const double *prev, double fac, double *host_slot,
                             unsigned long long seq);
 hipError_t launch_sor_sweep64(mdx_handle *h, int color, double omega);
-hipError_t launch_sor_residual64(mdx_handle *h, const double *phi);
+hipError_t launch_sor_residual64(mdx_handle *h, const double *phi, double *host_slot = nullptr,
+                                 unsigned long long seq = 0);
 // the projection; with hist != nullptr Phi is also copied there (the stage's history)
 // (inside a step: sets h->apply_wrote_bc, whether the launch also wrote the boundary conditions)
 hipError_t launch_sor_apply(mdx_handle *h, const double *phi, double dtg, double *hist = nullptr);
@@ -365,7 +370,8 @@ hipError_t launch_sor_iters32(mdx_handle *h, int m, float omega);
 hipError_t launch_zero32(mdx_handle *h, float *p, size_t n);
 hipError_t launch_zero64(mdx_handle *h, double *p, size_t n);
 hipError_t launch_scale_copy64(mdx_handle *h, double *dst, const double *src, double fac, size_t n);
-hipError_t launch_residual_field64(mdx_handle *h, const double *phi, double *field, double *host_slot = nullptr);
+hipError_t launch_residual_field64(mdx_handle *h, const double *phi, double *field, double *host_slot = nullptr,
+                                   unsigned long long seq = 0);
 hipError_t launch_phi0_residual(mdx_handle *h, const double *prev, double fac, double *phi0, double *res,
                                 double *host_slot, double *stat);
 // the learned start's input pass fused with the right-hand side (learned_input_kernel): rhs, r0 and
@@ -379,7 +385,8 @@ hipError_t launch_learned_input(mdx_handle *h, const double *prev, double fac, d
 hipError_t launch_select_start(mdx_handle *h, double margin, unsigned nb, double *rg_slot, const double *other_slot,
                                const double *phi0, const double *res0, double *host_slot, unsigned long long seq);
 bool rb_plan(const mdx_handle *h, bool fp32, RbPlanOut &out, std::string &why);
-// defect epilogue of an FP32 LDS batch: phi_out = phi_in + e, r32 = defect, max_part = its maxima
+// check epilogue of an LDS batch: FP32 phi_out = phi_in + e, r32 = defect; FP64 phi_out = the iterate
+// (phi_in unused); the maximum to the slot
 struct RbDefect {
     const double *phi_in;
     double *phi_out;

@@ -995,7 +995,8 @@ __global__ __launch_bounds__(256) void sor_residual64_kernel(GridK g, MuK<double
 
 // max |rhs - L_mu(phi)| into red_max (and host_slot); with field != nullptr the residual itself is
 // stored too
-hipError_t launch_residual_field64(mdx_handle *h, const double *phi, double *field, double *host_slot) {
+hipError_t launch_residual_field64(mdx_handle *h, const double *phi, double *field, double *host_slot,
+                                   unsigned long long seq) {
     GridK g = grid_k(h);
     MuK<double> mu = mu_k<double>(h, h->mu64);
     SorConst<double> s{1.0 / h->dx * (1.0 / h->dx), 1.0 / h->dy * (1.0 / h->dy), 1.0 / h->dz * (1.0 / h->dz)};
@@ -1006,11 +1007,11 @@ hipError_t launch_residual_field64(mdx_handle *h, const double *phi, double *fie
     else { if (h->ibm_on) MDX_RS(false, true); else MDX_RS(false, false); }
 #undef MDX_RS
     hipError_t e = hipGetLastError();
-    return e != hipSuccess ? e : launch_max_final(h, grd.x, host_slot, 0);
+    return e != hipSuccess ? e : launch_max_final(h, grd.x, host_slot, seq);
 }
 
-hipError_t launch_sor_residual64(mdx_handle *h, const double *phi) {
-    return launch_residual_field64(h, phi, nullptr, nullptr);
+hipError_t launch_sor_residual64(mdx_handle *h, const double *phi, double *host_slot, unsigned long long seq) {
+    return launch_residual_field64(h, phi, nullptr, host_slot, seq);
 }
 
 // fac * Phi of one cell: the value the previous-Phi copy (scale_copy_kernel) stores

@@ -240,7 +240,7 @@ static void free_all(mdx_handle *h) {
                     h->red_part, h->red_max, h->max_part, h->rb_faces, h->phi_hist, h->res64,
                     h->fft_phi, h->fft_res, h->fft_mean, h->hat32, h->cp32, h->den32, h->arow32, h->tw_x32,
                     h->tw_z32, h->rb_xl32, h->rb_xl64, h->cvel, h->lamx, h->lamz, h->tw_a, h->bdrow, h->crow, h->lamx32, h->lamz32,
-                    h->tw_a32, h->bdrow32, h->crow32, h->fr_part};
+                    h->tw_a32, h->bdrow32, h->crow32, h->fr_part, h->sola_tmp};
     for (auto &s : h->graphs)
         if (s.exec) (void)hipGraphExecDestroy(s.exec);
     for (void *p : ptrs)
@@ -424,6 +424,8 @@ extern "C" int mdx_create(const mdx_config *cfg, mdx_handle **out) {
         if ((e = dalloc(&h->phi_hist, 3 * h->ni)) != hipSuccess || (e = dalloc(&h->res64, h->ni)) != hipSuccess)
             return fail(e, "SOR guess history");
     }
+    if (cfg->solver == MDX_SOLVER_SOLA && (e = dalloc(&h->sola_tmp, 3 * h->ng)) != hipSuccess)
+        return fail(e, "SOLA buffers");
     if (cfg->solver == MDX_SOLVER_FFT) {
         const int nxh = nx / 2 + 1;
         const size_t nh = (size_t)nxh * ny * nz;
@@ -1579,11 +1581,15 @@ extern "C" int mdx_pressure_projection(mdx_handle *h, double dtg, mdx_solve_stat
     } else if (c.solver == MDX_SOLVER_SOLA) {
         ev_record(h, 1);
         const size_t bytes = h->ng * 8;
-        MDX_HIP(hipMemcpyAsync(h->un, h->us, bytes, hipMemcpyDeviceToDevice, h->stream));
-        MDX_HIP(hipMemcpyAsync(h->vn, h->vs, bytes, hipMemcpyDeviceToDevice, h->stream));
-        MDX_HIP(hipMemcpyAsync(h->wn, h->ws, bytes, hipMemcpyDeviceToDevice, h->stream));
-        for (int it = 0; it < c.niter; ++it)
-            for (int parity = 0; parity <= 1; ++parity) MDX_HIP(launch_sola_sweep(h, parity, c.omega, dtg));
+        if (sola_fused_fits(h)) {
+            MDX_HIP(launch_sola(h, dtg));
+        } else {
+            MDX_HIP(hipMemcpyAsync(h->un, h->us, bytes, hipMemcpyDeviceToDevice, h->stream));
+            MDX_HIP(hipMemcpyAsync(h->vn, h->vs, bytes, hipMemcpyDeviceToDevice, h->stream));
+            MDX_HIP(hipMemcpyAsync(h->wn, h->ws, bytes, hipMemcpyDeviceToDevice, h->stream));
+            for (int it = 0; it < c.niter; ++it)
+                for (int parity = 0; parity <= 1; ++parity) MDX_HIP(launch_sola_sweep(h, parity, c.omega, dtg));
+        }
         ev_record(h, 2);
         ev_record(h, 3);
         st.iterations = c.niter;

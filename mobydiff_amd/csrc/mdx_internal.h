@@ -150,6 +150,8 @@ struct mdx_handle {
     float *mu32[3] = {nullptr, nullptr, nullptr};
     double mu_dtg = -1.0;          // dt_gamma the mu tables were built for
 
+    double *sola_tmp = nullptr;    // SOLA: u, v, w between iterations (three ghosted arrays)
+
     // FFT path
     double *fft_rhs = nullptr, *hat = nullptr, *cp = nullptr, *den_inv = nullptr, *arow = nullptr;
     double *tw_x = nullptr, *tw_z = nullptr;
@@ -346,6 +348,10 @@ static constexpr unsigned MAX_PARTS = 1u << 17;
 
 // red-black solver
 hipError_t launch_sola_sweep(mdx_handle *h, int parity, double sor, double dtg);
+// all SOLA iterations of a projection, one launch each, from u* (inside a step the last one also
+// writes the boundary conditions and sets h->apply_wrote_bc); whether the configuration allows it
+bool sola_fused_fits(const mdx_handle *h);
+hipError_t launch_sola(mdx_handle *h, double dtg);
 hipError_t launch_build_mu(mdx_handle *h, double dtg);
 // the stage's tables for launch_build_mu's work (n = 0 without IBM)
 MuBuild mu_build(const mdx_handle *h, double dtg);

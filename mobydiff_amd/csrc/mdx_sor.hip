@@ -7,6 +7,9 @@
 //    residual of a cell is div(u*) - L_mu(Phi), the relaxation denominator is the reference's
 //    (wall faces included), so the iterates equal the SOLA iterates.  FP64 for the plain solve;
 //    FP32 sweeps on the defect equation inside an FP64 defect-correction loop for the mixed solve.
+#include <algorithm>
+#include <type_traits>
+
 #include "mdx_sor_core.h"
 
 namespace mdx {
@@ -297,9 +300,10 @@ hipError_t launch_sor_start(mdx_handle *h, const double *prev, double fac, doubl
 // the faces, and edges and corners keep the u* values.  Thread `first` of `stride` threads.
 // bc_faces: the projection's tiles write the faces the boundary conditions set (the interiors of
 // the x and z faces, u and w on the interiors of the y faces), and they are left to them.
+// own_top: they also write v on the interior of the j = ny + 1 plane.
 __device__ inline void proj_ghost(const Dims &d, int walled_y, double vtop, bool bc_faces, const double *__restrict__ us,
                                   const double *__restrict__ vs, const double *__restrict__ ws, double *un,
-                                  double *vn, double *wn, long long first, long long stride) {
+                                  double *vn, double *wn, long long first, long long stride, bool own_top = false) {
     const long long sz = d.nz + 2;
     const long long pa = (long long)d.sx * d.sy, pb = (long long)d.sx * d.nz, pc = (long long)d.ny * d.nz;
     const long long n = 2 * (pa + pb + pc);
@@ -331,7 +335,7 @@ __device__ inline void proj_ghost(const Dims &d, int walled_y, double vtop, bool
             wn[c] = ws[c];
         }
         const bool top = walled_y && j == d.ny + 1 && in_i && in_k;
-        vn[c] = top ? vtop : vs[c];
+        if (!(top && own_top)) vn[c] = top ? vtop : vs[c];
     }
 }
 
@@ -354,6 +358,313 @@ hipError_t launch_sor_prepare(mdx_handle *h, double *rhs_max_slot, unsigned long
 }
 
 static constexpr unsigned PROJ_GHOST_BLOCKS = 256;
+
+// ------------------------------------------------------------------------------- SOLA, one launch per iteration
+// Both colours of one SOLA iteration (sola_sweep_kernel's statements, in their order) in one pass
+// from (u, v, w) to another set of arrays; p is updated in place (only its own cell reads it).
+// A sweep is memory-bound: it reads and writes u, v, w, p once per colour, and the copies u = u*
+// before the first one as well.  Here an iteration reads and writes them once, and the first one
+// reads u* itself.  Every face has one neighbour of each colour, so its value after the red pass is
+// u -+ phi_red h mu and after the black pass that plus its black neighbour's term; the kernel
+// therefore only passes phi between cells.  A workgroup of SL_X x TYE threads owns SL_X - 2 x-pairs
+// by TYE - 3 rows and marches kz planes: a thread holds the pair (i0, i0 + 1) of its row, of which
+// exactly one cell per plane is red.  Per plane k: phi_red of plane k + 1 (its faces are loaded here
+// and kept in registers for plane k + 1's turn) goes to LDS; then phi_black of plane k from the faces
+// its six red neighbours have changed; then the final values of plane k's faces, which need the
+// phi of the cell and of its west, south and lower neighbours.  The pair to the west and the two
+// rows below, the pair to the east and the row above, two planes below and one above are recomputed
+// by every workgroup that needs them, from the same inputs: bit-identical to the one-colour sweeps.
+// x and z periodic, Dirichlet v on the y walls (or periodic y, ny even), z-invariant coefficients
+// or none.  200^3, three iterations: 1314 us of sweeps and 77 us of copies -> 480 us (3.1 TB/s of the
+// 64 B per cell and iteration; a plane's two barriers and FP64 chain leave the CUs' one or two
+// workgroups waiting, and 200 VGPRs allow no more).  32 x 24 x 16: 42 -> 21 us.
+// last: 0 an iteration whose result another one reads, 1 the last one (its ghost blocks fill the
+// ghost shell of un, vn, wn with u*'s values), 2 the last one inside a step: it also writes the
+// boundary conditions (as sor_apply_kernel with BC).
+static constexpr int SL_X = 16;
+
+struct SolaWalls {   // p type and value at the y walls, wall values of v, twice the wall u and w
+    int pt[2];
+    double pv[2], v[2], u2[2], w2[2];
+};
+
+template <bool IBM, int TYE>
+__global__ __launch_bounds__(SL_X * TYE) void sola_iter_kernel(
+    GridK g, SolaWalls wl, double sor, double dtg, double idx, double idy, double idz, double idx2, double idy2,
+    double idz2, double idt, const double *__restrict__ cu, const double *__restrict__ cv,
+    const double *__restrict__ cw, const double *__restrict__ su, const double *__restrict__ sv,
+    const double *__restrict__ sw, double *__restrict__ du, double *__restrict__ dv, double *__restrict__ dw,
+    double *__restrict__ pn, const double *__restrict__ us, const double *__restrict__ vs,
+    const double *__restrict__ ws, int kz, unsigned tiles, int last) {
+    constexpr int PX = SL_X - 2, PY = TYE - 3, RW = 2 * SL_X;
+    __shared__ double F[3][TYE][RW];   // phi of planes k-1, k, k+1 (plane k in slot k mod 3)
+    const Dims d = g.d;
+    const bool per2 = g.per[1];
+    const int lx = threadIdx.x, ly = threadIdx.y;
+    if (blockIdx.x >= tiles) {   // the ghost shell keeps u*'s values
+        proj_ghost(d, per2 ? 0 : 1, 0.0, last == 2, us, vs, ws, du, dv, dw,
+                   (long long)(blockIdx.x - tiles) * (SL_X * TYE) + lx + SL_X * ly,
+                   (long long)(gridDim.x - tiles) * (SL_X * TYE), true);
+        return;
+    }
+    const int np = d.nx / 2, nseg = (d.nz + kz - 1) / kz;
+    int tx_, ty_, tz_;
+    if (!xcd_tile(np, d.ny, nseg, PX, PY, tx_, ty_, tz_)) return;   // uniform per workgroup
+    const int pr = tx_ * PX - 1 + lx, jr = ty_ * PY - 1 + ly;   // unwrapped pair (0-based) and row (1-based)
+    const int p = ((pr % np) + np) % np;
+    const int j = per2 ? ((jr - 1) % d.ny + d.ny) % d.ny + 1 : jr;
+    const bool row = j >= 1 && j <= d.ny;   // rows beyond a wall hold no cells
+    const int k0 = tz_ * kz + 1, k1 = k0 + kz - 1 < d.nz ? k0 + kz - 1 : d.nz;
+    const int i0 = 2 * p + 1;
+    const int jp = (per2 && j == d.ny) ? 1 : j + 1;
+    const bool bot = !per2 && j == 1, top = !per2 && j == d.ny;
+    const bool own = row && lx >= 1 && lx <= PX && ly >= 2 && ly <= TYE - 2 && pr < np && jr <= d.ny;
+    // The pair's cells by colour, so that no plane selects: cell 0 is the red one of plane k0 - 2, of
+    // k0, k0 + 2, ..., cell 1 the red one of the planes between (every extent a colour wraps around
+    // is even).  Per cell: its coefficients and the byte offsets of its faces in a plane; a load is a
+    // plane's uniform base and one of these.
+    const int e = (j + k0) & 1;
+    double mul[2], muh[2], mvl[2], mvh[2], mw[2], q[2];   // west, east, south, north, z faces; -omega / denom
+    unsigned ol[2], oh[2], on[2];                         // cell (its west, south and lower faces), east, north face
+    int x[2];                                             // index in F
+    bool blk[2];                                          // phi_black of this cell is needed by an owned face
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int f = c ? 1 - e : e, i = i0 + f, ih = i == d.nx ? 1 : i + 1, jj = row ? j : 1;
+        mul[c] = muh[c] = mvl[c] = mvh[c] = mw[c] = 1.0;
+        if (IBM && row) {
+            auto m = [&](const double *a, int ii, int jx) { return 1.0 / (1.0 + dtg * a[d.g(ii, jx, 1)]); };
+            mul[c] = m(cu, i, j);
+            muh[c] = m(cu, ih, j);
+            mvl[c] = m(cv, i, j);
+            mvh[c] = m(cv, i, jp);
+            mw[c] = m(cw, i, j);
+        }
+        const double denom = (mul[c] + muh[c]) * idx2 + (mw[c] + mw[c]) * idz2 + (mvl[c] + mvh[c]) * idy2;
+        q[c] = -sor / denom;
+        ol[c] = 8u * (unsigned)(i + d.sx * jj);
+        oh[c] = 8u * (unsigned)(ih + d.sx * jj);
+        on[c] = 8u * (unsigned)(i + d.sx * (row ? jp : 1));
+        x[c] = 2 * lx + f;
+        blk[c] = row && ly >= 1 && ly <= TYE - 2 && lx <= SL_X - 2 && (lx >= 1 || f == 1);
+    }
+    const size_t ps = (size_t)d.sx * d.sy;
+    auto kw = [&](int k) { return k < 1 ? k + d.nz : (k > d.nz ? k - d.nz : k); };   // -1 .. nz + 2
+    auto at = [&](const double *a, int k, unsigned o) -> double {
+        return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(a + ps * (size_t)k) + o);
+    };
+    auto put = [&](double *a, int k, unsigned o, double v) {
+        *reinterpret_cast<double *>(reinterpret_cast<char *>(a + ps * (size_t)k) + o) = v;
+    };
+    // old face values of the two cells in one plane.  The loads of a plane are issued one plane before
+    // their use (w, which the red pass needs one plane early, two; p too: loads return in order, so
+    // waiting for one of this plane's would wait for the next plane's as well).
+    struct Plane {
+        double ul[2], uh[2], vl[2], vh[2], w[2];
+    };
+    auto load = [&](Plane &f, int k) {   // all but w
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            f.ul[c] = at(su, k, ol[c]);
+            f.uh[c] = at(su, k, oh[c]);
+            f.vl[c] = bot ? wl.v[0] : at(sv, k, ol[c]);
+            f.vh[c] = top ? wl.v[1] : at(sv, k, on[c]);
+        }
+    };
+    Plane cur{}, nxt{}, pre{};           // planes k, k + 1, k + 2 (pre.w: w of plane k + 2)
+    double w3[2] = {0.0, 0.0};           // w of plane k + 3
+    double fk[2] = {0.0, 0.0};           // phi of the two cells in plane k - 1
+    double pp[2] = {0.0, 0.0};           // p of the two cells in plane k + 1
+    if (row) {
+        load(pre, kw(k0 - 2));
+        for (int c = 0; c < 2; ++c) {
+            pre.w[c] = at(sw, kw(k0 - 2), ol[c]);
+            w3[c] = at(sw, kw(k0 - 1), ol[c]);
+        }
+    }
+    int sl = (k0 + 3) % 3;               // LDS slot of plane k
+    // one plane; r: the cell that is red in plane k, b the black one
+    auto plane = [&](int k, auto r_) {
+        constexpr int r = decltype(r_)::value, b = 1 - r;
+        // the offsets are loop-invariant: left visible, their 64-bit sums with every array's base
+        // would be kept in registers instead of being formed by the loads (scalar base + offset)
+        asm volatile("" : "+v"(ol[0]), "+v"(ol[1]), "+v"(oh[0]), "+v"(oh[1]), "+v"(on[0]), "+v"(on[1]));
+        const int sp = sl == 2 ? 0 : sl + 1, sm = sl == 0 ? 2 : sl - 1;   // slots of k+1, k-1
+        const double po[2] = {pp[0], pp[1]};
+        // ---- phi_red of plane k + 1 (there cell b is the red one)
+        cur = nxt;
+        nxt = pre;
+        const double w2[2] = {w3[0], w3[1]};
+        if (row) {
+            if (k < k1) {
+                load(pre, kw(k + 2));
+                const int k3 = kw(k + 3);
+                w3[0] = at(sw, k3, ol[0]);
+                w3[1] = at(sw, k3, ol[1]);
+                if (own && k >= k0 - 1) {
+                    pp[0] = at(pn, k + 1, ol[0]);
+                    pp[1] = at(pn, k + 1, ol[1]);
+                }
+            }
+            F[sp][ly][x[b]] = ((nxt.uh[b] - nxt.ul[b]) * idx + (nxt.vh[b] - nxt.vl[b]) * idy + (w2[b] - nxt.w[b]) * idz) * q[b];
+        }
+        pre.w[0] = w2[0];
+        pre.w[1] = w2[1];
+        __syncthreads();
+        if (k >= k0 - 1) {
+            // ---- phi_black of plane k, from the faces the red neighbours have changed
+            double fb = 0.0;
+            if (blk[b]) {
+                const double *Fr = &F[sl][ly][x[b]];
+                const double ul = cur.ul[b] + Fr[-1] * idx * mul[b], uh = cur.uh[b] - Fr[1] * idx * muh[b];
+                double vl = cur.vl[b], vh = cur.vh[b];
+                if (!bot) vl = vl + Fr[-RW] * idy * mvl[b];
+                if (!top) vh = vh - Fr[RW] * idy * mvh[b];
+                const double wlo = cur.w[b] + F[sm][ly][x[b]] * idz * mw[b], whi = nxt.w[b] - F[sp][ly][x[b]] * idz * mw[b];
+                fb = ((uh - ul) * idx + (vh - vl) * idy + (whi - wlo) * idz) * q[b];
+                F[sl][ly][x[b]] = fb;
+            }
+            __syncthreads();
+            // ---- the low faces and p of both cells after both passes
+            const double fr = F[sl][ly][x[r]];
+            if (own && k >= k0) {
+                double un_[2], vn_[2], wn_[2], pn_[2];
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const bool red = c == r;   // this cell is red: its term comes first
+                    const double *Fc = &F[sl][ly][x[c]];
+                    const double fc = red ? fr : fb;
+                    const double ax = fc * idx * mul[c], bx = Fc[-1] * idx * mul[c];
+                    un_[c] = red ? (cur.ul[c] - ax) + bx : (cur.ul[c] + bx) - ax;
+                    const double az = fc * idz * mw[c], bz = fk[c] * idz * mw[c];
+                    wn_[c] = red ? (cur.w[c] - az) + bz : (cur.w[c] + bz) - az;
+                    const double ay = fc * idy * mvl[c];
+                    if (bot) {
+                        const double v1 = cur.vl[c] - ay;
+                        vn_[c] = wl.pt[0] == 0 ? v1 + wl.pv[0] * idy * mvl[c] : v1 + (fc * idy - wl.pv[0]) * mvl[c];
+                        if (last == 2) vn_[c] = wl.v[0];
+                    } else {
+                        const double by = Fc[-RW] * idy * mvl[c];
+                        vn_[c] = red ? (cur.vl[c] - ay) + by : (cur.vl[c] + by) - ay;
+                    }
+                    pn_[c] = po[c] + fc * idt;
+                    put(du, k, ol[c], un_[c]);
+                    put(dv, k, ol[c], vn_[c]);
+                    put(dw, k, ol[c], wn_[c]);
+                    put(pn, k, ol[c], pn_[c]);
+                    if (top && last) {   // the wall face above
+                        const double v1 = wl.v[1] + fc * idy * mvh[c];
+                        const double vt = wl.pt[1] == 0 ? v1 - wl.pv[1] * idy * mvh[c] : v1 + (wl.pv[1] - fc * idy) * mvh[c];
+                        put(dv, k, on[c], last == 2 ? wl.v[1] : vt);
+                    }
+                }
+                if (last == 2) {   // the boundary conditions, each ghost value from the one cell it copies
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        const int i = i0 + (c ? 1 - e : e);
+                        auto copy = [&](size_t g_) {
+                            du[g_] = un_[c];
+                            dv[g_] = vn_[c];
+                            dw[g_] = wn_[c];
+                            pn[g_] = pn_[c];
+                        };
+                        if (i == d.nx) copy(d.g(0, j, k));
+                        if (i == 1) copy(d.g(d.nx + 1, j, k));
+                        if (k == d.nz) copy(d.g(i, j, 0));
+                        if (k == 1) copy(d.g(i, j, d.nz + 1));
+                        if (bot) {
+                            const size_t g_ = d.g(i, 0, k);
+                            du[g_] = wl.u2[0] - un_[c];
+                            dw[g_] = wl.w2[0] - wn_[c];
+                        }
+                        if (top) {
+                            const size_t g_ = d.g(i, d.ny + 1, k);
+                            du[g_] = wl.u2[1] - un_[c];
+                            dw[g_] = wl.w2[1] - wn_[c];
+                        }
+                    }
+                }
+            }
+            fk[r] = fr;
+            fk[b] = fb;
+        }
+        sl = sl == 2 ? 0 : sl + 1;
+    };
+    // planes k0 - 3 (cell 1 red) .. k1
+    for (int k = k0 - 3; k <= k1; k += 2) {
+        plane(k, std::integral_constant<int, 1>{});
+        if (k + 1 <= k1) plane(k + 1, std::integral_constant<int, 0>{});
+    }
+}
+
+// The channel (x and z periodic; Dirichlet v on the y walls, or a periodic even ny) without
+// coefficients that vary in z takes one launch per iteration; other boundary conditions and
+// geometries the one-colour sweeps.
+bool sola_fused_fits(const mdx_handle *h) {
+    const mdx_config &c = h->cfg;
+    if (!c.periodic[0] || !c.periodic[2] || (h->ibm_on && !h->coef_plane) || !h->sola_tmp) return false;
+    if (c.periodic[1]) return h->d.ny % 2 == 0;
+    return c.bc_type[bci(2, 0, 2)] == 0 && c.bc_type[bci(2, 1, 2)] == 0;
+}
+
+hipError_t launch_sola(mdx_handle *h, double dtg) {
+    GridK g = grid_k(h);
+    const Dims d = h->d;
+    const mdx_config &c = h->cfg;
+    SolaWalls wl;
+    for (int s = 0; s < 2; ++s) {
+        wl.pt[s] = c.bc_type[bci(2, s, 0)];
+        wl.pv[s] = c.bc_value[bci(2, s, 0)];
+        wl.v[s] = c.bc_value[bci(2, s, 2)];
+        wl.u2[s] = 2 * c.bc_value[bci(2, s, 1)];
+        wl.w2[s] = 2 * c.bc_value[bci(2, s, 3)];
+    }
+    const double idx = 1.0 / h->dx, idy = 1.0 / h->dy, idz = 1.0 / h->dz;
+    const bool bc = h->step_bc && apply_writes_bc(h);
+    // Rows and planes per workgroup: the pair with the least (rounds of workgroups on the device) x
+    // (planes marched, kz + 3 for kz owned).  The registers leave a CU one workgroup of 32 rows or
+    // two of 16; a plane takes about 2.8 us in either once the device is full, and less with at most
+    // one of 16 rows per CU.  200^3: 32 rows x 25 planes, 160 us (16 planes 168, 20 185, 34 199; 16
+    // rows x 25 planes 168); 32 x 24 x 16: 16 rows x 1 plane, 6.9 us (2 planes 8.6; 32 rows 8.5).
+    int kz = 1, tye = 16;
+    double best = 1e300;
+    for (int ty = 16; ty <= 32; ty += 16)
+        for (int q = 1; q <= 64 && q <= d.nz; ++q) {
+            const long n = (long)((d.nx / 2 + SL_X - 3) / (SL_X - 2)) * ((d.ny + ty - 4) / (ty - 3)) * ((d.nz + q - 1) / q);
+            const long slots = ty == 32 ? 256 : 512, rounds = (n + slots - 1) / slots;
+            const double cost = (double)rounds * (q + 3) * (ty == 32 ? 1.0 : (n > 256 ? 1.05 : 0.85));
+            if (cost < best) {
+                best = cost;
+                kz = q;
+                tye = ty;
+            }
+        }
+    const bool small = tye == 16;
+    const unsigned tiles = xcd_grid(d.nx / 2, d.ny, (d.nz + kz - 1) / kz, SL_X - 2, tye - 3);
+    const unsigned ghosts = std::min<unsigned>(PROJ_GHOST_BLOCKS, (unsigned)(((size_t)d.sx * d.sy + (size_t)d.sx * d.nz +
+                                                                              (size_t)d.ny * d.nz) * 2 / 512 + 1));
+    const size_t ng = h->ng;
+    double *tmp[3] = {h->sola_tmp, h->sola_tmp + ng, h->sola_tmp + 2 * ng}, *fin[3] = {h->un, h->vn, h->wn};
+    const double *src[3] = {h->us, h->vs, h->ws};
+    for (int it = 0; it < c.niter; ++it) {
+        const int left = c.niter - 1 - it;   // iterations after this one: the last writes un, vn, wn
+        double *const *dst = left % 2 == 0 ? fin : tmp;
+        const int last = left ? 0 : (bc ? 2 : 1);
+        const dim3 grd(tiles + (left ? 0 : ghosts)), blk(SL_X, tye);
+#define MDX_SOLA(I, R)                                                                                             \
+    hipLaunchKernelGGL((sola_iter_kernel<I, R>), grd, blk, 0, h->stream, g, wl, c.omega, dtg, idx, idy, idz, idx * idx, \
+                       idy * idy, idz * idz, 1.0 / dtg, h->cu, h->cv, h->cw, src[0], src[1], src[2], dst[0], dst[1], \
+                       dst[2], h->pn, h->us, h->vs, h->ws, kz, tiles, last)
+        if (h->ibm_on) { if (small) MDX_SOLA(true, 16); else MDX_SOLA(true, 32); }
+        else { if (small) MDX_SOLA(false, 16); else MDX_SOLA(false, 32); }
+#undef MDX_SOLA
+        for (int q = 0; q < 3; ++q) src[q] = dst[q];
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    h->apply_wrote_bc = bc;
+    return hipSuccess;
+}
 
 // un = u* - mu grad Phi (likewise v, w) and pn += Phi / dt on the interior, reading u* directly;
 // on a walled y the bottom v face keeps its wall value.  A thread takes the column (i, j) of a

@@ -433,11 +433,14 @@ extern "C" int mdx_create(const mdx_config *cfg, mdx_handle **out) {
         tridiag_tables(h, cp, di, ar);
         twiddles(nx, twx);
         twiddles(nz, twz);
-        if ((e = dalloc(&h->fft_rhs, h->ni)) != hipSuccess || (e = dalloc(&h->hat, 2 * nh)) != hipSuccess ||
+        const size_t nhat = (size_t)fft_stride(nx, false) * ny * nz;   // the spectrum, rows padded
+        if ((e = dalloc(&h->fft_rhs, h->ni)) != hipSuccess || (e = dalloc(&h->hat, 2 * nhat)) != hipSuccess ||
             (e = dalloc(&h->cp, nh)) != hipSuccess || (e = dalloc(&h->den_inv, nh)) != hipSuccess ||
             (e = dalloc(&h->arow, ny)) != hipSuccess || (e = dalloc(&h->tw_x, nx)) != hipSuccess ||
             (e = dalloc(&h->tw_z, nz)) != hipSuccess)
             return fail(e, "FFT workspace");
+        // the padding of the spectrum's rows is read (and ignored) by the tridiagonal solves
+        if ((e = hipMemset(h->hat, 0, 2 * nhat * 8)) != hipSuccess) return fail(e, "FFT workspace");
         std::vector<double> plx, plz, pa, pbd, pc;
         tridiag_row_tables(h, plx, plz, pa, pbd, pc);
         if ((e = dalloc(&h->lamx, nxh)) != hipSuccess || (e = dalloc(&h->lamz, nz)) != hipSuccess ||
@@ -460,12 +463,14 @@ extern "C" int mdx_create(const mdx_config *cfg, mdx_handle **out) {
             auto to32 = [](const std::vector<double> &v) { return std::vector<float>(v.begin(), v.end()); };
             const std::vector<float> cp32 = to32(cp), di32 = to32(di), ar32 = to32(ar), twx32 = to32(twx),
                                      twz32 = to32(twz);
+            const size_t nhat32 = (size_t)fft_stride(nx, true) * ny * nz;
             if ((e = dalloc(&h->fft_phi, h->ni)) != hipSuccess || (e = dalloc(&h->fft_res, h->ni)) != hipSuccess ||
                 (e = dalloc(&h->fft_mean, 17 * (size_t)ny)) != hipSuccess ||
-                (e = dalloc(&h->hat32, 2 * nh)) != hipSuccess || (e = dalloc(&h->cp32, nh)) != hipSuccess ||
+                (e = dalloc(&h->hat32, 2 * nhat32)) != hipSuccess || (e = dalloc(&h->cp32, nh)) != hipSuccess ||
                 (e = dalloc(&h->den32, nh)) != hipSuccess || (e = dalloc(&h->arow32, ny)) != hipSuccess ||
                 (e = dalloc(&h->tw_x32, nx)) != hipSuccess || (e = dalloc(&h->tw_z32, nz)) != hipSuccess)
                 return fail(e, "mixed FFT workspace");
+            if ((e = hipMemset(h->hat32, 0, 2 * nhat32 * 4)) != hipSuccess) return fail(e, "mixed FFT workspace");
             if ((e = hipMemcpy(h->cp32, cp32.data(), nh * 4, hipMemcpyHostToDevice)) != hipSuccess ||
                 (e = hipMemcpy(h->den32, di32.data(), nh * 4, hipMemcpyHostToDevice)) != hipSuccess ||
                 (e = hipMemcpy(h->arow32, ar32.data(), ny * 4, hipMemcpyHostToDevice)) != hipSuccess ||

@@ -9,8 +9,10 @@
 //   4. inverse z-FFT                                                         hat -> hat
 //   5. inverse real x-FFT with the 1/(nx nz) scaling per row                 hat -> phi
 //   6. projection u = (u* - dtg grad phi)/(1 + dtg coef), p += phi
-// Transforms are radix-4 Stockham (self-sorting) in LDS with a precomputed FP64 twiddle table;
-// hat keeps the reference's half-spectrum layout plane_hat(nxh, nz, ny), kx fastest.
+// Transforms of 16 to 1024 points hold 16 points per thread in registers (fft_line: one LDS
+// exchange for 32 to 256 points, two above); shorter ones are radix-4 Stockham (self-sorting) in
+// LDS.  hat keeps the reference's half-spectrum layout plane_hat(nxh, nz, ny), kx fastest, each kx
+// row padded to whole 128-byte lines (fft_stride).
 #include "mdx_internal.h"
 
 namespace mdx {
@@ -93,6 +95,377 @@ __device__ inline void stage_twiddles(C *dst, const C *__restrict__ tw, int n) {
     for (int t = threadIdx.x; t < n / 2; t += FFT_THREADS) dst[t] = tw[t];
 }
 
+// ------------------------------------------------------------------------------- register transforms
+// An N-point line (N = 16 M, M = 1 .. 64) on M threads with 16 points each.  In every pass thread t
+// of the line holds the points t + M s (s = 0 .. 15), which are whole butterflies of every radix
+// used: radix M first for N <= 256 (1, 2, 4, 8 or 16), radix N / 256 and 16 above, and 16 last.  A
+// pass is one to two of stockham's radix-2 and radix-4 steps done in registers, with its twiddles and
+// its order of operations, so a line's transform has the same bits (the FP32 passes of the defect
+// correction leave the same phi).  Between passes the points go through LDS once, instead of once
+// per radix-4 step with the whole line read from and written to LDS each time; a thread's first
+// loads and last stores are its own points, so no staging either.  LDS addresses are padded by one
+// element in 16, which keeps the radix-16 scatter (16 elements apart) and the gather (consecutive)
+// free of bank conflicts.  At 256 x 192 x 256 in FP64 the LDS kernels took 129 us (x, with the
+// right-hand side), 94 us (z, either way) and 89 us (x inverse); these take 99, 50 (42 inverse) and
+// 35 us, which is 4 to 5 TB/s of the fields and the spectrum read and written once.  In FP32: 49 us
+// (x), 62 (z) and 62 (x inverse, adding to phi) before, 25, 31 (24 inverse) and 40 now.
+template <typename C, bool INV> __device__ inline C ctw(C a, C w) {   // a w (forward) or a conj(w)
+    const typename Cx<C>::R wi = INV ? -w.y : w.y;
+    return Cx<C>::mk(a.x * w.x - a.y * wi, a.x * wi + a.y * w.x);
+}
+// 4-point transform; the forward one multiplies by (-i)^(pq), the inverse one by i^(pq)
+template <typename C, bool INV> __device__ inline void dft4(C &a, C &b, C &c, C &d) {
+    const C s02 = Cx<C>::mk(a.x + c.x, a.y + c.y), d02 = Cx<C>::mk(a.x - c.x, a.y - c.y),
+            s13 = Cx<C>::mk(b.x + d.x, b.y + d.y), d13 = Cx<C>::mk(b.x - d.x, b.y - d.y),
+            j = INV ? Cx<C>::mk(-d13.y, d13.x) : Cx<C>::mk(d13.y, -d13.x);
+    a = Cx<C>::mk(s02.x + s13.x, s02.y + s13.y);
+    b = Cx<C>::mk(d02.x + j.x, d02.y + j.y);
+    c = Cx<C>::mk(s02.x - s13.x, s02.y - s13.y);
+    d = Cx<C>::mk(d02.x - j.x, d02.y - j.y);
+}
+
+template <int N, int TH> struct RFft {   // TH threads per workgroup
+    static constexpr int M = N / 16;                       // threads per line
+    static constexpr int LPW = TH / M;                     // lines per workgroup
+    static constexpr int LS = N + M + 1;                   // LDS elements per line (padded)
+    static constexpr int R0 = M <= 16 ? M : M / 16;        // first radix
+    static constexpr int TW = 3 * N / 4;                   // twiddles w^m in LDS
+    static constexpr bool TW0 = M == 1 || R0 >= 8;         // the first pass needs them
+};
+__device__ inline int rf_pad(int q) { return q + (q >> 4); }
+
+// one pass of radix R on the thread's 16 points, as radix-2 and radix-4 steps in registers (the
+// groups of ns points become groups of R ns), and the scatter to line (LDS) unless it is the last
+// pass.  tw[m] = w^m, 0 <= m < 3 N / 4.
+template <typename C, int N, int R, int NS, bool INV, bool LAST>
+__device__ inline void rf_pass(C (&e)[16], int t, const C *tw, C *line) {
+    constexpr int M = N / 16, U = 16 / R;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int b = t + u * M, kk = b & (NS - 1);
+        C v[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) v[q] = e[u + q * U];
+        if constexpr (R == 2 || R == 8) {   // radix 2, groups of 1
+            constexpr int H = R / 2;
+#pragma unroll
+            for (int q = 0; q < H; ++q) {
+                const C x0 = v[q], x1 = v[q + H];
+                v[q] = Cx<C>::mk(x0.x + x1.x, x0.y + x1.y);
+                v[q + H] = Cx<C>::mk(x0.x - x1.x, x0.y - x1.y);
+            }
+        }
+        if constexpr (R == 8) {   // radix 4, groups of 2: v[q + 4 p] -> v[p + 2 q']
+#pragma unroll
+            for (int q = 1; q < 4; ++q) v[q + 4] = ctw<C, INV>(v[q + 4], tw[q * (N / 8)]);
+            dft4<C, INV>(v[0], v[1], v[2], v[3]);
+            dft4<C, INV>(v[4], v[5], v[6], v[7]);
+            const C w[8] = {v[0], v[4], v[1], v[5], v[2], v[6], v[3], v[7]};
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = w[q];
+        }
+        if constexpr (R == 4 || R == 16) {   // radix 4, groups of NS
+            constexpr int Q = R / 4;
+#pragma unroll
+            for (int a = 0; a < Q; ++a) {
+                if (NS > 1) {
+#pragma unroll
+                    for (int q = 1; q < 4; ++q) v[a + q * Q] = ctw<C, INV>(v[a + q * Q], tw[q * kk * (N / (4 * NS))]);
+                }
+                dft4<C, INV>(v[a], v[a + Q], v[a + 2 * Q], v[a + 3 * Q]);
+            }
+        }
+        if constexpr (R == 16) {   // radix 4, groups of 4 NS: v[a + 4 c] -> v[c + 4 d]
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if (NS > 1 || c > 0) {
+#pragma unroll
+                    for (int a = 1; a < 4; ++a)
+                        v[a + 4 * c] = ctw<C, INV>(v[a + 4 * c], tw[a * (kk + NS * c) * (N / (16 * NS))]);
+                }
+                dft4<C, INV>(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int d = 0; d < c; ++d) {
+                    const C x = v[4 * c + d];
+                    v[4 * c + d] = v[4 * d + c];
+                    v[4 * d + c] = x;
+                }
+        }
+        const int o = (b - kk) * R + kk;
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            if (LAST) e[u + q * U] = v[q];
+            else line[rf_pad(o + q * NS)] = v[q];
+        }
+    }
+}
+template <typename C, int N>
+__device__ inline void rf_gather(C (&e)[16], int t, const C *line) {
+#pragma unroll
+    for (int s = 0; s < 16; ++s) e[s] = line[rf_pad(t + N / 16 * s)];
+}
+// the transform of the line whose points t + M s thread t holds in e; line: the line's LDS, tw: the
+// twiddles in LDS (staged by the caller before the barrier in here); threads with
+// `on` false hold no line and only join the barriers
+template <typename C, int N, bool INV>
+__device__ inline void fft_line(C (&e)[16], int t, const C *tw, C *line, bool on = true) {
+    using F = RFft<N, 64>;
+    if constexpr (F::M == 1) {
+        __syncthreads();
+        if (on) rf_pass<C, N, 16, 1, INV, true>(e, t, tw, line);
+    } else {
+        if constexpr (F::TW0) __syncthreads();
+        if (on) rf_pass<C, N, F::R0, 1, INV, false>(e, t, tw, line);
+        __syncthreads();
+        if (on) rf_gather<C, N>(e, t, line);
+        if constexpr (F::M > 16) {
+            __syncthreads();
+            if (on) rf_pass<C, N, 16, F::R0, INV, false>(e, t, tw, line);
+            __syncthreads();
+            if (on) rf_gather<C, N>(e, t, line);
+        }
+        if (on) rf_pass<C, N, 16, F::M, INV, true>(e, t, tw, line);
+    }
+}
+// the twiddles of fft_line into LDS (tw: w^m, m < N / 2; w^(m + N/2) = -w^m)
+template <typename C, int N, int TH, int W = 1>
+__device__ inline void rf_stage(C *dst, const C *__restrict__ tw) {
+    for (int q = threadIdx.x; q < RFft<N, TH>::TW; q += TH * W) {
+        const C w = tw[q < N / 2 ? q : q - N / 2];
+        dst[q] = q < N / 2 ? w : Cx<C>::mk(-w.x, -w.y);
+    }
+}
+// Two real rows are one complex line: row r in the real parts, row r + 1 (the next plane's) in the
+// imaginary ones, so the x-transforms do half the work of real rows taken as complex lines.
+// F(m) = A(m) + i B(m), A(m) = (F(m) + conj F(N - m)) / 2, B(m) = (F(m) - conj F(N - m)) / 2i.
+// The line is in LDS in natural order; the rows' half spectra go to a and b.
+template <typename C, int N>
+__device__ inline void rf_split(const C *line, int m, C &a, C &b) {
+    using T = typename Cx<C>::R;
+    const C f = line[rf_pad(m)], g = line[rf_pad((N - m) & (N - 1))];
+    a = Cx<C>::mk(T(0.5) * (f.x + g.x), T(0.5) * (f.y - g.y));
+    b = Cx<C>::mk(T(0.5) * (f.y + g.y), T(0.5) * (g.x - f.x));
+}
+// rows 2 P and 2 P + 1 of the thread's line from its transform e to hat; every thread of the
+// workgroup calls it (barriers)
+template <typename C, int N, int TH, int W = 1>
+__device__ inline void rf_store_rows(C (&e)[16], int t, C *lds, int l, int P0, int npairs, int stride, C *hat) {
+    using F = RFft<N, TH>;
+    C *line = lds + (size_t)l * F::LS;
+    __syncthreads();
+    if (W == 1 || l < F::LPW) {
+#pragma unroll
+        for (int s = 0; s < 16; ++s) line[rf_pad(t + F::M * s)] = e[s];
+    }
+    __syncthreads();
+    constexpr int H = N / 2 + 1;
+    for (int q = threadIdx.x; q < F::LPW * H; q += TH * W) {
+        const int ll = q / H, m = q - ll * H, P = P0 + ll;
+        if (P >= npairs) break;
+        C a, b;
+        rf_split<C, N>(lds + (size_t)ll * F::LS, m, a, b);
+        hat[(size_t)stride * (2 * P) + m] = a;
+        hat[(size_t)stride * (2 * P + 1) + m] = b;
+    }
+}
+// the thread's points of the inverse line of rows 2 P and 2 P + 1, from their half spectra (the real
+// parts of the kx = 0 and kx = nx / 2 coefficients, Hermitian extension of the rest)
+template <typename C, int N>
+__device__ inline void rf_load_rows(C (&e)[16], int t, int P, int stride, const C *__restrict__ hat) {
+    const C *A = hat + (size_t)stride * (2 * P), *B = A + stride;
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+        const int q = t + N / 16 * s;
+        if (s < 8) {
+            C a = A[q], b = B[q];
+            if (s == 0 && q == 0) a.y = b.y = 0;
+            e[s] = Cx<C>::mk(a.x - b.y, a.y + b.x);
+        } else {
+            C a = A[N - q], b = B[N - q];
+            if (s == 8 && 2 * q == N) a.y = b.y = 0;
+            e[s] = Cx<C>::mk(a.x + b.y, b.x - a.y);
+        }
+    }
+}
+
+// complex elements per kx row of the spectrum: nx / 2 + 1 rounded up to 128 bytes, so every row and
+// every tile of 8 (FP64) or 16 (FP32) columns starts on a line (unpadded, the z-transform fetched
+// 1.9 times its data)
+template <typename C> static int fft_stride_t(int nx) {
+    const int per = 128 / (int)sizeof(C);
+    return (nx / 2 + 1 + per - 1) / per * per;
+}
+int fft_stride(int nx, bool fp32) { return fp32 ? fft_stride_t<float2>(nx) : fft_stride_t<double2>(nx); }
+
+// a / d with r = 1 / d rounded: the quotient corrected once by its residual, which is a / d rounded
+// (Markstein) for all but the ends of the exponent range: 3 operations where the division takes a
+// dozen.  A plain a * r would put the rounding of r into every cell alike.
+__device__ inline double div_by(double a, double d, double r) {
+    const double q = a * r;
+    return fma(fma(-q, d, a), r, q);
+}
+
+// 1. rhs(i,k,j) = div u* / dtg and the forward x-transform, two rows (planes k, k + 1) per line
+template <int N, int TH, int W, bool STRETCH>
+__global__ __launch_bounds__(TH * W) void rhs_xfft_reg_kernel(GridK g, const double *__restrict__ us,
+                                                              const double *__restrict__ vs,
+                                                              const double *__restrict__ ws, double dtg,
+                                                              const double2 *__restrict__ tw, int stride,
+                                                              double2 *__restrict__ hat) {
+    using F = RFft<N, TH>;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    double2 *lds = reinterpret_cast<double2 *>(lds_raw), *twl = lds + F::LPW * F::LS;
+    const Dims d = g.d;
+    const int npairs = d.ny * d.nz / 2, t = threadIdx.x % F::M, l = threadIdx.x / F::M;
+    const int P0 = blockIdx.x * F::LPW;
+    const double it = 1.0 / dtg, ix = 1.0 / g.dx, iy = 1.0 / g.dy, iz = 1.0 / g.dz;
+    const size_t sy = d.sx, sz = (size_t)d.sx * d.sy;
+    // the lines in row order (a wave's loads are consecutive cells), each thread 16 / W cell pairs
+#pragma unroll
+    for (int s = 0; s < 16 / W; ++s) {
+        const int q = threadIdx.x + TH * W * s, ll = q / N, i = q % N, P = P0 + ll;
+        double2 r = make_double2(0.0, 0.0);
+        if (P < npairs) {
+            const int k = (2 * P) % d.nz + 1, j = (2 * P) / d.nz + 1;
+            const size_t c0 = d.g(1 + i, j, k);
+            const double *u = us + c0, *v = vs + c0, *w = ws + c0;
+            const double w1 = w[sz], ih = STRETCH ? g.ihc[j] : 0.0;
+            auto rhs = [&](double du, double dv, double dw) {
+                const double dy = STRETCH ? dv * ih : div_by(dv, g.dy, iy);
+                return div_by(div_by(du, g.dx, ix) + dy + div_by(dw, g.dz, iz), dtg, it);
+            };
+            r.x = rhs(u[1] - u[0], v[sy] - v[0], w1 - w[0]);
+            r.y = rhs(u[sz + 1] - u[sz], v[sz + sy] - v[sz], w[2 * sz] - w1);
+        }
+        lds[(size_t)ll * F::LS + rf_pad(i)] = r;
+    }
+    rf_stage<double2, N, TH, W>(twl, tw);
+    __syncthreads();
+    const bool on = W == 1 || l < F::LPW;
+    double2 *line = lds + (on ? l : 0) * F::LS;
+    double2 e[16];
+    if (on) rf_gather<double2, N>(e, t, line);
+    if constexpr (!F::TW0) __syncthreads();   // the lines are read before they are written again
+    fft_line<double2, N, false>(e, t, twl, line, on);
+    rf_store_rows<double2, N, TH, W>(e, t, lds, l, P0, npairs, stride, hat);
+}
+
+// 1. (FP32) forward x-transform of a real FP64 field in (nx, nz, ny) layout, a row per line (two rows
+// in one line would mix their roundings, and a pass of the defect correction is only as accurate)
+template <int N, int TH>
+__global__ __launch_bounds__(TH) void xfft32_reg_kernel(Dims d, const double *__restrict__ in,
+                                                        const float2 *__restrict__ tw, int stride,
+                                                        float2 *__restrict__ hat) {
+    using F = RFft<N, TH>;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    float2 *lds = reinterpret_cast<float2 *>(lds_raw), *twl = lds + F::LPW * F::LS;
+    const int nrows = d.ny * d.nz, t = threadIdx.x % F::M, r = blockIdx.x * F::LPW + threadIdx.x / F::M;
+    rf_stage<float2, N, TH>(twl, tw);
+    float2 e[16];
+    const double *a = in + (size_t)N * (r < nrows ? r : 0) + t;
+#pragma unroll
+    for (int s = 0; s < 16; ++s) e[s] = make_float2((float)a[F::M * s], 0.f);
+    fft_line<float2, N, false>(e, t, twl, lds + threadIdx.x / F::M * F::LS);
+    if (r >= nrows) return;
+    float2 *h = hat + (size_t)stride * r + t;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) h[F::M * s] = e[s];
+    if (t == 0) h[N / 2] = e[8];
+}
+
+// 5. inverse x-transform: phi (nx, nz, ny) = scaled rows, two per line
+template <int N, int TH>
+__global__ __launch_bounds__(TH) void ixfft_reg_kernel(Dims d, const double2 *__restrict__ hat,
+                                                       const double2 *__restrict__ tw, int stride, double scale,
+                                                       double *__restrict__ phi) {
+    using F = RFft<N, TH>;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    double2 *lds = reinterpret_cast<double2 *>(lds_raw), *twl = lds + F::LPW * F::LS;
+    const int npairs = d.ny * d.nz / 2, t = threadIdx.x % F::M, l = threadIdx.x / F::M;
+    const int P = blockIdx.x * F::LPW + l;
+    rf_stage<double2, N, TH>(twl, tw);
+    double2 e[16];
+    rf_load_rows<double2, N>(e, t, P < npairs ? P : 0, stride, hat);
+    fft_line<double2, N, true>(e, t, twl, lds + l * F::LS);
+    if (P >= npairs) return;
+    double *p = phi + (size_t)N * (2 * P) + t;
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+        p[F::M * s] = e[s].x * scale;
+        p[N + F::M * s] = e[s].y * scale;
+    }
+}
+// 5. (FP32) inverse x-transform of each row, scaled and added to the FP64 phi
+template <int N, int TH>
+__global__ __launch_bounds__(TH) void ixfft32_add_reg_kernel(Dims d, const float2 *__restrict__ hat,
+                                                             const float2 *__restrict__ tw, int stride, float scale,
+                                                             double *__restrict__ phi) {
+    using F = RFft<N, TH>;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    float2 *lds = reinterpret_cast<float2 *>(lds_raw), *twl = lds + F::LPW * F::LS;
+    const int nrows = d.ny * d.nz, t = threadIdx.x % F::M, r = blockIdx.x * F::LPW + threadIdx.x / F::M;
+    rf_stage<float2, N, TH>(twl, tw);
+    const float2 *h = hat + (size_t)stride * (r < nrows ? r : 0);
+    double *p = phi + (size_t)N * (r < nrows ? r : 0) + t;
+    float2 e[16];
+    double a[16];
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+        const int q = t + F::M * s;
+        if (s < 8) {
+            e[s] = h[q];
+            if (s == 0 && q == 0) e[s].y = 0.f;
+        } else {
+            const float2 c = h[N - q];
+            e[s] = make_float2(c.x, s == 8 && 2 * q == N ? 0.f : -c.y);
+        }
+        a[s] = p[F::M * s];
+    }
+    fft_line<float2, N, true>(e, t, twl, lds + threadIdx.x / F::M * F::LS);
+    if (r >= nrows) return;
+#pragma unroll
+    for (int s = 0; s < 16; ++s) p[F::M * s] = a[s] + (double)(e[s].x * scale);
+}
+
+// 2./4. z-transform in place.  The first `tiles` workgroups take CW consecutive kx columns (CW = 16,
+// or the lines of a workgroup or half the x points if fewer) of LPW / CW planes; the others the nrem
+// columns past the last whole tile (one, the highest kx, where CW divides nx / 2), a plane per line:
+// in a tile of its own it would leave 15 of 16 threads idle.  The line index runs fastest over the
+// threads, so a load or store of one kz moves the CW columns' consecutive values.
+template <typename C, int N, int TH, bool INV>
+__global__ __launch_bounds__(TH) void zfft_reg_kernel(int ny, int stride, int cw, int ntx, int tiles, int nrem,
+                                                              const C *__restrict__ tw, C *__restrict__ hat) {
+    using F = RFft<N, TH>;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    C *lds = reinterpret_cast<C *>(lds_raw), *twl = lds + F::LPW * F::LS;
+    const int l = threadIdx.x % F::LPW, t = threadIdx.x / F::LPW;
+    int kx, j;
+    bool live;
+    if ((int)blockIdx.x < tiles) {
+        const int pw = F::LPW / cw, tx = blockIdx.x % ntx, ty = blockIdx.x / ntx;
+        kx = tx * cw + l % cw;
+        j = ty * pw + l / cw;
+        live = j < ny;
+    } else {
+        const int q = (blockIdx.x - tiles) * F::LPW + l;
+        kx = ntx * cw + q / ny;
+        j = q % ny;
+        live = q < nrem * ny;
+    }
+    rf_stage<C, N, TH>(twl, tw);
+    C *p = hat + (size_t)stride * N * (live ? j : 0) + (live ? kx : 0);
+    C e[16];
+#pragma unroll
+    for (int s = 0; s < 16; ++s) e[s] = p[(size_t)stride * (t + F::M * s)];
+    fft_line<C, N, INV>(e, t, twl, lds + l * F::LS);
+    if (!live) return;
+#pragma unroll
+    for (int s = 0; s < 16; ++s) p[(size_t)stride * (t + F::M * s)] = e[s];
+}
+
 // 1. rhs(i,k,j) = [(u*(i+1)-u*(i))/dx + (v*(j+1)-v*(j))/dy + (w*(k+1)-w*(k))/dz]/dtg, then the
 //    r2c x-transform; rows r = (k-1) + nz (j-1) are contiguous in hat.
 template <bool STRETCH>
@@ -100,7 +473,7 @@ __global__ __launch_bounds__(FFT_THREADS) void rhs_xfft_kernel(GridK g, const do
                                                               const double *__restrict__ vs,
                                                               const double *__restrict__ ws, double dtg,
                                                               const double2 *__restrict__ tw, int lines,
-                                                              double2 *hat) {
+                                                              int stride, double2 *hat) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     double2 *lds = reinterpret_cast<double2 *>(lds_raw);
     const Dims d = g.d;
@@ -126,14 +499,14 @@ __global__ __launch_bounds__(FFT_THREADS) void rhs_xfft_kernel(GridK g, const do
     for (int t = threadIdx.x; t < lines * nxh; t += FFT_THREADS) {
         const int line = t / nxh, m = t - line * nxh;
         const int r = blockIdx.x * lines + line;
-        if (r < nrows) hat[(size_t)nxh * r + m] = res[line * n + m];
+        if (r < nrows) hat[(size_t)stride * r + m] = res[line * n + m];
     }
 }
 
 // 2./4. z-transform of TX consecutive kx columns of one j plane.
 template <typename C>
 __global__ __launch_bounds__(FFT_THREADS) void zfft_kernel(Dims d, C *hat, const C *__restrict__ tw, int tx,
-                                                           int inverse) {
+                                                           int inverse, int stride) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     C *lds = reinterpret_cast<C *>(lds_raw);
     const int nz = d.nz, nxh = d.nx / 2 + 1;
@@ -143,19 +516,19 @@ __global__ __launch_bounds__(FFT_THREADS) void zfft_kernel(Dims d, C *hat, const
     // fall in different banks
     const int ls = nz + 1;
     C *a = lds, *b = lds + (size_t)tx * ls, *twl = b + (size_t)tx * ls;
-    C *plane = hat + (size_t)nxh * nz * j;
+    C *plane = hat + (size_t)stride * nz * j;
     stage_twiddles(twl, tw, nz);
     for (int t = threadIdx.x; t < tx * nz; t += FFT_THREADS) {
         const int c = t % tx, kz = t / tx;
         const int kx = kx0 + c;
-        a[c * ls + kz] = kx < nxh ? plane[(size_t)kx + (size_t)nxh * kz] : Cx<C>::mk(0, 0);
+        a[c * ls + kz] = kx < nxh ? plane[(size_t)kx + (size_t)stride * kz] : Cx<C>::mk(0, 0);
     }
     __syncthreads();
     C *res = stockham(a, b, nz, tx, ls, twl, inverse != 0, threadIdx.x, FFT_THREADS);
     for (int t = threadIdx.x; t < tx * nz; t += FFT_THREADS) {
         const int c = t % tx, kz = t / tx;
         const int kx = kx0 + c;
-        if (kx < nxh) plane[(size_t)kx + (size_t)nxh * kz] = res[c * ls + kz];
+        if (kx < nxh) plane[(size_t)kx + (size_t)stride * kz] = res[c * ls + kz];
     }
 }
 
@@ -166,16 +539,16 @@ __global__ __launch_bounds__(FFT_THREADS) void zfft_kernel(Dims d, C *hat, const
 //    time instead of one; the arithmetic and its order are those of the plane-by-plane loops.
 static constexpr int TB = 8;
 
-__global__ __launch_bounds__(64) void tridiag_kernel(Dims d, double2 *hat, const double *__restrict__ cp,
+__global__ __launch_bounds__(64) void tridiag_kernel(Dims d, int stride, double2 *hat, const double *__restrict__ cp,
                                                      const double *__restrict__ den_inv,
                                                      const double *__restrict__ arow) {
     const int nxh = d.nx / 2 + 1, ny = d.ny, nz = d.nz;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nxh * nz) return;
     const int kx = t % nxh, kz = t / nxh;
-    const size_t hs = (size_t)nxh * nz;                     // stride between j planes in hat
+    const size_t hs = (size_t)stride * nz;                  // stride between j planes in hat
     const size_t cs = (size_t)nxh;                          // stride between j in cp/den_inv
-    const size_t h0 = (size_t)kx + (size_t)nxh * kz;
+    const size_t h0 = (size_t)kx + (size_t)stride * kz;
     const size_t c0 = (size_t)kx + (size_t)nxh * (size_t)ny * kz;
     double2 dp;
     if (kx == 0 && kz == 0) {
@@ -283,7 +656,7 @@ __device__ inline V pick_hi(const V (&sh)[M], int q, bool wrap, V edge) {
 // C: double2 (the FP64 solve; the mean mode pins row 1) or float2 (the FP32 defect solves; the
 // mean mode is solved apart in FP64, so its line is zeroed, MEAN_ZERO)
 template <typename C, int M, bool MEAN_ZERO>
-__global__ __launch_bounds__(64 * TW_WAVES) void tridiag_wave_kernel(int nlines, int nxh, int ny, size_t plane, C *hat,
+__global__ __launch_bounds__(64 * TW_WAVES) void tridiag_wave_kernel(int nlines, int stride, int nxh, int ny, size_t plane, C *hat,
                                                                     const typename Cx<C>::R *__restrict__ lamx,
                                                                     const typename Cx<C>::R *__restrict__ lamz,
                                                                     const typename Cx<C>::R *__restrict__ arow,
@@ -309,12 +682,13 @@ __global__ __launch_bounds__(64 * TW_WAVES) void tridiag_wave_kernel(int nlines,
     for (int l = wave; l < TW_LINES; l += TW_WAVES) {
         const int t = t0 + l;
         if (t >= nlines) break;   // whole waves
+        if (t % stride >= nxh) continue;   // the padding of a kx row
         C *line = tile + (size_t)l * ldt;
         if (MEAN_ZERO && t == 0) {
             for (int j = lane; j < ny; j += 64) line[j] = zero2;
             continue;
         }
-        const int kx = t % nxh, kz = t / nxh;
+        const int kx = t % stride, kz = t / stride;
         const R k = lamx[kx] + lamz[kz];
         // the original rows (kept for the residual) and the right-hand side
         R a0[M], b0[M], c0[M];
@@ -463,8 +837,8 @@ __global__ __launch_bounds__(64 * TW_WAVES) void tridiag_wave_kernel(int nlines,
 //     mean mode pins row 1 as the wave solve does; MEAN_ZERO zeroes that line.
 static constexpr int TP_LINES = 16, TP_SEGS = 16;
 template <typename C, int M, bool MEAN_ZERO>
-__global__ __launch_bounds__(TP_LINES * TP_SEGS) void tridiag_part_kernel(int nlines, int nxh, int ny, size_t plane,
-                                                                        C *hat,
+__global__ __launch_bounds__(TP_LINES * TP_SEGS) void tridiag_part_kernel(int nlines, int stride, int nxh, int ny,
+                                                                        size_t plane, C *hat,
                                                                         const typename Cx<C>::R *__restrict__ lamx,
                                                                         const typename Cx<C>::R *__restrict__ lamz,
                                                                         const typename Cx<C>::R *__restrict__ arow,
@@ -484,8 +858,9 @@ __global__ __launch_bounds__(TP_LINES * TP_SEGS) void tridiag_part_kernel(int nl
     __syncthreads();
     C *line = tile + (size_t)tt * ldt;
     R k = R(0);
-    if (t < nlines) k = lamx[t % nxh] + lamz[t / nxh];
-    const bool ident_line = t >= nlines || (MEAN_ZERO && t == 0);
+    const bool live = t < nlines && t % stride < nxh;   // a line, not the padding of a kx row
+    if (live) k = lamx[t % stride] + lamz[t / stride];
+    const bool ident_line = !live || (MEAN_ZERO && t == 0);
     const int j0 = sg * M;
     // row r of the segment: (a, b, c); the data row is line[j0 + r]
     auto coef = [&](int r, R &a, R &b, R &c) {
@@ -601,7 +976,7 @@ __global__ __launch_bounds__(TP_LINES * TP_SEGS) void tridiag_part_kernel(int nl
         if (j0 + M - 1 < ny) line[j0 + M - 1] = E;
     }
     __syncthreads();
-    if (t < nlines)
+    if (live)
         for (int j = sg; j < ny; j += TP_SEGS) hat[(size_t)t + plane * j] = tile[tt * ldt + j];
 }
 
@@ -611,8 +986,8 @@ static bool launch_tridiag_part(hipStream_t st, const Dims &d, C *hat, const typ
                                 const typename Cx<C>::R *lamz, const typename Cx<C>::R *a,
                                 const typename Cx<C>::R *bd, const typename Cx<C>::R *c) {
     if (d.ny < 64 || d.ny > 256) return false;
-    const int nxh = d.nx / 2 + 1, nlines = nxh * d.nz, m = (d.ny + TP_SEGS - 1) / TP_SEGS;
-    const size_t plane = (size_t)nxh * d.nz;
+    const int nxh = d.nx / 2 + 1, stride = fft_stride_t<C>(d.nx), nlines = stride * d.nz, m = (d.ny + TP_SEGS - 1) / TP_SEGS;
+    const size_t plane = (size_t)nlines;
     const dim3 grid((nlines + TP_LINES - 1) / TP_LINES), blk(TP_LINES * TP_SEGS);
     const size_t lds = (size_t)TP_LINES * (d.ny + 1) * sizeof(C);   // <= 66 KB
 #define TP_CASE(MM)                                                                                            \
@@ -621,7 +996,7 @@ static bool launch_tridiag_part(hipStream_t st, const Dims &d, C *hat, const typ
             reinterpret_cast<const void *>(&tridiag_part_kernel<C, MM, MEAN_ZERO>),                            \
             hipFuncAttributeMaxDynamicSharedMemorySize, 16 * 257 * (int)sizeof(C));                            \
         if (attr != hipSuccess) return false;                                                                  \
-        hipLaunchKernelGGL((tridiag_part_kernel<C, MM, MEAN_ZERO>), grid, blk, lds, st, nlines, nxh, d.ny, plane, \
+        hipLaunchKernelGGL((tridiag_part_kernel<C, MM, MEAN_ZERO>), grid, blk, lds, st, nlines, stride, nxh, d.ny, plane, \
                            hat, lamx, lamz, a, bd, c);                                                         \
         return true;                                                                                           \
     }
@@ -635,8 +1010,8 @@ template <typename C, bool MEAN_ZERO>
 static bool launch_tridiag_wave(hipStream_t st, const Dims &d, C *hat, const typename Cx<C>::R *lamx,
                                 const typename Cx<C>::R *lamz, const typename Cx<C>::R *a,
                                 const typename Cx<C>::R *bd, const typename Cx<C>::R *c) {
-    const int nxh = d.nx / 2 + 1, nlines = nxh * d.nz, m = (d.ny + 63) / 64;
-    const size_t plane = (size_t)nxh * d.nz;
+    const int nxh = d.nx / 2 + 1, stride = fft_stride_t<C>(d.nx), nlines = stride * d.nz, m = (d.ny + 63) / 64;
+    const size_t plane = (size_t)nlines;
     const dim3 grid((nlines + TW_LINES - 1) / TW_LINES), blk(64 * TW_WAVES);
     const size_t lds = (size_t)TW_LINES * (d.ny + 1) * sizeof(C);   // <= 66 KB (ny <= 256)
 #define TW_CASE(MM)                                                                                            \
@@ -645,7 +1020,7 @@ static bool launch_tridiag_wave(hipStream_t st, const Dims &d, C *hat, const typ
             reinterpret_cast<const void *>(&tridiag_wave_kernel<C, MM, MEAN_ZERO>),                            \
             hipFuncAttributeMaxDynamicSharedMemorySize, 16 * 257 * (int)sizeof(C));                            \
         if (attr != hipSuccess) return false;                                                                  \
-        hipLaunchKernelGGL((tridiag_wave_kernel<C, MM, MEAN_ZERO>), grid, blk, lds, st, nlines, nxh, d.ny, plane, \
+        hipLaunchKernelGGL((tridiag_wave_kernel<C, MM, MEAN_ZERO>), grid, blk, lds, st, nlines, stride, nxh, d.ny, plane, \
                            hat, lamx, lamz, a, bd, c);                                                         \
         return true;                                                                                           \
     }
@@ -660,7 +1035,7 @@ static bool launch_tridiag_wave(hipStream_t st, const Dims &d, C *hat, const typ
 //    rest, inverse transform, times 1/(nx nz); phi in rhs layout (nx, nz, ny).
 __global__ __launch_bounds__(FFT_THREADS) void ixfft_kernel(Dims d, const double2 *__restrict__ hat,
                                                            const double2 *__restrict__ tw, int lines,
-                                                           double scale, double *phi) {
+                                                           int stride, double scale, double *phi) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     double2 *lds = reinterpret_cast<double2 *>(lds_raw);
     const int n = d.nx, nxh = n / 2 + 1;
@@ -672,7 +1047,7 @@ __global__ __launch_bounds__(FFT_THREADS) void ixfft_kernel(Dims d, const double
         const int r = blockIdx.x * lines + line;
         double2 v = make_double2(0.0, 0.0);
         if (r < nrows) {
-            const double2 *row = hat + (size_t)nxh * r;
+            const double2 *row = hat + (size_t)stride * r;
             if (m == 0 || 2 * m == n) v = make_double2(row[m].x, 0.0);
             else if (m < nxh) v = row[m];
             else v = make_double2(row[n - m].x, -row[n - m].y);
@@ -754,27 +1129,141 @@ static hipError_t zfft_allow(size_t bytes) {
     return e;
 }
 
-hipError_t launch_fft_forward(mdx_handle *h, double dtg) {
+// allow a kernel more than the default 64 KB of dynamic LDS (once per kernel)
+template <auto FN> static hipError_t rf_allow(size_t bytes) {
+    if (bytes <= 65536) return hipSuccess;
+    static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(FN),
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    return e;
+}
+// a kernel of the register transforms on `blocks` workgroups
+template <typename C, int N, int TH, auto FN, int W = 1, typename... A>
+static hipError_t rf_launch(hipStream_t st, unsigned blocks, A... args) {
+    using F = RFft<N, TH>;
+    const size_t lds = ((size_t)F::LPW * F::LS + F::TW) * sizeof(C);
+    const hipError_t e = rf_allow<FN>(lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(FN, dim3(blocks), dim3(TH * W), lds, st, args...);
+    return hipGetLastError();
+}
+// CALL(N) for the register transforms' lengths (it returns); shorter lines fall through
+#define RF_SIZES(n, CALL)  \
+    switch (n) {           \
+    case 16: CALL(16);     \
+    case 32: CALL(32);     \
+    case 64: CALL(64);     \
+    case 128: CALL(128);   \
+    case 256: CALL(256);   \
+    case 512: CALL(512);   \
+    case 1024: CALL(1024); \
+    default: break;        \
+    }
+
+template <int N, int TH>
+static unsigned rf_row_blocks(const Dims &d, int rows = 2) {   // rows: rows per line
+    return (unsigned)((d.ny * d.nz / rows + RFft<N, TH>::LPW - 1) / RFft<N, TH>::LPW);
+}
+// Workgroups of one transforming wavefront (64 threads; the x-transform with the right-hand side adds
+// three that only load and store) where those of 256 would leave CUs without two: `blocks256` is the
+// number of the latter.  Measured at 64^3 (32 to 36 workgroups of 256): z 10.2 us -> 5.0 us, x with
+// the right-hand side 17.3 -> 7.5, x inverse 5.8 -> 4.2; 128 x 97 x 64: 10.9 -> 6.8, 18.2 -> 9.5,
+// 6.4 -> 5.1.  At 256 x 192 x 256 (1536 and more) 256 threads take 48 and 39 us in z where 64 take 57
+// and 52 (a wavefront alone has 4 columns, 64 bytes, of each kz), and x does not depend on it.
+
+static bool rf_small(unsigned blocks256) {
+    return blocks256 < 512;
+}
+
+template <typename C, int N, int TH, bool INV>
+static hipError_t rf_zfft_t(hipStream_t st, const Dims &d, C *hat, const C *tw) {
+    using F = RFft<N, TH>;
+    const int nxh = d.nx / 2 + 1;
+    int cw = F::LPW < 16 ? F::LPW : 16;
+    while (cw > d.nx / 2) cw /= 2;
+    const int pw = F::LPW / cw, ntx = nxh / cw, nrem = nxh - ntx * cw;
+    const int tiles = ntx * ((d.ny + pw - 1) / pw), rem = (nrem * d.ny + F::LPW - 1) / F::LPW;
+    return rf_launch<C, N, TH, zfft_reg_kernel<C, N, TH, INV>>(st, (unsigned)(tiles + rem), d.ny, fft_stride_t<C>(d.nx), cw,
+                                                               ntx, tiles, nrem, tw, hat);
+}
+template <typename C, int N, bool INV>
+static hipError_t rf_zfft(hipStream_t st, const Dims &d, C *hat, const C *tw) {
+    return rf_small((unsigned)((d.nx / 2 + 1) * d.ny / RFft<N, 256>::LPW)) ? rf_zfft_t<C, N, 64, INV>(st, d, hat, tw)
+                                                                         : rf_zfft_t<C, N, 256, INV>(st, d, hat, tw);
+}
+// z-transform of the whole spectrum
+template <typename C, bool INV>
+static hipError_t launch_zfft(hipStream_t st, const Dims &d, C *hat, const C *tw) {
+#define ZF(N) return rf_zfft<C, N, INV>(st, d, hat, tw)
+    RF_SIZES(d.nz, ZF)
+#undef ZF
+    const int tx = z_tile(d.nz), nxh = d.nx / 2 + 1;
+    const size_t shz = fft_lds<C>(tx, d.nz + 1, d.nz);
+    hipError_t e = zfft_allow<C>(shz);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(zfft_kernel<C>, dim3(d.ny * ((nxh + tx - 1) / tx)), dim3(FFT_THREADS), shz, st, d, hat, tw, tx,
+                       INV ? 1 : 0, fft_stride_t<C>(d.nx));
+    return hipGetLastError();
+}
+
+static hipError_t launch_rhs_xfft(mdx_handle *h, double dtg) {
     GridK g = grid_k(h);
     const Dims d = h->d;
+    const int stride = fft_stride_t<double2>(d.nx);
+#define XF_(N, TH, W, S)                                                                                              \
+    return rf_launch<double2, N, TH, rhs_xfft_reg_kernel<N, TH, W, S>, W>(                                            \
+        h->stream, rf_row_blocks<N, TH>(d), g, (const double *)h->us, (const double *)h->vs, (const double *)h->ws, dtg, \
+        (const double2 *)h->tw_x, stride, (double2 *)h->hat)
+#define XF(N)                                                  \
+    if (rf_small(rf_row_blocks<N, 256>(d))) {                  \
+        if (h->stretched) XF_(N, 64, 4, true);                 \
+        XF_(N, 64, 4, false);                                  \
+    }                                                          \
+    if (h->stretched) XF_(N, 256, 1, true);                    \
+    XF_(N, 256, 1, false)
+    RF_SIZES(d.nx, XF)
+#undef XF
+#undef XF_
     const int lines = rows_per_block(d.nx);
     const int nrows = d.ny * d.nz;
     const size_t shx = fft_lds<double2>(lines, d.nx, d.nx);
     if (h->stretched)
         hipLaunchKernelGGL(rhs_xfft_kernel<true>, dim3((nrows + lines - 1) / lines), dim3(FFT_THREADS), shx,
-                           h->stream, g, h->us, h->vs, h->ws, dtg, (const double2 *)h->tw_x, lines,
+                           h->stream, g, h->us, h->vs, h->ws, dtg, (const double2 *)h->tw_x, lines, stride,
                            (double2 *)h->hat);
     else
         hipLaunchKernelGGL(rhs_xfft_kernel<false>, dim3((nrows + lines - 1) / lines), dim3(FFT_THREADS), shx,
-                           h->stream, g, h->us, h->vs, h->ws, dtg, (const double2 *)h->tw_x, lines,
+                           h->stream, g, h->us, h->vs, h->ws, dtg, (const double2 *)h->tw_x, lines, stride,
                            (double2 *)h->hat);
-    const int tx = z_tile(d.nz), nxh = d.nx / 2 + 1;
-    const size_t shz = fft_lds<double2>(tx, d.nz + 1, d.nz);
-    hipError_t e = zfft_allow<double2>(shz);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(zfft_kernel<double2>, dim3(d.ny * ((nxh + tx - 1) / tx)), dim3(FFT_THREADS), shz, h->stream, d,
-                       (double2 *)h->hat, (const double2 *)h->tw_z, tx, 0);
     return hipGetLastError();
+}
+
+static hipError_t launch_ixfft(mdx_handle *h, double *phi) {
+    const Dims d = h->d;
+    const int stride = fft_stride_t<double2>(d.nx);
+    const double scale = 1.0 / (double)(d.nx * d.nz);
+#define IX_(N, TH)                                                                                                  \
+    return rf_launch<double2, N, TH, ixfft_reg_kernel<N, TH>>(h->stream, rf_row_blocks<N, TH>(d), d, \
+                                                                              (const double2 *)h->hat,              \
+                                                                              (const double2 *)h->tw_x, stride,    \
+                                                                              scale, phi)
+#define IX(N)                                                \
+    if (rf_small(rf_row_blocks<N, 256>(d))) IX_(N, 64);      \
+    IX_(N, 256)
+    RF_SIZES(d.nx, IX)
+#undef IX
+#undef IX_
+    const int lines = rows_per_block(d.nx);
+    const int nrows = d.ny * d.nz;
+    const size_t shx = fft_lds<double2>(lines, d.nx, d.nx);
+    hipLaunchKernelGGL(ixfft_kernel, dim3((nrows + lines - 1) / lines), dim3(FFT_THREADS), shx, h->stream, d,
+                       (const double2 *)h->hat, (const double2 *)h->tw_x, lines, stride, scale, phi);
+    return hipGetLastError();
+}
+
+hipError_t launch_fft_forward(mdx_handle *h, double dtg) {
+    const hipError_t e = launch_rhs_xfft(h, dtg);
+    return e != hipSuccess ? e
+                           : launch_zfft<double2, false>(h->stream, h->d, (double2 *)h->hat, (const double2 *)h->tw_z);
 }
 
 hipError_t launch_tridiag(mdx_handle *h) {
@@ -787,26 +1276,17 @@ hipError_t launch_tridiag(mdx_handle *h) {
     if (h->wave_tridiag && launch_tridiag_wave<double2, false>(h->stream, d, (double2 *)h->hat, h->lamx, h->lamz, h->tw_a,
                                                      h->bdrow, h->crow))
         return hipGetLastError();
-    hipLaunchKernelGGL(tridiag_kernel, dim3((nlines + 63) / 64), dim3(64), 0, h->stream, d, (double2 *)h->hat,
-                       h->cp, h->den_inv, h->arow);
+    hipLaunchKernelGGL(tridiag_kernel, dim3((nlines + 63) / 64), dim3(64), 0, h->stream, d, fft_stride_t<double2>(d.nx),
+                       (double2 *)h->hat, h->cp, h->den_inv, h->arow);
     return hipGetLastError();
 }
 
 hipError_t launch_fft_backward_correct(mdx_handle *h, double dtg) {
     GridK g = grid_k(h);
     const Dims d = h->d;
-    const int tx = z_tile(d.nz), nxh = d.nx / 2 + 1;
-    const size_t shz = fft_lds<double2>(tx, d.nz + 1, d.nz);
-    hipError_t e = zfft_allow<double2>(shz);
+    hipError_t e = launch_zfft<double2, true>(h->stream, d, (double2 *)h->hat, (const double2 *)h->tw_z);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(zfft_kernel<double2>, dim3(d.ny * ((nxh + tx - 1) / tx)), dim3(FFT_THREADS), shz, h->stream, d,
-                       (double2 *)h->hat, (const double2 *)h->tw_z, tx, 1);
-    const int lines = rows_per_block(d.nx);
-    const int nrows = d.ny * d.nz;
-    const size_t shx = fft_lds<double2>(lines, d.nx, d.nx);
-    const double scale = 1.0 / (double)(d.nx * d.nz);
-    hipLaunchKernelGGL(ixfft_kernel, dim3((nrows + lines - 1) / lines), dim3(FFT_THREADS), shx, h->stream, d,
-                       (const double2 *)h->hat, (const double2 *)h->tw_x, lines, scale, h->fft_rhs);
+    if ((e = launch_ixfft(h, h->fft_rhs)) != hipSuccess) return e;
     dim3 blk(64, 4), grd((d.nx + 63) / 64, (d.ny + 3) / 4, d.nz);
 #define MDX_CORR(S, I)                                                                                     \
     hipLaunchKernelGGL((fft_correct_kernel<S, I>), grd, blk, 0, h->stream, g, h->fft_rhs, h->us, h->vs, h->ws, \
@@ -976,7 +1456,8 @@ __global__ __launch_bounds__(256) void fft_residual_kernel(GridK g, const double
 
 // 1. (FP32) r2c x-transform of a real FP64 field in (nx, nz, ny) layout
 __global__ __launch_bounds__(FFT_THREADS) void xfft32_kernel(Dims d, const double *__restrict__ in,
-                                                             const float2 *__restrict__ tw, int lines, float2 *hat) {
+                                                             const float2 *__restrict__ tw, int lines, int stride,
+                                                             float2 *hat) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     float2 *lds = reinterpret_cast<float2 *>(lds_raw);
     const int n = d.nx, nxh = n / 2 + 1;
@@ -993,21 +1474,21 @@ __global__ __launch_bounds__(FFT_THREADS) void xfft32_kernel(Dims d, const doubl
     for (int t = threadIdx.x; t < lines * nxh; t += FFT_THREADS) {
         const int line = t / nxh, m = t - line * nxh;
         const int r = blockIdx.x * lines + line;
-        if (r < nrows) hat[(size_t)nxh * r + m] = res[line * n + m];
+        if (r < nrows) hat[(size_t)stride * r + m] = res[line * n + m];
     }
 }
 
 // 3. (FP32) Thomas per (kx, kz) line with FP32 tables; the mean mode line is set to zero (it is
 //    solved in FP64 separately)
-__global__ __launch_bounds__(64) void tridiag32_kernel(Dims d, float2 *hat, const float *__restrict__ cp,
+__global__ __launch_bounds__(64) void tridiag32_kernel(Dims d, int stride, float2 *hat, const float *__restrict__ cp,
                                                        const float *__restrict__ den_inv,
                                                        const float *__restrict__ arow) {
     const int nxh = d.nx / 2 + 1, ny = d.ny, nz = d.nz;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nxh * nz) return;
     const int kx = t % nxh, kz = t / nxh;
-    const size_t hs = (size_t)nxh * nz, cs = (size_t)nxh;
-    const size_t h0 = (size_t)kx + (size_t)nxh * kz;
+    const size_t hs = (size_t)stride * nz, cs = (size_t)nxh;
+    const size_t h0 = (size_t)kx + (size_t)stride * kz;
     const size_t c0 = (size_t)kx + (size_t)nxh * (size_t)ny * kz;
     if (kx == 0 && kz == 0) {
         for (int jj = 1; jj <= ny; ++jj) hat[h0 + hs * (jj - 1)] = make_float2(0.f, 0.f);
@@ -1066,8 +1547,8 @@ __global__ __launch_bounds__(64) void tridiag32_kernel(Dims d, float2 *hat, cons
 
 // 5. (FP32) c2r x-transform, scaled, added to the FP64 phi
 __global__ __launch_bounds__(FFT_THREADS) void ixfft32_add_kernel(Dims d, const float2 *__restrict__ hat,
-                                                                  const float2 *__restrict__ tw, int lines, float scale,
-                                                                  double *phi) {
+                                                                  const float2 *__restrict__ tw, int lines, int stride,
+                                                                  float scale, double *phi) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     float2 *lds = reinterpret_cast<float2 *>(lds_raw);
     const int n = d.nx, nxh = n / 2 + 1;
@@ -1079,7 +1560,7 @@ __global__ __launch_bounds__(FFT_THREADS) void ixfft32_add_kernel(Dims d, const 
         const int r = blockIdx.x * lines + line;
         float2 v = make_float2(0.f, 0.f);
         if (r < nrows) {
-            const float2 *row = hat + (size_t)nxh * r;
+            const float2 *row = hat + (size_t)stride * r;
             if (m == 0 || 2 * m == n) v = make_float2(row[m].x, 0.f);
             else if (m < nxh) v = row[m];
             else v = make_float2(row[n - m].x, -row[n - m].y);
@@ -1122,6 +1603,48 @@ hipError_t launch_fft_residual(mdx_handle *h) {
     return e != hipSuccess ? e : launch_max_final(h, blocks);
 }
 
+// the FP32 x-transforms of the defect solves
+static hipError_t launch_xfft32(mdx_handle *h) {
+    const Dims d = h->d;
+    const int stride = fft_stride_t<float2>(d.nx);
+#define XF_(N, TH)                                                                                               \
+    return rf_launch<float2, N, TH, xfft32_reg_kernel<N, TH>>(h->stream, rf_row_blocks<N, TH>(d, 1), d,          \
+                                                              (const double *)h->fft_res,                        \
+                                                              (const float2 *)h->tw_x32, stride, (float2 *)h->hat32)
+#define XF(N)                                                \
+    if (rf_small(rf_row_blocks<N, 256>(d, 1))) XF_(N, 64);   \
+    XF_(N, 256)
+    RF_SIZES(d.nx, XF)
+#undef XF
+#undef XF_
+    const int lines = rows_per_block(d.nx), nrows = d.ny * d.nz;
+    hipLaunchKernelGGL(xfft32_kernel, dim3((nrows + lines - 1) / lines), dim3(FFT_THREADS),
+                       fft_lds<float2>(lines, d.nx, d.nx), h->stream, d, h->fft_res, (const float2 *)h->tw_x32, lines,
+                       stride, (float2 *)h->hat32);
+    return hipGetLastError();
+}
+
+static hipError_t launch_ixfft32_add(mdx_handle *h) {
+    const Dims d = h->d;
+    const int stride = fft_stride_t<float2>(d.nx);
+    const float scale = 1.0f / (float)(d.nx * d.nz);
+#define IX_(N, TH)                                                                                               \
+    return rf_launch<float2, N, TH, ixfft32_add_reg_kernel<N, TH>>(h->stream, rf_row_blocks<N, TH>(d, 1), d,     \
+                                                                   (const float2 *)h->hat32,                     \
+                                                                   (const float2 *)h->tw_x32, stride, scale, h->fft_phi)
+#define IX(N)                                                \
+    if (rf_small(rf_row_blocks<N, 256>(d, 1))) IX_(N, 64);   \
+    IX_(N, 256)
+    RF_SIZES(d.nx, IX)
+#undef IX
+#undef IX_
+    const int lines = rows_per_block(d.nx), nrows = d.ny * d.nz;
+    hipLaunchKernelGGL(ixfft32_add_kernel, dim3((nrows + lines - 1) / lines), dim3(FFT_THREADS),
+                       fft_lds<float2>(lines, d.nx, d.nx), h->stream, d, (const float2 *)h->hat32,
+                       (const float2 *)h->tw_x32, lines, stride, scale, h->fft_phi);
+    return hipGetLastError();
+}
+
 // one defect-correction pass on res = rhs - L phi: the mean mode in FP64 (plane sums, pinned
 // Thomas), the other modes by FP32 transforms and Thomas; both corrections added to h->fft_phi
 hipError_t launch_fft32_solve_add(mdx_handle *h) {
@@ -1133,30 +1656,21 @@ hipError_t launch_fft32_solve_add(mdx_handle *h) {
     hipLaunchKernelGGL(fft_mean_mode_kernel, dim3(1), dim3(256), 0, h->stream, d, h->fft_mean, h->cp, h->den_inv,
                        h->arow, 1.0 / (double)(d.nx * d.nz), mean);
     hipLaunchKernelGGL(fft_add_mean_kernel, dim3(4096), dim3(256), 0, h->stream, d, mean, h->fft_phi);
-    const int lines = rows_per_block(d.nx), nrows = d.ny * d.nz, nxh = d.nx / 2 + 1;
-    const size_t shx = fft_lds<float2>(lines, d.nx, d.nx);
-    hipLaunchKernelGGL(xfft32_kernel, dim3((nrows + lines - 1) / lines), dim3(FFT_THREADS), shx, h->stream, d,
-                       h->fft_res, (const float2 *)h->tw_x32, lines, (float2 *)h->hat32);
-    const int tx = z_tile(d.nz);
-    const size_t shz = fft_lds<float2>(tx, d.nz + 1, d.nz);
-    hipError_t ez = zfft_allow<float2>(shz);
-    if (ez != hipSuccess) return ez;
-    hipLaunchKernelGGL(zfft_kernel<float2>, dim3(d.ny * ((nxh + tx - 1) / tx)), dim3(FFT_THREADS), shz, h->stream, d,
-                       (float2 *)h->hat32, (const float2 *)h->tw_z32, tx, 0);
-    const int nlines = nxh * d.nz;
+    hipError_t e = launch_xfft32(h);
+    if (e != hipSuccess) return e;
+    if ((e = launch_zfft<float2, false>(h->stream, d, (float2 *)h->hat32, (const float2 *)h->tw_z32)) != hipSuccess)
+        return e;
+    const int nlines = (d.nx / 2 + 1) * d.nz;
     if (!(h->wave_tridiag && h->part_tridiag &&
           launch_tridiag_part<float2, true>(h->stream, d, (float2 *)h->hat32, h->lamx32, h->lamz32, h->tw_a32,
                                             h->bdrow32, h->crow32)) &&
         !(h->wave_tridiag && launch_tridiag_wave<float2, true>(h->stream, d, (float2 *)h->hat32, h->lamx32, h->lamz32,
                                                      h->tw_a32, h->bdrow32, h->crow32)))
-        hipLaunchKernelGGL(tridiag32_kernel, dim3((nlines + 63) / 64), dim3(64), 0, h->stream, d, (float2 *)h->hat32,
-                           h->cp32, h->den32, h->arow32);
-    hipLaunchKernelGGL(zfft_kernel<float2>, dim3(d.ny * ((nxh + tx - 1) / tx)), dim3(FFT_THREADS), shz, h->stream, d,
-                       (float2 *)h->hat32, (const float2 *)h->tw_z32, tx, 1);
-    hipLaunchKernelGGL(ixfft32_add_kernel, dim3((nrows + lines - 1) / lines), dim3(FFT_THREADS), shx, h->stream, d,
-                       (const float2 *)h->hat32, (const float2 *)h->tw_x32, lines, 1.0f / (float)(d.nx * d.nz),
-                       h->fft_phi);
-    return hipGetLastError();
+        hipLaunchKernelGGL(tridiag32_kernel, dim3((nlines + 63) / 64), dim3(64), 0, h->stream, d,
+                           fft_stride_t<float2>(d.nx), (float2 *)h->hat32, h->cp32, h->den32, h->arow32);
+    if ((e = launch_zfft<float2, true>(h->stream, d, (float2 *)h->hat32, (const float2 *)h->tw_z32)) != hipSuccess)
+        return e;
+    return launch_ixfft32_add(h);
 }
 
 hipError_t launch_fft_pin(mdx_handle *h) {

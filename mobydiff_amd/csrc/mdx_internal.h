@@ -409,6 +409,7 @@ size_t rb_xlist_bytes(const RbPlanOut &p);
 hipError_t rb_build_xlists(mdx_handle *h, const RbPlanOut &p, int *xl);
 
 // FFT path
+int fft_stride(int nx, bool fp32);   // complex elements per kx row of the spectrum
 hipError_t launch_fft_forward(mdx_handle *h, double dtg);
 hipError_t launch_tridiag(mdx_handle *h);
 hipError_t launch_fft_backward_correct(mdx_handle *h, double dtg);

@@ -1801,15 +1801,20 @@ extern "C" int mdx_step(mdx_handle *h, double dt, mdx_step_stats *stats) {
         ev_record(h, 0);
         if (h->cfg.flowrate && h->fr_part) {
             // momentum forms the flow-rate partial sums of u*; one launch folds them, shifts u* and
-            // builds the stage's face-coefficient tables if the solve needs new ones
+            // builds the stage's face-coefficient tables if the solve needs new ones (with the FFT
+            // and no body the shift is uniform, and the projection's last pass makes it)
             MDX_HIP(launch_momentum(h, dta, dtb, dtg, h->fr_part));
             ev_record(h, 5);
-            // (the tables exist for the SOR solver only)
-            const bool tables = h->fused_mu && h->ibm_on && h->mu_dtg != dtg && h->cfg.solver == MDX_SOLVER_SOR &&
-                                h->mu64[0] && h->mu32[0];
-            MDX_HIP(launch_flow_fold(h, dtg, h->fr_part, momentum_tiles(h), h->red_part + 2048,
-                                     tables ? mu_build(h, dtg) : MuBuild{}));
-            if (tables) h->mu_dtg = dtg;
+            if (h->cfg.solver == MDX_SOLVER_FFT && !h->ibm_on) {
+                h->step_parts = momentum_tiles(h);
+            } else {
+                // (the tables exist for the SOR solver only)
+                const bool tables = h->fused_mu && h->ibm_on && h->mu_dtg != dtg &&
+                                    h->cfg.solver == MDX_SOLVER_SOR && h->mu64[0] && h->mu32[0];
+                MDX_HIP(launch_flow_fold(h, dtg, h->fr_part, momentum_tiles(h), h->red_part + 2048,
+                                         tables ? mu_build(h, dtg) : MuBuild{}));
+                if (tables) h->mu_dtg = dtg;
+            }
         } else {
             if ((rc = mdx_momentum(h, dta, dtb, dtg))) return rc;
             ev_record(h, 5);
@@ -1817,20 +1822,25 @@ extern "C" int mdx_step(mdx_handle *h, double dt, mdx_step_stats *stats) {
         }
         // the predictor's arrays are the only ones written since the last call (the current
         // fields' ghosts are those of the previous stage's projection or of the upload)
-        if (h->cfg.solver == MDX_SOLVER_FFT) MDX_HIP(launch_apply_bc_fft(h, BC_S));
+        // (the FFT's projection takes their ghosts as filled: the fill itself waits for the last one)
+        const bool fft = h->cfg.solver == MDX_SOLVER_FFT;
+        if (fft && !h->fused_bc) MDX_HIP(launch_apply_bc_fft(h, BC_S));
         mdx_solve_stats st{};
         h->proj_count = s;   // RK stage of this projection (initial-guess history)
         // the fill follows the projection at once: its kernel may write the boundary conditions
         h->step_bc = true;
+        h->step_last = s == 2;
         h->apply_wrote_bc = false;
         rc = mdx_pressure_projection(h, dtg, &st);
         h->step_bc = false;
+        h->step_parts = 0;
         if (rc) {
             if (stats) stats->stage[s] = st;
             return rc;
         }
         if (h->apply_wrote_bc) h->apply_wrote_bc = false;
         else if ((rc = post_bc(h))) return rc;
+        if (fft && h->fused_bc && s == 2) MDX_HIP(launch_apply_bc_fft(h, BC_S));
         ev_record(h, 4);
         if (stats) stats->stage[s] = st;
         h->ph_skip = false;

@@ -106,8 +106,8 @@ __device__ inline void stage_twiddles(C *dst, const C *__restrict__ tw, int n) {
 // loads and last stores are its own points, so no staging either.  LDS addresses are padded by one
 // element in 16, which keeps the radix-16 scatter (16 elements apart) and the gather (consecutive)
 // free of bank conflicts.  At 256 x 192 x 256 in FP64 the LDS kernels took 129 us (x, with the
-// right-hand side), 94 us (z, either way) and 89 us (x inverse); these take 99, 50 (42 inverse) and
-// 35 us, which is 4 to 5 TB/s of the fields and the spectrum read and written once.  In FP32: 49 us
+// right-hand side), 94 us (z, either way) and 89 us (x inverse); these take 99 (116 with u* not in a
+// cache), 41 (38 inverse) and 35 us, 4 to 5 TB/s of the fields and the spectrum read and written once.  In FP32: 49 us
 // (x), 62 (z) and 62 (x inverse, adding to phi) before, 25, 31 (24 inverse) and 40 now.
 template <typename C, bool INV> __device__ inline C ctw(C a, C w) {   // a w (forward) or a conj(w)
     const typename Cx<C>::R wi = INV ? -w.y : w.y;
@@ -308,11 +308,13 @@ __device__ inline double div_by(double a, double d, double r) {
     return fma(fma(-q, d, a), r, q);
 }
 
-// 1. rhs(i,k,j) = div u* / dtg and the forward x-transform, two rows (planes k, k + 1) per line
+// 1. rhs(i,k,j) = div u* / dtg and the forward x-transform, two rows (planes k, k + 1) per line.
+//    wrap: u*'s ghosts are taken as apply_bc fills them (periodic in x and z, v* = 0 on the walls)
+//    instead of read; inside a step nothing else reads them, so their fill is left to its end.
 template <int N, int TH, int W, bool STRETCH>
 __global__ __launch_bounds__(TH * W) void rhs_xfft_reg_kernel(GridK g, const double *__restrict__ us,
                                                               const double *__restrict__ vs,
-                                                              const double *__restrict__ ws, double dtg,
+                                                              const double *__restrict__ ws, double dtg, int wrap,
                                                               const double2 *__restrict__ tw, int stride,
                                                               double2 *__restrict__ hat) {
     using F = RFft<N, TH>;
@@ -333,12 +335,17 @@ __global__ __launch_bounds__(TH * W) void rhs_xfft_reg_kernel(GridK g, const dou
             const size_t c0 = d.g(1 + i, j, k);
             const double *u = us + c0, *v = vs + c0, *w = ws + c0;
             const double w1 = w[sz], ih = STRETCH ? g.ihc[j] : 0.0;
+            const int up = wrap && i == N - 1 ? 1 - N : 1;
+            const double w2 = wrap && k + 1 == d.nz ? (w - (size_t)(k - 1) * sz)[0] : w[2 * sz];
+            double va = v[0], vb = v[sz], vc = v[sy], vd = v[sz + sy];
+            if (wrap && j == 1) va = vb = 0.0;
+            if (wrap && j == d.ny) vc = vd = 0.0;
             auto rhs = [&](double du, double dv, double dw) {
                 const double dy = STRETCH ? dv * ih : div_by(dv, g.dy, iy);
                 return div_by(div_by(du, g.dx, ix) + dy + div_by(dw, g.dz, iz), dtg, it);
             };
-            r.x = rhs(u[1] - u[0], v[sy] - v[0], w1 - w[0]);
-            r.y = rhs(u[sz + 1] - u[sz], v[sz + sy] - v[sz], w[2 * sz] - w1);
+            r.x = rhs(u[up] - u[0], vc - va, w1 - w[0]);
+            r.y = rhs(u[sz + up] - u[sz], vd - vb, w2 - w1);
         }
         lds[(size_t)ll * F::LS + rf_pad(i)] = r;
     }
@@ -471,7 +478,7 @@ __global__ __launch_bounds__(TH) void zfft_reg_kernel(int ny, int stride, int cw
 template <bool STRETCH>
 __global__ __launch_bounds__(FFT_THREADS) void rhs_xfft_kernel(GridK g, const double *__restrict__ us,
                                                               const double *__restrict__ vs,
-                                                              const double *__restrict__ ws, double dtg,
+                                                              const double *__restrict__ ws, double dtg, int wrap,
                                                               const double2 *__restrict__ tw, int lines,
                                                               int stride, double2 *hat) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -487,10 +494,11 @@ __global__ __launch_bounds__(FFT_THREADS) void rhs_xfft_kernel(GridK g, const do
         double v = 0.0;
         if (r < nrows) {
             const int k = r % d.nz + 1, j = r / d.nz + 1;
-            const double dv = STRETCH ? (vs[d.g(i, j + 1, k)] - vs[d.g(i, j, k)]) * g.ihc[j]
-                                      : (vs[d.g(i, j + 1, k)] - vs[d.g(i, j, k)]) / g.dy;
-            v = ((us[d.g(i + 1, j, k)] - us[d.g(i, j, k)]) / g.dx + dv +
-                 (ws[d.g(i, j, k + 1)] - ws[d.g(i, j, k)]) / g.dz) / dtg;
+            const int ip = wrap && i == n ? 1 : i + 1, kp = wrap && k == d.nz ? 1 : k + 1;
+            const double vn = wrap && j == d.ny ? 0.0 : vs[d.g(i, j + 1, k)], vc = wrap && j == 1 ? 0.0 : vs[d.g(i, j, k)];
+            const double dv = STRETCH ? (vn - vc) * g.ihc[j] : (vn - vc) / g.dy;
+            v = ((us[d.g(ip, j, k)] - us[d.g(i, j, k)]) / g.dx + dv +
+                 (ws[d.g(i, j, kp)] - ws[d.g(i, j, k)]) / g.dz) / dtg;
         }
         a[t] = make_double2(v, 0.0);
     }
@@ -1066,37 +1074,179 @@ __global__ __launch_bounds__(FFT_THREADS) void ixfft_kernel(Dims d, const double
 // workgroup shape of the k-marching fft_div_rhs_kernel: 64 x FC_Y cells, FC_KZ planes
 static constexpr int FC_Y = 4, FC_KZ = 16;
 
-// 6. pressure_solver.f90:150-169
+// a plane's sum from the partial sums of fft_plane_sum_kernel
+static constexpr int PLANE_CHUNKS = 16;
+__device__ inline double plane_sum(const double *part, int j) {
+    double a = 0.0;
+    for (int c = 0; c < PLANE_CHUNKS; ++c) a += part[j * PLANE_CHUNKS + c];
+    return a;
+}
+
+// 6. u = (u* - dtg grad phi)/(1 + dtg coef) and p += phi (pressure_solver.f90:129-173).  Each thread
+// takes one column (i,j) of a 64 x 4 tile and marches `kz` planes, FC_CH planes' loads in flight at
+// a time (phi(k-1) stays in a register).  Inside a step (FftStep) the same pass also
+//   * shifts u* by the flow-rate correction, folded here from the partial sums in every workgroup's
+//     own order-fixed way (a uniform shift drops out of the divergence, so the right-hand side does
+//     not need it; a pass of its own read and wrote u* once more, 54 us at 256 x 192 x 256), and
+//     stores it if the step leaves u* visible (store_us);
+//   * writes the ghosts of the new fields as apply_bc fills them, from the cells at the boundary
+//     (the separate fill took three launches and 31 us, 10 at 64^3).
+// pin: the plane sums whose mean (plane 1) is taken off phi, where the solve leaves that to this pass.
+// Bound by HBM: 9 arrays once, 72 B per cell.
+static constexpr int FC_CH = 4;
+struct FftStep {
+    const double *part = nullptr;   // flow-rate partial sums, nparts pairs (none: no shift)
+    int nparts = 0;
+    double norm = 1.0, target = 0.0;
+    double *out = nullptr;          // bulk velocity, mean mu_u, du
+    int store_us = 0, ghosts = 0;
+    const double *pin = nullptr;
+};
 template <bool STRETCH, bool IBM>
-__global__ __launch_bounds__(256) void fft_correct_kernel(GridK g, const double *__restrict__ phi,
-                                                          const double *__restrict__ us,
+__global__ __launch_bounds__(256) void fft_correct_kernel(GridK g, const double *__restrict__ phi, double *us,
                                                           const double *__restrict__ vs,
                                                           const double *__restrict__ ws,
                                                           const double *__restrict__ cu,
                                                           const double *__restrict__ cv,
-                                                          const double *__restrict__ cw, double dtg,
-                                                          double *un, double *vn, double *wn, double *pn) {
+                                                          const double *__restrict__ cw, double dtg, int kz,
+                                                          FftStep fs, double *un, double *vn, double *wn, double *pn) {
     const Dims d = g.d;
-    const int i = blockIdx.x * 64 + threadIdx.x + 1;
-    const int j = blockIdx.y * 4 + threadIdx.y + 1;
-    const int k = blockIdx.z + 1;
-    if (i > d.nx || j > d.ny) return;
-    const int nx = d.nx, nz = d.nz;
-    int im = i - 1, km = k - 1;
-    if (im < 1) im = nx;
-    if (km < 1) km = nz;
-#define RI(ii, kk, jj) ((size_t)((ii) - 1) + (size_t)nx * ((size_t)((kk) - 1) + (size_t)nz * (size_t)((jj) - 1)))
-    const size_t c = d.g(i, j, k);
-    const double p0 = phi[RI(i, k, j)];
-    un[c] = (us[c] - dtg * (p0 - phi[RI(im, k, j)]) / g.dx) / (1.0 + dtg * (IBM ? cu[c] : 0.0));
-    wn[c] = (ws[c] - dtg * (p0 - phi[RI(i, km, j)]) / g.dz) / (1.0 + dtg * (IBM ? cw[c] : 0.0));
-    pn[c] = pn[c] + p0;
-    if (j >= 2) {
-        const double gy = STRETCH ? dtg * (p0 - phi[RI(i, k, j - 1)]) * g.ihv[j]
-                                  : dtg * (p0 - phi[RI(i, k, j - 1)]) / g.dy;
-        vn[c] = (vs[c] - gy) / (1.0 + dtg * (IBM ? cv[c] : 0.0));
+    int tx, ty, tz;
+    if (!xcd_tile(d.nx, d.ny, (d.nz + kz - 1) / kz, 64, 4, tx, ty, tz)) return;   // uniform per workgroup
+    const int nx = d.nx, ny = d.ny, nz = d.nz;
+    const int i0 = tx * 64 + threadIdx.x + 1, j0 = ty * 4 + threadIdx.y + 1;
+    const int i = i0 < nx ? i0 : nx, j = j0 < ny ? j0 : ny;   // threads past the grid load the last cells'
+    const int k0 = tz * kz + 1, k1 = k0 + kz - 1 < nz ? k0 + kz - 1 : nz;
+    const size_t sz = (size_t)d.sx * d.sy;
+    const double rx = 1.0 / g.dx, ry = 1.0 / g.dy, rz = 1.0 / g.dz, ih = STRETCH ? g.ihv[j] : 0.0;
+    // phi(i,k,j) in (nx, nz, ny) layout, its x neighbour and the row below
+    const double *p = phi + (size_t)(i - 1) + (size_t)nx * ((size_t)(k0 - 1) + (size_t)nz * (size_t)(j - 1));
+    const ptrdiff_t om = i == 1 ? nx - 1 : -1, oj = j >= 2 ? -(ptrdiff_t)nx * nz : 0;
+    size_t c = d.g(i, j, k0);
+    double pp[FC_CH], px[FC_CH], py[FC_CH], a[FC_CH], b[FC_CH], e[FC_CH], q[FC_CH];
+    auto load = [&](int k) {   // planes k .. k + FC_CH - 1 (past the end: the last one again, unused)
+#pragma unroll
+        for (int u = 0; u < FC_CH; ++u) {
+            const int w = k + u <= k1 ? u : k1 - k;
+            const size_t cc = c + w * sz;
+            pp[u] = p[w * (ptrdiff_t)nx];
+            px[u] = p[w * (ptrdiff_t)nx + om];
+            py[u] = p[w * (ptrdiff_t)nx + oj];
+            a[u] = us[cc];
+            b[u] = j >= 2 ? vs[cc] : 0.0;
+            e[u] = ws[cc];
+            q[u] = pn[cc];
+        }
+    };
+    load(k0);   // before the folds, whose loads and barriers take as long
+    const double pkm = k0 > 1 ? p[-(ptrdiff_t)nx] : p[(ptrdiff_t)nx * (nz - k0)];
+    double du = 0.0;
+    if (fs.part) {
+        __shared__ double s1[256], s2[256];
+        double o[3];
+        flow_fold(fs.part, fs.nparts, fs.norm, fs.target, threadIdx.x + 64 * threadIdx.y, s1, s2, o);
+        du = o[2];
+        if (blockIdx.x == 0 && threadIdx.x + threadIdx.y == 0) {
+            fs.out[0] = o[0];
+            fs.out[1] = o[1];
+            fs.out[2] = o[2];
+        }
     }
-#undef RI
+    const double pc = fs.pin ? plane_sum(fs.pin, 0) / (double)((long)nx * nz) : 0.0;
+    if (i0 > nx || j0 > ny) return;
+    double pm = pkm - pc;
+    const int xi = i == nx ? -nx : i == 1 ? nx : 0;   // to the column's x image, if it has one
+    auto put = [&](double *f, size_t cc, double v, ptrdiff_t zi) {   // a value and its periodic images
+        f[cc] = v;
+        if (!fs.ghosts) return;
+        if (xi) f[cc + xi] = v;
+        if (zi) {
+            f[cc + zi] = v;
+            if (xi) f[cc + zi + xi] = v;
+        }
+    };
+    for (int k = k0;;) {
+#pragma unroll
+        for (int u = 0; u < FC_CH; ++u) {
+            if (k + u > k1) break;
+            const size_t cc = c + u * sz;
+            const ptrdiff_t zi = k + u == nz ? -(ptrdiff_t)(nz * sz) : k + u == 1 ? (ptrdiff_t)(nz * sz) : 0;
+            const double p0 = pp[u] - pc;
+            if (fs.part) {
+                a[u] = a[u] + du;
+                if (fs.store_us) us[cc] = a[u];
+            }
+            double U = a[u] - div_by(dtg * (p0 - (px[u] - pc)), g.dx, rx);
+            double W = e[u] - div_by(dtg * (p0 - pm), g.dz, rz);
+            const double gy = dtg * (p0 - (py[u] - pc));
+            double V = b[u] - (STRETCH ? gy * ih : div_by(gy, g.dy, ry));
+            if (IBM) {
+                U = U / (1.0 + dtg * cu[cc]);
+                W = W / (1.0 + dtg * cw[cc]);
+                V = V / (1.0 + dtg * cv[cc]);
+            }
+            put(un, cc, U, zi);
+            put(wn, cc, W, zi);
+            put(pn, cc, q[u] + p0, zi);
+            if (j >= 2) put(vn, cc, V, zi);
+            if (fs.ghosts) {
+                if (j == 1) {
+                    put(un, cc - d.sx, -U, zi);
+                    put(wn, cc - d.sx, -W, zi);
+                    put(vn, cc, 0.0, zi);
+                }
+                if (j == ny) {
+                    put(un, cc + d.sx, -U, zi);
+                    put(wn, cc + d.sx, -W, zi);
+                    put(vn, cc + d.sx, 0.0, zi);
+                }
+            }
+            pm = p0;
+        }
+        k += FC_CH;
+        if (k > k1) break;
+        c += FC_CH * sz;
+        p += FC_CH * (ptrdiff_t)nx;
+        load(k);
+    }
+}
+
+// whether the projection takes u*'s ghosts as filled and writes the new fields' itself
+static int fft_wrap(const mdx_handle *h) { return h->step_bc && h->fused_bc; }
+
+// the flow-rate shift the projection of a step makes
+static FftStep fft_step(const mdx_handle *h) {
+    FftStep fs;
+    if (!h->step_bc || !h->step_parts) return fs;
+    fs.part = h->fr_part;
+    fs.nparts = h->step_parts;
+    fs.norm = (double)h->d.nx * (double)h->d.nz * h->cfg.flow_height;
+    fs.target = h->cfg.ub_target;
+    fs.out = h->red_part + 2048;
+    fs.store_us = h->step_last;
+    return fs;
+}
+
+// Planes per workgroup of the correction: up to 16 (the phi(k-1) loads and the folds are per
+// workgroup), down to one chunk while the workgroups would not give every CU four: 7.5 us at 64^3
+// with 4 planes against 9.9 with 1; 214 us at 256 x 192 x 256 with 4 as with 16 or 32.
+static hipError_t launch_correct(mdx_handle *h, const double *phi, double dtg, const double *pin) {
+    GridK g = grid_k(h);
+    const Dims d = h->d;
+    int kz = 16;
+    while (kz > FC_CH && xcd_grid(d.nx, d.ny, (d.nz + kz - 1) / kz, 64, 4) < 1024) kz /= 2;
+    FftStep fs = fft_step(h);
+    fs.ghosts = fft_wrap(h);
+    fs.pin = pin;
+#define MDX_CORR(S, I)                                                                                             \
+    hipLaunchKernelGGL((fft_correct_kernel<S, I>), dim3(xcd_grid(d.nx, d.ny, (d.nz + kz - 1) / kz, 64, 4)),        \
+                       dim3(64, 4), 0, h->stream, g, phi, h->us, h->vs, h->ws, h->cu, h->cv, h->cw, dtg, kz, fs,   \
+                       h->un, h->vn, h->wn, h->pn)
+    if (h->stretched) { if (h->ibm_on) MDX_CORR(true, true); else MDX_CORR(true, false); }
+    else { if (h->ibm_on) MDX_CORR(false, true); else MDX_CORR(false, false); }
+#undef MDX_CORR
+    h->apply_wrote_bc = fs.ghosts;
+    return hipGetLastError();
 }
 
 static int rows_per_block(int n) {
@@ -1167,9 +1317,9 @@ static unsigned rf_row_blocks(const Dims &d, int rows = 2) {   // rows: rows per
 // three that only load and store) where those of 256 would leave CUs without two: `blocks256` is the
 // number of the latter.  Measured at 64^3 (32 to 36 workgroups of 256): z 10.2 us -> 5.0 us, x with
 // the right-hand side 17.3 -> 7.5, x inverse 5.8 -> 4.2; 128 x 97 x 64: 10.9 -> 6.8, 18.2 -> 9.5,
-// 6.4 -> 5.1.  At 256 x 192 x 256 (1536 and more) 256 threads take 48 and 39 us in z where 64 take 57
-// and 52 (a wavefront alone has 4 columns, 64 bytes, of each kz), and x does not depend on it.
-
+// 6.4 -> 5.1.  At 256 x 192 x 256 (1536 and more) x does not depend on it; in z a wavefront alone has
+// 4 columns, 64 bytes, of each kz: FP64 56 and 51 us against 48 and 42 with 256 threads and 41 and 38
+// with the 128 taken there, whose 8 columns are one cache line (FP32: 16 columns, 256 threads).
 static bool rf_small(unsigned blocks256) {
     return blocks256 < 512;
 }
@@ -1188,7 +1338,7 @@ static hipError_t rf_zfft_t(hipStream_t st, const Dims &d, C *hat, const C *tw) 
 template <typename C, int N, bool INV>
 static hipError_t rf_zfft(hipStream_t st, const Dims &d, C *hat, const C *tw) {
     return rf_small((unsigned)((d.nx / 2 + 1) * d.ny / RFft<N, 256>::LPW)) ? rf_zfft_t<C, N, 64, INV>(st, d, hat, tw)
-                                                                         : rf_zfft_t<C, N, 256, INV>(st, d, hat, tw);
+                                                                         : rf_zfft_t<C, N, sizeof(C) == 16 ? 128 : 256, INV>(st, d, hat, tw);
 }
 // z-transform of the whole spectrum
 template <typename C, bool INV>
@@ -1212,7 +1362,7 @@ static hipError_t launch_rhs_xfft(mdx_handle *h, double dtg) {
 #define XF_(N, TH, W, S)                                                                                              \
     return rf_launch<double2, N, TH, rhs_xfft_reg_kernel<N, TH, W, S>, W>(                                            \
         h->stream, rf_row_blocks<N, TH>(d), g, (const double *)h->us, (const double *)h->vs, (const double *)h->ws, dtg, \
-        (const double2 *)h->tw_x, stride, (double2 *)h->hat)
+        fft_wrap(h), (const double2 *)h->tw_x, stride, (double2 *)h->hat)
 #define XF(N)                                                  \
     if (rf_small(rf_row_blocks<N, 256>(d))) {                  \
         if (h->stretched) XF_(N, 64, 4, true);                 \
@@ -1228,11 +1378,11 @@ static hipError_t launch_rhs_xfft(mdx_handle *h, double dtg) {
     const size_t shx = fft_lds<double2>(lines, d.nx, d.nx);
     if (h->stretched)
         hipLaunchKernelGGL(rhs_xfft_kernel<true>, dim3((nrows + lines - 1) / lines), dim3(FFT_THREADS), shx,
-                           h->stream, g, h->us, h->vs, h->ws, dtg, (const double2 *)h->tw_x, lines, stride,
+                           h->stream, g, h->us, h->vs, h->ws, dtg, fft_wrap(h), (const double2 *)h->tw_x, lines, stride,
                            (double2 *)h->hat);
     else
         hipLaunchKernelGGL(rhs_xfft_kernel<false>, dim3((nrows + lines - 1) / lines), dim3(FFT_THREADS), shx,
-                           h->stream, g, h->us, h->vs, h->ws, dtg, (const double2 *)h->tw_x, lines, stride,
+                           h->stream, g, h->us, h->vs, h->ws, dtg, fft_wrap(h), (const double2 *)h->tw_x, lines, stride,
                            (double2 *)h->hat);
     return hipGetLastError();
 }
@@ -1282,19 +1432,11 @@ hipError_t launch_tridiag(mdx_handle *h) {
 }
 
 hipError_t launch_fft_backward_correct(mdx_handle *h, double dtg) {
-    GridK g = grid_k(h);
     const Dims d = h->d;
     hipError_t e = launch_zfft<double2, true>(h->stream, d, (double2 *)h->hat, (const double2 *)h->tw_z);
     if (e != hipSuccess) return e;
     if ((e = launch_ixfft(h, h->fft_rhs)) != hipSuccess) return e;
-    dim3 blk(64, 4), grd((d.nx + 63) / 64, (d.ny + 3) / 4, d.nz);
-#define MDX_CORR(S, I)                                                                                     \
-    hipLaunchKernelGGL((fft_correct_kernel<S, I>), grd, blk, 0, h->stream, g, h->fft_rhs, h->us, h->vs, h->ws, \
-                       h->cu, h->cv, h->cw, dtg, h->un, h->vn, h->wn, h->pn)
-    if (h->stretched) { if (h->ibm_on) MDX_CORR(true, true); else MDX_CORR(true, false); }
-    else { if (h->ibm_on) MDX_CORR(false, true); else MDX_CORR(false, false); }
-#undef MDX_CORR
-    return hipGetLastError();
+    return launch_correct(h, h->fft_rhs, dtg, nullptr);
 }
 
 // ------------------------------------------------------------------------------- mixed precision
@@ -1307,13 +1449,23 @@ hipError_t launch_fft_backward_correct(mdx_handle *h, double dtg) {
 // rhs(i,k,j) of rhs_xfft_kernel, in FP64, layout (nx, nz, ny).  A 64 x FC_Y workgroup owns rows
 // j0 .. j0+FC_Y-1 of a 64-cell x segment and marches FC_KZ planes: w*(k+1) becomes w*(k) of the
 // next plane in a register and u*(i+1) comes from the lane above (lane 63 reads it), so w* and u*
-// are fetched about once; v*(j+1) is the row above's v*(j) (a cache hit).
+// are fetched about once; v*(j+1) is the row above's v*(j) (a cache hit).  wrap: as in
+// rhs_xfft_reg_kernel; fs: the flow-rate shift of u*, added before the differences (it drops out of
+// them but for rounding, which the FP32 passes would turn into differences of their own precision).
 template <bool STRETCH>
 __global__ __launch_bounds__(64 * FC_Y) void fft_div_rhs_kernel(GridK g, const double *__restrict__ us,
                                                                const double *__restrict__ vs,
-                                                               const double *__restrict__ ws, double dtg,
-                                                               double *__restrict__ rhs) {
+                                                               const double *__restrict__ ws, double dtg, int wrap,
+                                                               FftStep fs, double *__restrict__ rhs) {
+    static_assert(64 * FC_Y == 256, "the fold's threads");
     const Dims d = g.d;
+    double du = 0.0;
+    if (fs.part) {
+        __shared__ double s1[256], s2[256];
+        double o[3];
+        flow_fold(fs.part, fs.nparts, fs.norm, fs.target, threadIdx.x + 64 * threadIdx.y, s1, s2, o);
+        du = o[2];
+    }
     const int lane = threadIdx.x;
     const int i = blockIdx.x * 64 + lane + 1;
     const int j = blockIdx.y * FC_Y + threadIdx.y + 1;
@@ -1324,12 +1476,16 @@ __global__ __launch_bounds__(64 * FC_Y) void fft_div_rhs_kernel(GridK g, const d
         double uc = 0.0, up = 0.0, vj = 0.0, vjp = 0.0, wkp = 0.0;
         if (act) {
             uc = us[d.g(i, j, k)];
-            vj = vs[d.g(i, j, k)];
-            vjp = vs[d.g(i, j + 1, k)];
-            wkp = ws[d.g(i, j, k + 1)];
+            if (fs.part) uc = uc + du;
+            vj = wrap && j == 1 ? 0.0 : vs[d.g(i, j, k)];
+            vjp = wrap && j == d.ny ? 0.0 : vs[d.g(i, j + 1, k)];
+            wkp = ws[d.g(i, j, wrap && k == d.nz ? 1 : k + 1)];
         }
         up = __shfl_down(uc, 1, 64);
-        if (act && (lane == 63 || i == d.nx)) up = us[d.g(i + 1, j, k)];
+        if (act && (lane == 63 || i == d.nx)) {
+            up = us[d.g(wrap && i == d.nx ? 1 : i + 1, j, k)];
+            if (fs.part) up = up + du;
+        }
         if (act) {
             const double dv = STRETCH ? (vjp - vj) * g.ihc[j] : (vjp - vj) / g.dy;
             rhs[(size_t)(i - 1) + (size_t)d.nx * ((size_t)(k - 1) + (size_t)d.nz * (size_t)(j - 1))] =
@@ -1339,10 +1495,8 @@ __global__ __launch_bounds__(64 * FC_Y) void fft_div_rhs_kernel(GridK g, const d
     }
 }
 
-// sums[j-1] = sum over the (x, z) plane j of rhs (one workgroup per plane, fixed order)
 // partial sums of the (nx, nz) planes: workgroup (plane j, chunk c) sums chunk c of PLANE_CHUNKS
 // equal parts of plane j into part[j * PLANE_CHUNKS + c]; consumers fold a plane's chunks in order
-static constexpr int PLANE_CHUNKS = 16;
 __global__ __launch_bounds__(256) void fft_plane_sum_kernel(Dims d, const double *__restrict__ rhs, double *part) {
     __shared__ double s[256];
     const long plane = (long)d.nx * d.nz;
@@ -1358,12 +1512,6 @@ __global__ __launch_bounds__(256) void fft_plane_sum_kernel(Dims d, const double
         __syncthreads();
     }
     if (threadIdx.x == 0) part[blockIdx.x] = s[0];
-}
-
-__device__ inline double plane_sum(const double *part, int j) {
-    double a = 0.0;
-    for (int c = 0; c < PLANE_CHUNKS; ++c) a += part[j * PLANE_CHUNKS + c];
-    return a;
 }
 
 // the kx = kz = 0 line of tridiag_kernel in FP64 on the plane sums; mean[j-1] = x_j / (nx nz).
@@ -1579,12 +1727,13 @@ __global__ __launch_bounds__(FFT_THREADS) void ixfft32_add_kernel(Dims d, const 
 // the FP64 right-hand side -> h->fft_rhs, phi = 0
 hipError_t launch_fft_mixed_setup(mdx_handle *h, double dtg) {
     GridK g = grid_k(h);
+    const FftStep fs = fft_step(h);
     const Dims d = h->d;
     dim3 blk(64, FC_Y), grd((d.nx + 63) / 64, (d.ny + FC_Y - 1) / FC_Y, (d.nz + FC_KZ - 1) / FC_KZ);
     if (h->stretched)
-        hipLaunchKernelGGL(fft_div_rhs_kernel<true>, grd, blk, 0, h->stream, g, h->us, h->vs, h->ws, dtg, h->fft_rhs);
+        hipLaunchKernelGGL(fft_div_rhs_kernel<true>, grd, blk, 0, h->stream, g, h->us, h->vs, h->ws, dtg, fft_wrap(h), fs, h->fft_rhs);
     else
-        hipLaunchKernelGGL(fft_div_rhs_kernel<false>, grd, blk, 0, h->stream, g, h->us, h->vs, h->ws, dtg, h->fft_rhs);
+        hipLaunchKernelGGL(fft_div_rhs_kernel<false>, grd, blk, 0, h->stream, g, h->us, h->vs, h->ws, dtg, fft_wrap(h), fs, h->fft_rhs);
     hipError_t e = hipGetLastError();
     return e != hipSuccess ? e : launch_zero64(h, h->fft_phi, h->ni);
 }
@@ -1681,17 +1830,6 @@ hipError_t launch_fft_pin(mdx_handle *h) {
 }
 
 // the projection with a given FP64 phi in (nx, nz, ny) layout (step 6)
-hipError_t launch_fft_correct(mdx_handle *h, const double *phi, double dtg) {
-    GridK g = grid_k(h);
-    const Dims d = h->d;
-    dim3 blk(64, 4), grd((d.nx + 63) / 64, (d.ny + 3) / 4, d.nz);
-#define MDX_CORR(S, I)                                                                                     \
-    hipLaunchKernelGGL((fft_correct_kernel<S, I>), grd, blk, 0, h->stream, g, phi, h->us, h->vs, h->ws, h->cu, \
-                       h->cv, h->cw, dtg, h->un, h->vn, h->wn, h->pn)
-    if (h->stretched) { if (h->ibm_on) MDX_CORR(true, true); else MDX_CORR(true, false); }
-    else { if (h->ibm_on) MDX_CORR(false, true); else MDX_CORR(false, false); }
-#undef MDX_CORR
-    return hipGetLastError();
-}
+hipError_t launch_fft_correct(mdx_handle *h, const double *phi, double dtg) { return launch_correct(h, phi, dtg, nullptr); }
 
 }  // namespace mdx

@@ -94,6 +94,38 @@ __device__ inline bool xcd_tile(int items_x, int items_y, int nz, int bxx, int b
     return true;
 }
 
+// The flow-rate correction from the n partial sums (pairs u*, mu_u) in part, by a workgroup of 256
+// (t: its thread; s1, s2: 256 values of LDS each): o = bulk velocity, mean mu_u, du = (target - ub)
+// / mean mu_u, the same in every thread.  The lanes' sums fold in halves, 128 down to 1, the last six
+// within the first wavefront.
+__device__ inline void flow_fold(const double *part, int n, double norm, double target, int t, double *s1, double *s2,
+                                 double (&o)[3]) {
+    double a = 0.0, b = 0.0;
+    for (int q = t; q < n; q += 256) {
+        a += part[2 * q];
+        b += part[2 * q + 1];
+    }
+    s1[t] = a;
+    s2[t] = b;
+    __syncthreads();
+    if (t < 64) {
+        a = (s1[t] + s1[t + 128]) + (s1[t + 64] + s1[t + 192]);
+        b = (s2[t] + s2[t + 128]) + (s2[t + 64] + s2[t + 192]);
+        for (int w = 32; w > 0; w >>= 1) {
+            a += __shfl_down(a, w, 64);
+            b += __shfl_down(b, w, 64);
+        }
+        if (t == 0) {
+            s1[0] = a;
+            s2[0] = b;
+        }
+    }
+    __syncthreads();
+    o[0] = s1[0] / norm;
+    o[1] = s2[0] / norm;
+    o[2] = (target - o[0]) / o[1];
+}
+
 // per-workgroup maximum of non-negative doubles into part[workgroup]; NaN propagates
 __device__ inline double nanmax_any(double a, double b) { return (a != a || a > b) ? a : b; }
 __device__ inline void block_max_part(double v, double *part) {
@@ -218,6 +250,11 @@ struct mdx_handle {
     // coefficient tables (MOBYDIFF_FUSED_MU=0: build_mu_kernel before the solve)
     bool fused_mu = true;
     bool apply_wrote_bc = false;
+    // FFT projection inside a step: it takes u*'s ghosts as filled (MOBYDIFF_FUSED_BC=0: reads them),
+    // adds the flow-rate shift of the step_parts partial sums in fr_part (0: none) and, in the
+    // step's last stage, stores the shifted u*
+    int step_parts = 0;
+    bool step_last = false;
     // streaming red-black sweeps: z planes marched per thread (0: one cell per thread)
     int sweep_kz = 4;
     // one launch per red+black iteration (halo-recomputing tiles) instead of one per colour

@@ -24,7 +24,7 @@ struct mdx_net {
     bf16 *wp[11] = {}, *wd[11] = {};   // forward / input-gradient weights in MFMA fragment order
     bf16 *x_in = nullptr, *a[10] = {}, *p1 = nullptr, *p2 = nullptr, *cat1 = nullptr, *cat2 = nullptr;
     bf16 *g[10] = {}, *gp1 = nullptr, *gp2 = nullptr, *gcat1 = nullptr, *gcat2 = nullptr;
-    float *out = nullptr, *dout = nullptr, *target = nullptr, *loss = nullptr, *x2_stage = nullptr;
+    float *out = nullptr, *target = nullptr, *loss = nullptr, *x2_stage = nullptr;
     double *stats = nullptr, *part = nullptr, *h_pinned = nullptr;
     double *vsum = nullptr;        // per voxel: the sums of r0 and of Phi_0 over its cells (fused input pass)
     std::vector<void *> allocs;

@@ -25,6 +25,7 @@
 #include "mdx_unet.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 namespace mdx {
@@ -329,100 +330,167 @@ __global__ __launch_bounds__(256) void conv3_tiled_kernel(const bf16 *__restrict
 }
 
 // ------------------------------------------------------------------------------- weight gradient
-// One workgroup = one tap x one slice of voxels.  Each 32-voxel chunk: dY (32 x COUT) and the
-// tap-shifted input (32 x CIN) are staged transposed in LDS ([c][v], so 8 consecutive voxels of one
-// channel are one 16-byte read); each wave owns a subset of the (CIN/16 x COUT/16) output tiles.
+// One workgroup = one tap x one slice of voxels.  Each 128-voxel chunk: dY (128 x COUT) and the
+// tap-shifted input (128 x CIN) are staged transposed in LDS ([c][v], so 8 consecutive voxels of one
+// channel are one 16-byte read; rows 272 bytes apart, which spreads 16 of them over the banks); a
+// thread packs two voxels per LDS word, and the next chunk's loads are in flight while a chunk is
+// multiplied.  Four or more (CIN/16 x COUT/16) output tiles are shared out to the waves, each over the
+// whole chunk; with fewer, each wave takes a quarter of the chunk for all of them and the partial
+// tiles meet in LDS at the end.  The centre tap's workgroups also form the bias gradient, db[n] =
+// sum_v dY[v][n], as one more tile row with an input of ones (exact products).
+// Bound by latency (a chunk's loads, two barriers): with 32-voxel chunks, nothing in flight and one
+// wave of four multiplying, 16 -> 16 channels at 48 x 32 x 24 took 22.8 us, 11.5 now; the bias sums in
+// kernels of their own took 119 us there (16 channels: every wave's atomic additions went to one
+// cache line, 17 ns each).
 template <int CIN, int COUT>
 __global__ __launch_bounds__(256) void conv3_wgrad_kernel(const bf16 *__restrict__ in, const bf16 *__restrict__ dy,
-                                                          float *__restrict__ dw, int W, int H, int D, int slices) {
-    constexpr int MT = CIN / 16, NT = COUT / 16, TILES = MT * NT;
-    constexpr int TPW = (TILES + 3) / 4;   // tiles per wave
-    __shared__ __attribute__((aligned(16))) bf16 sx[CIN * 32];
-    __shared__ __attribute__((aligned(16))) bf16 sd[COUT * 32];
+                                                          float *__restrict__ dw, float *__restrict__ db, int W, int H,
+                                                          int D, int slices) {
+    constexpr int MT = CIN / 16, NT = COUT / 16, TILES = MT * NT, CV = 128, LS = CV + 8;
+    constexpr bool KSPLIT = TILES < 4;
+    constexpr int TPW = KSPLIT ? TILES : TILES / 4;   // tiles per wave
+    static_assert(KSPLIT || TILES % 4 == 0, "whole tiles per wave");
+    constexpr int QX = CV / 2 * (CIN / 8), QD = CV / 2 * (COUT / 8);   // pairs of voxels x 8 channels
+    constexpr int NX = (QX + 255) / 256, ND = (QD + 255) / 256;
+    __shared__ __attribute__((aligned(16))) bf16 sx[CIN * LS];
+    __shared__ __attribute__((aligned(16))) bf16 sd[COUT * LS];
     const int tap = blockIdx.x % 27, slice = blockIdx.x / 27;
     const int dxo = tap % 3 - 1, dyo = (tap / 3) % 3 - 1, dzo = tap / 9 - 1;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long V = (long)W * H * D;
-    const long nchunks = V / 32;
-    const long c_begin = nchunks * slice / slices, c_end = nchunks * (slice + 1) / slices;
-    f32x4 acc[TPW];
+    const int V = W * H * D, nchunks = (V + CV - 1) / CV;
+    const int c_begin = (int)((long)nchunks * slice / slices), c_end = (int)((long)nchunks * (slice + 1) / slices);
+    f32x4 acc[TPW], accb[KSPLIT ? NT : 1];
 #pragma unroll
     for (int q = 0; q < TPW; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (long ch = c_begin; ch < c_end; ++ch) {
-        const long vb = ch * 32;
-        __syncthreads();
-        // stage: thread t covers (voxel t/8... ) -- CIN/8 and COUT/8 vector loads per voxel
-        for (int q = threadIdx.x; q < 32 * (CIN / 8); q += 256) {
-            const int vv = q / (CIN / 8), c0 = (q % (CIN / 8)) * 8;
-            const long v = vb + vv;
-            const int x = (int)(v % W), y = (int)((v / W) % H), z = (int)(v / ((long)W * H));
-            const int xx = x + dxo, yy = y + dyo, zz = z + dzo;
-            bf16x8 a = {};
-            if (xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D)
-                a = *reinterpret_cast<const bf16x8 *>(in + (((long)zz * H + yy) * W + xx) * CIN + c0);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) sx[(c0 + e) * 32 + vv] = a[e];
-        }
-        for (int q = threadIdx.x; q < 32 * (COUT / 8); q += 256) {
-            const int vv = q / (COUT / 8), c0 = (q % (COUT / 8)) * 8;
-            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(dy + (vb + vv) * COUT + c0);
+    for (int q = 0; q < (KSPLIT ? NT : 1); ++q) accb[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 rx[NX][2], rd[ND][2];
+    auto load = [&](int ch) {   // V is even: a pair is whole
 #pragma unroll
-            for (int e = 0; e < 8; ++e) sd[(c0 + e) * 32 + vv] = a[e];
+        for (int c = 0; c < NX; ++c) {
+            const int q = threadIdx.x + 256 * c;
+            rx[c][0] = rx[c][1] = bf16x8{};
+            if (QX % 256 && q >= QX) continue;
+            const int v = ch * CV + 2 * (q / (CIN / 8)), c0 = (q % (CIN / 8)) * 8;
+            if (v >= V) continue;
+            int x = v % W, y = v / W % H, z = v / W / H;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int xx = x + dxo, yy = y + dyo, zz = z + dzo;
+                if (xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D)
+                    rx[c][e] = *reinterpret_cast<const bf16x8 *>(in + (((long)zz * H + yy) * W + xx) * CIN + c0);
+                if (++x == W) {
+                    x = 0;
+                    if (++y == H) {
+                        y = 0;
+                        ++z;
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < ND; ++c) {
+            const int q = threadIdx.x + 256 * c;
+            rd[c][0] = rd[c][1] = bf16x8{};
+            if (QD % 256 && q >= QD) continue;
+            const int v = ch * CV + 2 * (q / (COUT / 8)), c0 = (q % (COUT / 8)) * 8;
+            if (v >= V) continue;
+            const bf16 *p = dy + (long)v * COUT + c0;
+            rd[c][0] = *reinterpret_cast<const bf16x8 *>(p);
+            rd[c][1] = *reinterpret_cast<const bf16x8 *>(p + COUT);
+        }
+    };
+    const int r = lane & 15, g = lane >> 4;
+    bf16x8 ones;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ones[e] = (bf16)1.f;
+    load(c_begin);
+    for (int ch = c_begin; ch < c_end; ++ch) {
+        if (ch > c_begin) __syncthreads();   // the last chunk's operands have been read
+#pragma unroll
+        for (int c = 0; c < NX; ++c) {
+            const int q = threadIdx.x + 256 * c;
+            if (QX % 256 && q >= QX) continue;
+            const int vv = 2 * (q / (CIN / 8)), c0 = (q % (CIN / 8)) * 8;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                *reinterpret_cast<bf16x2 *>(&sx[(c0 + e) * LS + vv]) = bf16x2{rx[c][0][e], rx[c][1][e]};
+        }
+#pragma unroll
+        for (int c = 0; c < ND; ++c) {
+            const int q = threadIdx.x + 256 * c;
+            if (QD % 256 && q >= QD) continue;
+            const int vv = 2 * (q / (COUT / 8)), c0 = (q % (COUT / 8)) * 8;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                *reinterpret_cast<bf16x2 *>(&sd[(c0 + e) * LS + vv]) = bf16x2{rd[c][0][e], rd[c][1][e]};
         }
         __syncthreads();
+        if (ch + 1 < c_end) load(ch + 1);
         // D[m = cin][n = cout] += sum_{v in chunk} X[v][m] dY[v][n]:  A[m][k=v], B[k=v][n]
-        const int r = lane & 15, g = lane >> 4;
+        auto xop = [&](int mt, int ks) { return *reinterpret_cast<const bf16x8 *>(&sx[(mt * 16 + r) * LS + 32 * ks + 8 * g]); };
+        auto dop = [&](int nt, int ks) { return *reinterpret_cast<const bf16x8 *>(&sd[(nt * 16 + r) * LS + 32 * ks + 8 * g]); };
+        if (KSPLIT) {
 #pragma unroll
-        for (int q = 0; q < TPW; ++q) {
-            const int tile = wave * TPW + q;
-            if (tile < TILES) {
-                const int mt = tile / NT, nt = tile % NT;
-                const bf16x8 a = *reinterpret_cast<const bf16x8 *>(&sx[(mt * 16 + r) * 32 + 8 * g]);
-                const bf16x8 bb = *reinterpret_cast<const bf16x8 *>(&sd[(nt * 16 + r) * 32 + 8 * g]);
-                acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bb, acc[q], 0, 0, 0);
+            for (int q = 0; q < TPW; ++q)
+                acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xop(q / NT, wave), dop(q % NT, wave), acc[q], 0, 0, 0);
+            if (tap == 13) {
+#pragma unroll
+                for (int q = 0; q < NT; ++q)
+                    accb[KSPLIT ? q : 0] =
+                        __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, dop(q, wave), accb[KSPLIT ? q : 0], 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int ks = 0; ks < CV / 32; ++ks) {
+#pragma unroll
+                for (int q = 0; q < TPW; ++q) {
+                    const int tile = wave * TPW + q;
+                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xop(tile / NT, ks), dop(tile % NT, ks), acc[q], 0, 0, 0);
+                }
+                if (tap == 13 && wave < NT)
+                    accb[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, dop(wave, ks), accb[0], 0, 0, 0);
             }
         }
     }
     // accumulate: lane holds D[4g+i][lane%16] -> dw[(tap*CIN + m)*COUT + n]
-    const int g = lane >> 4;
+    if (KSPLIT) {
+        constexpr int PF = KSPLIT ? TILES * 256 : 1;
+        __shared__ float part[3][PF];   // waves 1 .. 3; wave 0 adds its own
+        if (wave > 0) {
 #pragma unroll
-    for (int q = 0; q < TPW; ++q) {
-        const int tile = wave * TPW + q;
-        if (tile < TILES) {
-            const int mt = tile / NT, nt = tile % NT;
+            for (int q = 0; q < TPW; ++q)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) part[wave - 1][KSPLIT ? (q * 4 + i) * 64 + lane : 0] = acc[q][i];
+        }
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int q = 0; q < TPW; ++q)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int o = KSPLIT ? (q * 4 + i) * 64 + lane : 0, m = q / NT * 16 + 4 * g + i, n = q % NT * 16 + r;
+                    atomicAdd(&dw[((long)tap * CIN + m) * COUT + n], acc[q][i] + part[0][o] + part[1][o] + part[2][o]);
+                }
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < TPW; ++q) {
+            const int tile = wave * TPW + q, mt = tile / NT, nt = tile % NT;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int m = mt * 16 + 4 * g + i, n = nt * 16 + (lane & 15);
+                const int m = mt * 16 + 4 * g + i, n = nt * 16 + r;
                 atomicAdd(&dw[((long)tap * CIN + m) * COUT + n], acc[q][i]);
             }
         }
     }
-}
-
-// bias gradient: db[n] = sum_v dY[v][n].  The COUT channels of a voxel are G = COUT/8 16-byte
-// vectors; thread t reads vectors q = t, t + stride, ... of the flat array (consecutive lanes,
-// consecutive 16 bytes: whole cache lines per wave), and since the stride is a multiple of G a thread
-// always sees the same channel group q % G.  The lanes of one group are then folded by shuffles
-// (offsets G .. 32) and one atomic addition per channel and wave is left.
-template <int COUT>
-__global__ __launch_bounds__(256) void bias_grad_kernel(const bf16 *__restrict__ dy, float *__restrict__ db, long V) {
-    constexpr int G = COUT / 8;
-    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    const long nvec = V * G;
-    const bf16x8 *__restrict__ d8 = reinterpret_cast<const bf16x8 *>(dy);
-    for (long q = (long)blockIdx.x * 256 + threadIdx.x; q < nvec; q += (long)gridDim.x * 256) {
-        const bf16x8 a = d8[q];
+    if (tap == 13 && g == 0) {   // every row of a bias tile holds the sums
+        if (KSPLIT) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) s[e] += (float)a[e];
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-        for (int off = 32; off >= G; off >>= 1) s[e] += __shfl_xor(s[e], off, 64);
-    const int lane = threadIdx.x & 63;
-    if (lane < G) {
-        const int g = (int)(((long)blockIdx.x * 256 + threadIdx.x) % G);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) atomicAdd(&db[g * 8 + e], s[e]);
+            for (int q = 0; q < NT; ++q) atomicAdd(&db[q * 16 + r], accb[KSPLIT ? q : 0][0]);
+        } else if (wave < NT) {
+            atomicAdd(&db[wave * 16 + r], accb[0][0]);
+        }
     }
 }
 
@@ -491,17 +559,19 @@ __global__ void upcat_bwd_coarse_kernel(const bf16 *__restrict__ dcat, bf16 *__r
     }
 }
 
-// d_out (gradient arriving at a ReLU layer's output) = (d_from_next + d_skip) * (y > 0)
+// d_out (gradient arriving at a ReLU layer's output) = (d_from_next + d_skip) * (y > 0); a thread
+// per voxel and 8 channels
 __global__ void relu_bwd_kernel(bf16 *__restrict__ g, const bf16 *__restrict__ extra, int Ce, int coff, int C,
-                                const bf16 *__restrict__ y, long n) {
-    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
-        float d = (float)g[q];
-        if (extra) {
-            const long v = q / C;
-            const int c = (int)(q % C);
-            d += (float)extra[v * Ce + coff + c];
-        }
-        g[q] = (bf16)((float)y[q] > 0.f ? d : 0.f);
+                                const bf16 *__restrict__ y, long n8) {
+    const int G = C / 8;
+    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n8; q += (long)gridDim.x * blockDim.x) {
+        bf16x8 d = reinterpret_cast<const bf16x8 *>(g)[q];
+        const bf16x8 yy = reinterpret_cast<const bf16x8 *>(y)[q];
+        bf16x8 ex = {};
+        if (extra) ex = *reinterpret_cast<const bf16x8 *>(extra + q / G * Ce + coff + q % G * 8);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) d[e] = (bf16)((float)yy[e] > 0.f ? (float)d[e] + (float)ex[e] : 0.f);
+        reinterpret_cast<bf16x8 *>(g)[q] = d;
     }
 }
 
@@ -527,66 +597,96 @@ __global__ void head_fwd_kernel(const bf16 *__restrict__ x, const float *__restr
     }
 }
 
-// MSE loss against the target: dout = 2 (out - t) / (V * batch); loss partial sums
-__global__ void mse_kernel(const float *__restrict__ out, const float *__restrict__ t, float *__restrict__ dout,
-                           float scale, long V, float *__restrict__ loss) {
+// MSE loss against the target
+__global__ __launch_bounds__(256) void mse_kernel(const float *__restrict__ out, const float *__restrict__ t, float scale,
+                                                  long V, float *__restrict__ loss) {
+    __shared__ float part[4];
     float s = 0.f;
     for (long v = (long)blockIdx.x * blockDim.x + threadIdx.x; v < V; v += (long)gridDim.x * blockDim.x) {
         const float e = out[v] - t[v];
-        dout[v] = 2.f * e * scale;
         s += e * e;
     }
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(loss, s * scale);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(loss, ((part[0] + part[1]) + (part[2] + part[3])) * scale);
 }
 
-// head backward: dx[v][c] = dout[v] w[c]; dw[c] += sum_v dout[v] x[v][c]; db += sum dout
+// MSE loss against the target and the head's backward: d = 2 (out - t) / (V * batch); dx[v][c] =
+// d w[c], through the ReLU of x; dw[c] += sum_v d x[v][c]; db += sum d; loss += sum (out - t)^2 / (V
+// batch).  The 18 sums fold within the workgroup and leave it in one atomic instruction: all
+// workgroups' go to the same two cache lines, 17 ns each, and one per wave and sum took 119 us at
+// 48 x 32 x 24 (8.3 now, with the loss and the ReLU in the same pass).
 __global__ __launch_bounds__(256) void head_bwd_kernel(const bf16 *__restrict__ x, const float *__restrict__ w,
-                                                       const float *__restrict__ dout, bf16 *__restrict__ dx,
-                                                       float *__restrict__ dw, float *__restrict__ db, long V) {
-    float sw[16], sb = 0.f;
+                                                       const float *__restrict__ out, const float *__restrict__ target,
+                                                       float scale, bf16 *__restrict__ dx, float *__restrict__ dw,
+                                                       float *__restrict__ db, float *__restrict__ loss, long V) {
+    __shared__ float part[4][18];
+    float sw[18];   // dw, db, loss
 #pragma unroll
-    for (int c = 0; c < 16; ++c) sw[c] = 0.f;
+    for (int c = 0; c < 18; ++c) sw[c] = 0.f;
     for (long v = (long)blockIdx.x * blockDim.x + threadIdx.x; v < V; v += (long)gridDim.x * blockDim.x) {
-        const float d = dout[v];
-        sb += d;
+        const float e = out[v] - target[v], d = 2.f * e * scale;
+        sw[16] += d;
+        sw[17] += e * e;
 #pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            sw[c] += d * (float)x[v * 16 + c];
-            dx[v * 16 + c] = (bf16)(d * w[c]);
+        for (int h = 0; h < 2; ++h) {
+            const bf16x8 a = reinterpret_cast<const bf16x8 *>(x)[2 * v + h];
+            bf16x8 o;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                sw[8 * h + c] += d * (float)a[c];
+                o[c] = (float)a[c] > 0.f ? (bf16)(d * w[8 * h + c]) : (bf16)0.f;
+            }
+            reinterpret_cast<bf16x8 *>(dx)[2 * v + h] = o;
         }
     }
 #pragma unroll
-    for (int c = 0; c < 16; ++c) {
+    for (int c = 0; c < 18; ++c) {
         float t = sw[c];
         for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
-        if ((threadIdx.x & 63) == 0) atomicAdd(&dw[c], t);
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6][c] = t;
     }
-    for (int off = 32; off > 0; off >>= 1) sb += __shfl_xor(sb, off, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(db, sb);
+    __syncthreads();
+    if (threadIdx.x < 18) {
+        const int c = threadIdx.x;
+        const float t = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+        atomicAdd(c < 16 ? dw + c : c == 16 ? db : loss, c < 17 ? t : t * scale);
+    }
 }
 
 // ------------------------------------------------------------------------------- weights
 // fragment repack: wp[(kc*NT+nt)*64 + lane][e] = W[k][n], k = 32 kc + 8 (lane/16) + e, n = 16 nt + lane%16;
-// flip != 0 builds the input-gradient weights W'[tap'][cout][cin] = W[26-tap'][cin][cout]
-__global__ void repack_kernel(const float *__restrict__ w, bf16 *__restrict__ wp, int cin, int cout, int flip) {
-    const int ci = flip ? cout : cin, co = flip ? cin : cout;   // GEMM input / output channels
-    const int K = 27 * ci, KC = (K + 31) / 32, NT = co / 16;
-    const long n = (long)KC * NT * 64 * 8;
-    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
-        const int e = (int)(q % 8);
-        const int lane = (int)((q / 8) % 64);
-        const long blk = q / 512;
-        const int nt = (int)(blk % NT), kc = (int)(blk / NT);
-        const int k = 32 * kc + 8 * (lane / 16) + e, nn = 16 * nt + lane % 16;
-        float val = 0.f;
-        if (k < K) {
-            const int tap = k / ci, c = k % ci;
-            if (!flip) val = w[((long)tap * cin + c) * cout + nn];
-            else val = w[((long)(26 - tap) * cin + nn) * cout + c];
-        }
-        wp[q] = (bf16)val;
+// flip != 0 builds the input-gradient weights W'[tap'][cout][cin] = W[26-tap'][cin][cout].  All layers
+// and both directions in one launch (20 of them took 52 us): jobs[j] starts at block jobs[j].block.
+struct RepackJob {
+    const float *w;
+    bf16 *wp;
+    int cin, cout, flip, block;
+};
+struct RepackJobs {
+    RepackJob job[2 * NL];
+    int n;
+};
+__global__ __launch_bounds__(256) void repack_kernel(RepackJobs jobs) {
+    int jj = 0;
+    while (jj + 1 < jobs.n && (int)blockIdx.x >= jobs.job[jj + 1].block) ++jj;
+    const RepackJob &J = jobs.job[jj];
+    const int cin = J.cin, cout = J.cout;
+    const int ci = J.flip ? cout : cin, co = J.flip ? cin : cout;   // GEMM input / output channels
+    const int K = 27 * ci, NT = co / 16;
+    // a job's count is a multiple of 512: no workgroup straddles two
+    const int q = ((int)blockIdx.x - J.block) * 256 + threadIdx.x;
+    const int e = q % 8, lane = (q / 8) % 64, blk = q / 512;
+    const int nt = blk % NT, kc = blk / NT;
+    const int k = 32 * kc + 8 * (lane / 16) + e, nn = 16 * nt + lane % 16;
+    float val = 0.f;
+    if (k < K) {
+        const int tap = k / ci, c = k % ci;
+        if (!J.flip) val = J.w[((long)tap * cin + c) * cout + nn];
+        else val = J.w[((long)(26 - tap) * cin + nn) * cout + c];
     }
+    J.wp[q] = (bf16)val;
 }
 
 // Adam (Kingma & Ba 2015, Alg. 1) on FP32 master weights; grads are averaged over the batch
@@ -1022,40 +1122,42 @@ static hipError_t wgrad(mdx_net *n, int l, const bf16 *in, const bf16 *dy) {
     const LayerDesc &L = LAYERS[l];
     const int lvl = L.level;
     const int W = n->W[lvl], H = n->H[lvl], D = n->D[lvl];
-    const long chunks = n->V[lvl] / 32;
-    int slices = (int)std::min<long>(48, std::max<long>(1, chunks / 16));
+    const int chunks = (int)((n->V[lvl] + 127) / 128);
+    // two chunks a slice, so one is in flight while the other is multiplied; at most 36, as every slice
+    // adds its whole tile to dw (48 -> 16 channels at 48 x 32 x 24: 25 us with 48 slices, 22 with 36, 28
+    // with 18; one or three chunks a slice at 24 x 16 x 12: 17 and 15 us against 15 for 96 -> 32)
+    const int slices = std::min(36, std::max(1, chunks / 2));
 #define WG_CASE(CI, CO)                                                                                       \
     if (L.cin == CI && L.cout == CO) {                                                                       \
         hipLaunchKernelGGL((conv3_wgrad_kernel<CI, CO>), dim3(27 * slices), dim3(256), 0, n->stream, in, dy,    \
-                           dWt(n, l), W, H, D, slices);                                                      \
+                           dWt(n, l), dBs(n, l), W, H, D, slices);                                           \
     } else
     WG_CASE(16, 16) WG_CASE(16, 32) WG_CASE(32, 32) WG_CASE(32, 64) WG_CASE(64, 64) WG_CASE(96, 32) WG_CASE(48, 16)
     return hipErrorInvalidValue;
 #undef WG_CASE
-    const long V = n->V[lvl];
-    if (L.cout == 16) hipLaunchKernelGGL(bias_grad_kernel<16>, dim3(nred(V * 2)), dim3(256), 0, n->stream, dy, dBs(n, l), V);
-    else if (L.cout == 32) hipLaunchKernelGGL(bias_grad_kernel<32>, dim3(nred(V * 4)), dim3(256), 0, n->stream, dy, dBs(n, l), V);
-    else hipLaunchKernelGGL(bias_grad_kernel<64>, dim3(nred(V * 8)), dim3(256), 0, n->stream, dy, dBs(n, l), V);
     return hipGetLastError();
 }
 
 static hipError_t relu_bwd(mdx_net *n, bf16 *g, const bf16 *extra, int Ce, int coff, int C, const bf16 *y, int lvl) {
-    const long cnt = n->V[lvl] * C;
+    const long cnt = n->V[lvl] * C / 8;
     hipLaunchKernelGGL(relu_bwd_kernel, dim3(nblk(cnt)), dim3(256), 0, n->stream, g, extra, Ce, coff, C, y, cnt);
     return hipGetLastError();
 }
 
 hipError_t repack_all(mdx_net *n) {
+    RepackJobs jobs;
+    jobs.n = 0;
+    int blocks = 0;
     for (int l = 0; l < NL; ++l) {
         const LayerDesc &L = LAYERS[l];
         if (L.ks != 3) continue;
-        const long cf = (long)((27 * L.cin + 31) / 32) * (L.cout / 16) * 512;
-        hipLaunchKernelGGL(repack_kernel, dim3(nblk(cf)), dim3(256), 0, n->stream, Wt(n, l), n->wp[l], L.cin, L.cout, 0);
-        if (n->wd[l]) {
-            const long cd = (long)((27 * L.cout + 31) / 32) * (L.cin / 16) * 512;
-            hipLaunchKernelGGL(repack_kernel, dim3(nblk(cd)), dim3(256), 0, n->stream, Wt(n, l), n->wd[l], L.cin, L.cout, 1);
-        }
+        jobs.job[jobs.n++] = RepackJob{Wt(n, l), n->wp[l], L.cin, L.cout, 0, blocks};
+        blocks += (27 * L.cin + 31) / 32 * (L.cout / 16) * 2;
+        if (!n->wd[l]) continue;
+        jobs.job[jobs.n++] = RepackJob{Wt(n, l), n->wd[l], L.cin, L.cout, 1, blocks};
+        blocks += (27 * L.cout + 31) / 32 * (L.cin / 16) * 2;
     }
+    hipLaunchKernelGGL(repack_kernel, dim3(blocks), dim3(256), 0, n->stream, jobs);
     return hipGetLastError();
 }
 
@@ -1117,12 +1219,9 @@ hipError_t net_backward(mdx_net *n, float scale) {
     const long V0 = n->V[0];
     const int W0 = n->W[0], H0 = n->H[0], D0 = n->D[0], W1 = n->W[1], H1 = n->H[1], D1 = n->D[1];
     TRY(hipMemsetAsync(n->loss, 0, 4, n->stream));
-    hipLaunchKernelGGL(mse_kernel, dim3(nred(V0)), dim3(256), 0, n->stream, n->out, n->target, n->dout,
-                       scale / (float)V0, V0, n->loss);
-    hipLaunchKernelGGL(head_bwd_kernel, dim3(nred(V0)), dim3(256), 0, n->stream, n->a[9], Wt(n, 10), n->dout, n->g[9],
-                       dWt(n, 10), dBs(n, 10), V0);
+    hipLaunchKernelGGL(head_bwd_kernel, dim3(nred(V0)), dim3(256), 0, n->stream, n->a[9], Wt(n, 10), n->out, n->target,
+                       scale / (float)V0, n->g[9], dWt(n, 10), dBs(n, 10), n->loss, V0);
     // decoder level 0
-    TRY(relu_bwd(n, n->g[9], nullptr, 0, 0, 16, n->a[9], 0));
     TRY(wgrad(n, 9, n->a[8], n->g[9]));
     TRY(conv3(n, 16, 16, false, n->g[9], n->wd[9], nullptr, n->g[8], 0));
     TRY(relu_bwd(n, n->g[8], nullptr, 0, 0, 16, n->a[8], 0));
@@ -1274,7 +1373,7 @@ hipError_t net_capture(mdx_net *n, const double *phi, const double *phi_prev, do
 hipError_t net_mse_only(mdx_net *n) {
     hipError_t e = hipMemsetAsync(n->loss, 0, 4, n->stream);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(mse_kernel, dim3(nred(n->V[0])), dim3(256), 0, n->stream, n->out, n->target, n->dout,
+    hipLaunchKernelGGL(mse_kernel, dim3(nred(n->V[0])), dim3(256), 0, n->stream, n->out, n->target,
                        1.0f / (float)n->V[0], n->V[0], n->loss);
     return hipGetLastError();
 }

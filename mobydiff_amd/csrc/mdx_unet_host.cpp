@@ -110,7 +110,7 @@ extern "C" int mdx_net_create_strided(int32_t nx, int32_t ny, int32_t nz, int32_
     };
     for (auto &b : bufs)
         if ((e = nalloc(n, b.p, b.n)) != hipSuccess) return fail(e);
-    if ((e = nalloc(n, &n->out, V0)) != hipSuccess || (e = nalloc(n, &n->dout, V0)) != hipSuccess ||
+    if ((e = nalloc(n, &n->out, V0)) != hipSuccess ||
         (e = nalloc(n, &n->x2_stage, 2 * V0)) != hipSuccess ||
         (e = nalloc(n, &n->target, V0)) != hipSuccess || (e = nalloc(n, &n->loss, 4)) != hipSuccess ||
         (e = nalloc(n, &n->stats, 8)) != hipSuccess || (e = nalloc(n, &n->part, 3 * 512)) != hipSuccess ||

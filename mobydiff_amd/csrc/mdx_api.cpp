@@ -1803,9 +1803,11 @@ extern "C" int mdx_step(mdx_handle *h, double dt, mdx_step_stats *stats) {
             // momentum forms the flow-rate partial sums of u*; one launch folds them, shifts u* and
             // builds the stage's face-coefficient tables if the solve needs new ones (with the FFT
             // and no body the shift is uniform, and the projection's last pass makes it)
-            MDX_HIP(launch_momentum(h, dta, dtb, dtg, h->fr_part));
+            const bool late = h->cfg.solver == MDX_SOLVER_FFT && !h->ibm_on;
+            h->step_sum = late && fft_sums(h);
+            MDX_HIP(launch_momentum(h, dta, dtb, dtg, h->step_sum ? nullptr : h->fr_part));
             ev_record(h, 5);
-            if (h->cfg.solver == MDX_SOLVER_FFT && !h->ibm_on) {
+            if (late) {
                 h->step_parts = momentum_tiles(h);
             } else {
                 // (the tables exist for the SOR solver only)
@@ -1834,6 +1836,7 @@ extern "C" int mdx_step(mdx_handle *h, double dt, mdx_step_stats *stats) {
         rc = mdx_pressure_projection(h, dtg, &st);
         h->step_bc = false;
         h->step_parts = 0;
+        h->step_sum = false;
         if (rc) {
             if (stats) stats->stage[s] = st;
             return rc;

@@ -311,14 +311,44 @@ __device__ inline double div_by(double a, double d, double r) {
 // 1. rhs(i,k,j) = div u* / dtg and the forward x-transform, two rows (planes k, k + 1) per line.
 //    wrap: u*'s ghosts are taken as apply_bc fills them (periodic in x and z, v* = 0 on the walls)
 //    instead of read; inside a step nothing else reads them, so their fill is left to its end.
+//    The workgroups past `lines` form the flow-rate partial sums of u* instead, tile by tile as the
+//    momentum kernel would (64 x 4 columns, mkz planes): on the grids where it is faster without.
+struct FlowSum {
+    int lines, mkz;
+    double *part;
+};
+__device__ inline void flow_sum_tile(const GridK &g, const double *__restrict__ us, const FlowSum &f, double *s) {
+    const Dims d = g.d;
+    const int ntx = (d.nx + 63) / 64, nty = (d.ny + 3) / 4;
+    const int wg = (int)blockIdx.x - f.lines, tx = wg % ntx, ty = wg / ntx % nty, tz = wg / ntx / nty;
+    const int i = tx * 64 + threadIdx.x % 64 + 1, j = ty * 4 + threadIdx.x / 64 + 1, k0 = tz * f.mkz + 1;
+    const int nk = k0 + f.mkz - 1 < d.nz ? f.mkz : d.nz - k0 + 1;
+    double fa = 0.0, fb = 0.0;
+    if (i <= d.nx && j <= d.ny) {
+        const double hj = g.ihc ? 1.0 / g.ihc[j] : g.dy;
+        const double *u = us + d.g(i, j, k0);
+        const size_t sz = (size_t)d.sx * d.sy;
+#pragma unroll 4
+        for (int k = 0; k < nk; ++k) {
+            fa += u[k * sz] * hj;
+            fb += hj;
+        }
+    }
+    flow_tile_sum<4>(fa, fb, threadIdx.x, s, f.part, (size_t)wg);
+}
 template <int N, int TH, int W, bool STRETCH>
 __global__ __launch_bounds__(TH * W) void rhs_xfft_reg_kernel(GridK g, const double *__restrict__ us,
                                                               const double *__restrict__ vs,
                                                               const double *__restrict__ ws, double dtg, int wrap,
-                                                              const double2 *__restrict__ tw, int stride,
+                                                              FlowSum fsum, const double2 *__restrict__ tw, int stride,
                                                               double2 *__restrict__ hat) {
     using F = RFft<N, TH>;
     extern __shared__ __align__(16) unsigned char lds_raw[];
+    if ((int)blockIdx.x >= fsum.lines) {
+        static_assert(TH * W == 256, "the sums' 64 x 4 columns");
+        flow_sum_tile(g, us, fsum, reinterpret_cast<double *>(lds_raw));
+        return;
+    }
     double2 *lds = reinterpret_cast<double2 *>(lds_raw), *twl = lds + F::LPW * F::LS;
     const Dims d = g.d;
     const int npairs = d.ny * d.nz / 2, t = threadIdx.x % F::M, l = threadIdx.x / F::M;
@@ -1211,6 +1241,10 @@ __global__ __launch_bounds__(256) void fft_correct_kernel(GridK g, const double 
     }
 }
 
+bool fft_sums(const mdx_handle *h) {
+    return h->cfg.precision != MDX_PREC_MIXED && h->d.nx >= 16 && momentum_sums_apart(h);
+}
+
 // whether the projection takes u*'s ghosts as filled and writes the new fields' itself
 static int fft_wrap(const mdx_handle *h) { return h->step_bc && h->fused_bc; }
 
@@ -1360,9 +1394,13 @@ static hipError_t launch_rhs_xfft(mdx_handle *h, double dtg) {
     const Dims d = h->d;
     const int stride = fft_stride_t<double2>(d.nx);
 #define XF_(N, TH, W, S)                                                                                              \
-    return rf_launch<double2, N, TH, rhs_xfft_reg_kernel<N, TH, W, S>, W>(                                            \
-        h->stream, rf_row_blocks<N, TH>(d), g, (const double *)h->us, (const double *)h->vs, (const double *)h->ws, dtg, \
-        fft_wrap(h), (const double2 *)h->tw_x, stride, (double2 *)h->hat)
+    do {                                                                                                              \
+        const unsigned nb = rf_row_blocks<N, TH>(d);                                                                  \
+        const FlowSum fsum{(int)nb, h->mom_kz, h->fr_part};                                                           \
+        return rf_launch<double2, N, TH, rhs_xfft_reg_kernel<N, TH, W, S>, W>(                                        \
+            h->stream, nb + (h->step_sum ? momentum_tiles(h) : 0), g, (const double *)h->us, (const double *)h->vs,   \
+            (const double *)h->ws, dtg, fft_wrap(h), fsum, (const double2 *)h->tw_x, stride, (double2 *)h->hat);      \
+    } while (0)
 #define XF(N)                                                  \
     if (rf_small(rf_row_blocks<N, 256>(d))) {                  \
         if (h->stretched) XF_(N, 64, 4, true);                 \

@@ -94,6 +94,34 @@ __device__ inline bool xcd_tile(int items_x, int items_y, int nz, int bxx, int b
     return true;
 }
 
+// the sums of a workgroup's first NW waves' fa and fb into frpart[2 wg], frpart[2 wg + 1], in a fixed
+// order: a butterfly within each wave (every lane ends with the same sums), then the waves in index
+// order.  s: 2 NW values of LDS; every thread calls it (barrier)
+template <int NW>
+__device__ inline void flow_tile_sum(double fa, double fb, int tid, double *s, double *__restrict__ frpart, size_t wg) {
+    if (tid < 64 * NW) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            fa += __shfl_xor(fa, o);
+            fb += __shfl_xor(fb, o);
+        }
+        if ((tid & 63) == 0) {
+            s[tid >> 6] = fa;
+            s[NW + (tid >> 6)] = fb;
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {
+        double a = 0.0, b = 0.0;
+        for (int w = 0; w < NW; ++w) {
+            a += s[w];
+            b += s[NW + w];
+        }
+        frpart[2 * wg] = a;
+        frpart[2 * wg + 1] = b;
+    }
+}
+
 // The flow-rate correction from the n partial sums (pairs u*, mu_u) in part, by a workgroup of 256
 // (t: its thread; s1, s2: 256 values of LDS each): o = bulk velocity, mean mu_u, du = (target - ub)
 // / mean mu_u, the same in every thread.  The lanes' sums fold in halves, 128 down to 1, the last six
@@ -254,6 +282,7 @@ struct mdx_handle {
     // adds the flow-rate shift of the step_parts partial sums in fr_part (0: none) and, in the
     // step's last stage, stores the shifted u*
     int step_parts = 0;
+    bool step_sum = false;     // the partial sums are the right-hand side's to form (momentum_sums_apart)
     bool step_last = false;
     // streaming red-black sweeps: z planes marched per thread (0: one cell per thread)
     int sweep_kz = 4;
@@ -357,6 +386,8 @@ BcK bc_k(const mdx_handle *h);
 
 // frpart: the tiled kernel also writes the flow-rate partial sums of its momentum_tiles(h) tiles
 hipError_t launch_momentum(mdx_handle *h, double dta, double dtb, double dtg, double *frpart = nullptr);
+// whether momentum is faster without the flow-rate sums (its tiles of 64 x 4 columns are few)
+bool momentum_sums_apart(const mdx_handle *h);
 int momentum_tiles(const mdx_handle *h);
 int momentum_default_planes(const Dims &d);
 // array sets of the FFT build's apply_bc: the current fields and the predictor's
@@ -447,6 +478,7 @@ hipError_t rb_build_xlists(mdx_handle *h, const RbPlanOut &p, int *xl);
 
 // FFT path
 int fft_stride(int nx, bool fp32);   // complex elements per kx row of the spectrum
+bool fft_sums(const mdx_handle *h);   // a step's right-hand side forms the flow-rate sums
 hipError_t launch_fft_forward(mdx_handle *h, double dtg);
 hipError_t launch_tridiag(mdx_handle *h);
 hipError_t launch_fft_backward_correct(mdx_handle *h, double dtg);

@@ -171,7 +171,8 @@ __global__ __launch_bounds__(BX * BY) void momentum_kernel(
 }
 
 // LDS-tiled momentum: a 64 x TY workgroup owns a 64 x TY column of cells and marches mkz planes in z
-// (8 or 12, momentum_default_planes; 4, 16 and 32 measured slower).  The u, v, w planes k-1, k, k+1 (with a one-cell
+// (8 or 12, momentum_default_planes; 4, 16 and 32 measured slower on grids that fill the chip; fewer on
+// small ones, launch_momentum).  The u, v, w planes k-1, k, k+1 (with a one-cell
 // x-y halo) and the p plane k live in LDS as a rolling window, so each value is fetched from global
 // memory about 1.3 (x-y halo) x (mkz+2)/mkz (z halo) times instead of once per stencil use (about
 // 30 loads per cell in the direct kernel).
@@ -294,32 +295,9 @@ __global__ __launch_bounds__(MTX * TY) void momentum_tiled_kernel(
         m = mn;
         __syncthreads();
     }
-    if (FR) {
-        // a fixed order: a butterfly within each wave (every lane ends with the same sums), then
-        // the waves in index order; the window's LDS is free after the march's last barrier
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            fa += __shfl_xor(fa, o);
-            fb += __shfl_xor(fb, o);
-        }
-        constexpr int NW = MTX * TY / 64;
-        if ((tid & 63) == 0) {
-            su[tid >> 6] = fa;
-            su[NW + (tid >> 6)] = fb;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            double a = 0.0, b = 0.0;
-            for (int w = 0; w < NW; ++w) {
-                a += su[w];
-                b += su[NW + w];
-            }
-            const size_t nbx = (d.nx + MTX - 1) / MTX, nby = (d.ny + TY - 1) / TY;
-            const size_t wg = (size_t)tx + nbx * ((size_t)ty + nby * (size_t)tz);
-            frpart[2 * wg] = a;
-            frpart[2 * wg + 1] = b;
-        }
-    }
+    // (the window's LDS is free after the march's last barrier)
+    if (FR) flow_tile_sum<MTX * TY / 64>(fa, fb, tid, su, frpart, (size_t)tx + (size_t)((d.nx + MTX - 1) / MTX) *
+                                         ((size_t)ty + (size_t)((d.ny + TY - 1) / TY) * (size_t)tz));
 }
 
 // rows per tiled workgroup (TY above) when each marches kz planes
@@ -345,19 +323,36 @@ int momentum_default_planes(const Dims &d) {
     return fill(12) > fill(8) ? 12 : 8;
 }
 
-int momentum_tiles(const mdx_handle *h) {
-    const int ty = momentum_rows(h);
-    return ((h->d.nx + MTX - 1) / MTX) * ((h->d.ny + ty - 1) / ty) * ((h->d.nz + h->mom_kz - 1) / h->mom_kz);
+static long momentum_groups(const Dims &d, int ty, int kz) {
+    return (long)((d.nx + MTX - 1) / MTX) * ((d.ny + ty - 1) / ty) * ((d.nz + kz - 1) / kz);
+}
+int momentum_tiles(const mdx_handle *h) { return (int)momentum_groups(h->d, momentum_rows(h), h->mom_kz); }
+static constexpr long MOM_FULL = 768;   // workgroups from which the long march wins (launch_momentum)
+// (64^3 with sums, in a step: 22.6 us; without 12.0, and the sums ride in the FFT's first launch)
+bool momentum_sums_apart(const mdx_handle *h) {
+    return h->tiled_momentum && momentum_rows(h) == 4 && momentum_tiles(h) < MOM_FULL;
 }
 
 hipError_t launch_momentum(mdx_handle *h, double dta, double dtb, double dtg, double *frpart) {
     GridK g = grid_k(h);
     const double dx = h->dx, dy = h->dy, dz = h->dz;
     const double dx2 = dx * dx, dy2 = dy * dy, dz2 = dz * dz;
-    const bool tiled = h->tiled_momentum;
-    const int mkz = h->mom_kz;
+    int mkz = h->mom_kz, ty = momentum_rows(h);
+    bool tiled = h->tiled_momentum;
+    if (tiled && !frpart) {
+        // Without the sums, which follow the tiling, a workgroup marches fewer planes where that many
+        // give every CU less than three of them, and the smallest grids go a thread per cell (a march
+        // is a chain of loads and barriers; hot caches, 8 planes against these): 14.9 -> 4.0 us at
+        // 32 x 24 x 16 (per cell; 5.4 tiled), 16.9 -> 8.9 at 64^3 (1 plane; 9.9 per cell), 18.3 -> 12.4 at
+        // 100 x 70 x 54 (2; 13.8 with 4), 22.6 -> 19.4 at 128 x 97 x 64 (4; 20.6 with 2); from 768
+        // workgroups on the longer march wins (192 x 128 x 96: 40.3 with 12 planes, 43.8 with 4).
+        while (mkz > 1 && momentum_groups(h->d, ty, mkz) < MOM_FULL) {
+            mkz = mkz > 8 ? 8 : mkz / 2;
+            ty = 4;
+        }
+        tiled = momentum_groups(h->d, ty, mkz) >= 256;
+    }
     const int nseg = (h->d.nz + mkz - 1) / mkz;
-    const int ty = momentum_rows(h);
     dim3 blk = tiled ? dim3(MTX, ty, 1) : dim3(BX, BY, 1);
     dim3 grd(tiled ? xcd_grid(h->d.nx, h->d.ny, nseg, MTX, ty) : xcd_grid(h->d.nx, h->d.ny, h->d.nz, BX, BY));
     // the partials come from the tiled kernel, over a periodic x (as constant flow rate requires)

@@ -1073,10 +1073,10 @@ static int wait_check(mdx_handle *h, int w, unsigned long long seq, double *r) {
             if (q == hipErrorNotReady) continue;
             if (*sq == seq) break;
             if (q != hipSuccess) {
-                mdx_set_error(std::string("SOR check: ") + hipGetErrorString(q));
+                mdx_set_error(std::string("residual check: ") + hipGetErrorString(q));
                 return MDX_ERR_HIP;
             }
-            mdx_set_error("SOR check: the stream finished without posting its residual");
+            mdx_set_error("residual check: the stream finished without posting its residual");
             return MDX_ERR_HIP;
         }
         _mm_pause();
@@ -1087,6 +1087,12 @@ static int wait_check(mdx_handle *h, int w, unsigned long long seq, double *r) {
     std::memcpy(&err, &h->h_pinned[w + 1], sizeof err);
     if (err) return lds_timeout_seen(h);
     return MDX_OK;
+}
+
+// wait_check for the FFT's checks, which an error word of an earlier batch does not concern (read_norm)
+static int wait_norm(mdx_handle *h, int w, unsigned long long seq, double *r) {
+    const int rc = wait_check(h, w, seq, r);
+    return rc == MDX_LDS_TIMEOUT ? MDX_OK : rc;
 }
 
 // Plain FP64 red-black SOR to ||div||_inf < tol; Phi starts at zero (the previous-step pressure).
@@ -1553,27 +1559,44 @@ extern "C" int mdx_pressure_projection(mdx_handle *h, double dtg, mdx_solve_stat
         // FP32 transforms and Thomas solves in an FP64 defect correction: from phi = 0, each pass
         // solves L e = rhs - L phi (mean mode in FP64, the rest in FP32) and adds e, until
         // ||div||_inf = dt_gamma ||rhs - L phi||_inf < tol (at most MAX_FFT_PASSES passes)
+        // The first pass and its check are queued before the first check (max |rhs|) is read: one
+        // wait for the host instead of two where a pass converges, as it nearly always does.  A
+        // residual is only stored once it is known that another pass needs it.
         constexpr int MAX_FFT_PASSES = 4;
+        double *const slot = h->d_pinned + CHECK_PIN;
+        int passes = 1, rc;
+        double r = 0.0, r0 = 0.0;
         ev_record(h, 1);
-        MDX_HIP(launch_fft_mixed_setup(h, dtg));
-        int passes = 0, rc;
-        double r = 0.0;
+        const unsigned long long seq0 = ++h->chk_seq;
+        MDX_HIP(launch_fft_mixed_setup(h, dtg, slot, seq0));
+        MDX_HIP(launch_fft32_solve_add(h, true));
         for (;;) {
-            MDX_HIP(launch_reset_max(h));
-            MDX_HIP(launch_fft_residual(h));
-            if ((rc = read_norm(h, &r))) return rc;
-            if (passes == 0) st.div0_inf = r * dtg;
+            const unsigned long long seq = ++h->chk_seq;
+            MDX_HIP(launch_fft_residual(h, false, slot + 4, seq));
+            MDX_HIP(launch_fft_pin(h));
+            if ((rc = wait_norm(h, CHECK_PIN + 4, seq, &r))) return rc;
+            if (passes == 1) {
+                if ((rc = wait_norm(h, CHECK_PIN, seq0, &r0))) return rc;
+                st.div0_inf = r0 * dtg;
+                ++st.checks;
+                if (!(r0 * dtg >= c.tol)) {   // converged as it stood (or not a number): phi = 0
+                    passes = 0;
+                    r = r0;
+                    MDX_HIP(launch_zero64(h, h->fft_phi, h->ni));
+                    break;
+                }
+            }
             ++st.checks;
             if (!(r * dtg >= c.tol) || passes >= MAX_FFT_PASSES) break;
-            MDX_HIP(launch_fft32_solve_add(h));
+            MDX_HIP(launch_fft_residual(h, true, nullptr, 0));
+            MDX_HIP(launch_fft32_solve_add(h, false));
             ++passes;
         }
         st.iterations = passes;
         st.div_inf = r * dtg;
         st.converged = r * dtg < c.tol;
-        MDX_HIP(launch_fft_pin(h));
         ev_record(h, 2);
-        MDX_HIP(launch_fft_correct(h, h->fft_phi, dtg));
+        MDX_HIP(launch_fft_correct(h, dtg, passes > 0));
         ev_record(h, 3);
     } else if (c.solver == MDX_SOLVER_FFT) {
         ev_record(h, 1);

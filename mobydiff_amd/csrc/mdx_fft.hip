@@ -435,15 +435,17 @@ __global__ __launch_bounds__(TH) void ixfft_reg_kernel(Dims d, const double2 *__
         p[N + F::M * s] = e[s].y * scale;
     }
 }
-// 5. (FP32) inverse x-transform of each row, scaled and added to the FP64 phi
-template <int N, int TH>
+// 5. (FP32) inverse x-transform of each row, scaled, and the mean mode's solution added to the FP64 phi
+// (FIRST: to zero)
+template <int N, int TH, bool FIRST>
 __global__ __launch_bounds__(TH) void ixfft32_add_reg_kernel(Dims d, const float2 *__restrict__ hat,
                                                              const float2 *__restrict__ tw, int stride, float scale,
-                                                             double *__restrict__ phi) {
+                                                             const double *__restrict__ mean, double *__restrict__ phi) {
     using F = RFft<N, TH>;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     float2 *lds = reinterpret_cast<float2 *>(lds_raw), *twl = lds + F::LPW * F::LS;
     const int nrows = d.ny * d.nz, t = threadIdx.x % F::M, r = blockIdx.x * F::LPW + threadIdx.x / F::M;
+    const double mj = mean[r < nrows ? r / d.nz : 0];
     rf_stage<float2, N, TH>(twl, tw);
     const float2 *h = hat + (size_t)stride * (r < nrows ? r : 0);
     double *p = phi + (size_t)N * (r < nrows ? r : 0) + t;
@@ -459,7 +461,7 @@ __global__ __launch_bounds__(TH) void ixfft32_add_reg_kernel(Dims d, const float
             const float2 c = h[N - q];
             e[s] = make_float2(c.x, s == 8 && 2 * q == N ? 0.f : -c.y);
         }
-        a[s] = p[F::M * s];
+        a[s] = FIRST ? mj : p[F::M * s] + mj;
     }
     fft_line<float2, N, true>(e, t, twl, lds + threadIdx.x / F::M * F::LS);
     if (r >= nrows) return;
@@ -1490,11 +1492,12 @@ hipError_t launch_fft_backward_correct(mdx_handle *h, double dtg) {
 // are fetched about once; v*(j+1) is the row above's v*(j) (a cache hit).  wrap: as in
 // rhs_xfft_reg_kernel; fs: the flow-rate shift of u*, added before the differences (it drops out of
 // them but for rounding, which the FP32 passes would turn into differences of their own precision).
+// The first pass starts from phi = 0, whose residual is the right-hand side, so max |rhs| is formed here.
 template <bool STRETCH>
 __global__ __launch_bounds__(64 * FC_Y) void fft_div_rhs_kernel(GridK g, const double *__restrict__ us,
                                                                const double *__restrict__ vs,
                                                                const double *__restrict__ ws, double dtg, int wrap,
-                                                               FftStep fs, double *__restrict__ rhs) {
+                                                               FftStep fs, double *__restrict__ rhs, double *part) {
     static_assert(64 * FC_Y == 256, "the fold's threads");
     const Dims d = g.d;
     double du = 0.0;
@@ -1509,7 +1512,7 @@ __global__ __launch_bounds__(64 * FC_Y) void fft_div_rhs_kernel(GridK g, const d
     const int j = blockIdx.y * FC_Y + threadIdx.y + 1;
     const int k0 = blockIdx.z * FC_KZ + 1, k1 = k0 + FC_KZ - 1 < d.nz ? k0 + FC_KZ - 1 : d.nz;
     const bool act = i <= d.nx && j <= d.ny;
-    double wk = act ? ws[d.g(i, j, k0)] : 0.0;
+    double wk = act ? ws[d.g(i, j, k0)] : 0.0, m = 0.0;
     for (int k = k0; k <= k1; ++k) {
         double uc = 0.0, up = 0.0, vj = 0.0, vjp = 0.0, wkp = 0.0;
         if (act) {
@@ -1526,11 +1529,13 @@ __global__ __launch_bounds__(64 * FC_Y) void fft_div_rhs_kernel(GridK g, const d
         }
         if (act) {
             const double dv = STRETCH ? (vjp - vj) * g.ihc[j] : (vjp - vj) / g.dy;
-            rhs[(size_t)(i - 1) + (size_t)d.nx * ((size_t)(k - 1) + (size_t)d.nz * (size_t)(j - 1))] =
-                ((up - uc) / g.dx + dv + (wkp - wk) / g.dz) / dtg;
+            const double r = ((up - uc) / g.dx + dv + (wkp - wk) / g.dz) / dtg;
+            rhs[(size_t)(i - 1) + (size_t)d.nx * ((size_t)(k - 1) + (size_t)d.nz * (size_t)(j - 1))] = r;
+            m = nanmax_any(m, fabs(r));
         }
         wk = wkp;
     }
+    block_max_part(m, part);
 }
 
 // partial sums of the (nx, nz) planes: workgroup (plane j, chunk c) sums chunk c of PLANE_CHUNKS
@@ -1589,55 +1594,58 @@ __global__ __launch_bounds__(256) void fft_mean_mode_kernel(Dims d, const double
     for (int q = threadIdx.x; q < ny; q += 256) mean[q] = sm[q];
 }
 
-// phi += mean[j] everywhere in plane j
-__global__ void fft_add_mean_kernel(Dims d, const double *__restrict__ mean, double *__restrict__ phi) {
-    const long n = (long)d.nx * d.ny * d.nz;
-    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x)
-        phi[q] += mean[q / ((long)d.nx * d.nz)];
-}
-
-// phi -= (plane-1 sum of phi) / (nx nz): re-imposes the pin phi_hat(y_1) = 0 exactly (the FP32
-// inverse transforms leave plane means of the order of their rounding, and a constant is invisible
-// to the residual); velocities see only differences of phi and do not change
-__global__ void fft_pin_kernel(Dims d, const double *__restrict__ part, double *__restrict__ phi) {
-    const long n = (long)d.nx * d.ny * d.nz;
-    const double c = plane_sum(part, 0) / (double)((long)d.nx * d.nz);
-    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) phi[q] -= c;
-}
-
-// res = rhs - L phi (FP64), and max |res| per workgroup; layout (nx, nz, ny), x and z periodic
-template <bool STRETCH>
+// max |rhs - L phi| (FP64) per workgroup, and with STORE the residual itself, which only a further pass
+// reads; layout (nx, nz, ny), x and z periodic.  A thread takes a column (i, k) of a 64 x 4 tile and
+// marches jm rows, FR_CH rows' loads in flight and phi(j-1), phi(j) in registers.  Bound by HBM: 16 B
+// per cell, 24 with STORE (256 x 192 x 256: 121 us before, a thread per cell with 64-bit index divisions
+// and always storing; 51 and 68 now).
+static constexpr int FR_CH = 4;
+template <bool STRETCH, bool STORE>
 __global__ __launch_bounds__(256) void fft_residual_kernel(GridK g, const double *__restrict__ rhs,
                                                            const double *__restrict__ phi, const double *__restrict__ arow,
-                                                           double *__restrict__ res, double *part) {
+                                                           int jm, double *__restrict__ res, double *part) {
     const Dims d = g.d;
     const int nx = d.nx, ny = d.ny, nz = d.nz;
-    const long n = (long)nx * ny * nz;
+    const int i0 = blockIdx.x * 64 + threadIdx.x, k0 = blockIdx.y * 4 + threadIdx.y;   // 0-based
+    const bool act = i0 < nx && k0 < nz;
+    const int i = act ? i0 : 0, k = act ? k0 : 0;
+    const int j0 = blockIdx.z * jm, j1 = j0 + jm < ny ? j0 + jm : ny;
     const double idx2 = 1.0 / (g.dx * g.dx), idz2 = 1.0 / (g.dz * g.dz);
-    double m = 0.0;
-    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
-        const int i = (int)(q % nx);
-        const long r = q / nx;
-        const int k = (int)(r % nz), j = (int)(r / nz);   // 0-based
-        const long row = q - i;
-        const double p0 = phi[q];
-        const double pxp = phi[row + (i + 1 == nx ? 0 : i + 1)], pxm = phi[row + (i == 0 ? nx - 1 : i - 1)];
-        const long plane = (long)nx * nz * j;
-        const long kp = k + 1 == nz ? 0 : k + 1, km = k == 0 ? nz - 1 : k - 1;
-        const double pzp = phi[plane + (long)nx * kp + i], pzm = phi[plane + (long)nx * km + i];
-        double ly = 0.0;
-        if (j > 0) ly += arow[j] * (phi[q - (long)nx * nz] - p0);
-        if (j < ny - 1) {
-            const double c = STRETCH ? g.ihv[j + 2] * g.ihc[j + 1] : arow[j + 1];
-            ly += c * (phi[q + (long)nx * nz] - p0);
+    const ptrdiff_t sp = (ptrdiff_t)nx * nz;
+    const ptrdiff_t xp = i + 1 == nx ? 1 - nx : 1, xm = i == 0 ? nx - 1 : -1;
+    const ptrdiff_t zp = k + 1 == nz ? (ptrdiff_t)nx * (1 - nz) : nx, zm = k == 0 ? (ptrdiff_t)nx * (nz - 1) : -(ptrdiff_t)nx;
+    const size_t q0 = (size_t)i + (size_t)nx * ((size_t)k + (size_t)nz * (size_t)j0);
+    const double *p = phi + q0, *f = rhs + q0;
+    double m = 0.0, pm = j0 > 0 ? p[-sp] : 0.0, p0 = p[0];
+    for (int j = j0; j < j1; j += FR_CH, p += FR_CH * sp, f += FR_CH * sp) {
+        double py[FR_CH], a[FR_CH], b[FR_CH], c[FR_CH], e[FR_CH], r[FR_CH];
+#pragma unroll
+        for (int u = 0; u < FR_CH; ++u) {   // past the end: the last row again, unused
+            const int w = j + u < j1 ? u : j1 - 1 - j;
+            const double *q = p + w * sp;
+            a[u] = q[xp];
+            b[u] = q[xm];
+            c[u] = q[zp];
+            e[u] = q[zm];
+            r[u] = f[w * sp];
+            py[u] = j + w + 1 < ny ? q[sp] : 0.0;
         }
-        const double lap = (pxp - 2.0 * p0 + pxm) * idx2 + (pzp - 2.0 * p0 + pzm) * idz2 + ly;
-        const double rr = rhs[q] - lap;
-        res[q] = rr;
-        const double a = fabs(rr);
-        m = nanmax_any(m, a);
+#pragma unroll
+        for (int u = 0; u < FR_CH; ++u) {
+            const int jj = j + u;
+            if (jj >= j1) break;
+            double ly = 0.0;
+            if (jj > 0) ly += arow[jj] * (pm - p0);
+            if (jj < ny - 1) ly += (STRETCH ? g.ihv[jj + 2] * g.ihc[jj + 1] : arow[jj + 1]) * (py[u] - p0);
+            const double lap = (a[u] - 2.0 * p0 + b[u]) * idx2 + (c[u] - 2.0 * p0 + e[u]) * idz2 + ly;
+            const double rr = r[u] - lap;
+            if (STORE && act) res[q0 + (size_t)(jj - j0) * sp] = rr;
+            m = nanmax_any(m, fabs(rr));
+            pm = p0;
+            p0 = py[u];
+        }
     }
-    block_max_part(m, part);
+    block_max_part(act ? m : 0.0, part);
 }
 
 // 1. (FP32) r2c x-transform of a real FP64 field in (nx, nz, ny) layout
@@ -1731,10 +1739,11 @@ __global__ __launch_bounds__(64) void tridiag32_kernel(Dims d, int stride, float
     }
 }
 
-// 5. (FP32) c2r x-transform, scaled, added to the FP64 phi
+// 5. (FP32) c2r x-transform, scaled, and the mean mode's solution added to the FP64 phi (first: to zero)
 __global__ __launch_bounds__(FFT_THREADS) void ixfft32_add_kernel(Dims d, const float2 *__restrict__ hat,
                                                                   const float2 *__restrict__ tw, int lines, int stride,
-                                                                  float scale, double *phi) {
+                                                                  float scale, const double *__restrict__ mean, int first,
+                                                                  double *phi) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     float2 *lds = reinterpret_cast<float2 *>(lds_raw);
     const int n = d.nx, nxh = n / 2 + 1;
@@ -1758,45 +1767,53 @@ __global__ __launch_bounds__(FFT_THREADS) void ixfft32_add_kernel(Dims d, const 
     for (int t = threadIdx.x; t < lines * n; t += FFT_THREADS) {
         const int line = t / n, i = t - line * n;
         const int r = blockIdx.x * lines + line;
-        if (r < nrows) phi[(size_t)n * r + i] += (double)(res[t].x * scale);
+        if (r < nrows) {
+            const double p = (first ? 0.0 : phi[(size_t)n * r + i]) + mean[r / d.nz];
+            phi[(size_t)n * r + i] = p + (double)(res[t].x * scale);
+        }
     }
 }
 
-// the FP64 right-hand side -> h->fft_rhs, phi = 0
-hipError_t launch_fft_mixed_setup(mdx_handle *h, double dtg) {
+// the FP64 right-hand side -> h->fft_rhs; its max |.| into the max reduction
+hipError_t launch_fft_mixed_setup(mdx_handle *h, double dtg, double *host_slot, unsigned long long seq) {
     GridK g = grid_k(h);
-    const FftStep fs = fft_step(h);
     const Dims d = h->d;
     dim3 blk(64, FC_Y), grd((d.nx + 63) / 64, (d.ny + FC_Y - 1) / FC_Y, (d.nz + FC_KZ - 1) / FC_KZ);
-    if (h->stretched)
-        hipLaunchKernelGGL(fft_div_rhs_kernel<true>, grd, blk, 0, h->stream, g, h->us, h->vs, h->ws, dtg, fft_wrap(h), fs, h->fft_rhs);
-    else
-        hipLaunchKernelGGL(fft_div_rhs_kernel<false>, grd, blk, 0, h->stream, g, h->us, h->vs, h->ws, dtg, fft_wrap(h), fs, h->fft_rhs);
-    hipError_t e = hipGetLastError();
-    return e != hipSuccess ? e : launch_zero64(h, h->fft_phi, h->ni);
+#define MDX_RHS(S)                                                                                              \
+    hipLaunchKernelGGL(fft_div_rhs_kernel<S>, grd, blk, 0, h->stream, g, h->us, h->vs, h->ws, dtg, fft_wrap(h), \
+                       fft_step(h), h->fft_rhs, h->max_part)
+    if (h->stretched) MDX_RHS(true);
+    else MDX_RHS(false);
+#undef MDX_RHS
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess ? e : launch_max_final(h, grd.x * grd.y * grd.z, host_slot, seq);
 }
 
-// res = rhs - L phi into h->fft_res; its max |.| into the max reduction
-hipError_t launch_fft_residual(mdx_handle *h) {
+// max |rhs - L phi| into the max reduction, or (store) the residual into h->fft_res
+hipError_t launch_fft_residual(mdx_handle *h, bool store, double *host_slot, unsigned long long seq) {
     GridK g = grid_k(h);
-    const unsigned blocks = 2048;
-    if (h->stretched)
-        hipLaunchKernelGGL(fft_residual_kernel<true>, dim3(blocks), dim3(256), 0, h->stream, g, h->fft_rhs, h->fft_phi,
-                           h->arow, h->fft_res, h->max_part);
-    else
-        hipLaunchKernelGGL(fft_residual_kernel<false>, dim3(blocks), dim3(256), 0, h->stream, g, h->fft_rhs,
-                           h->fft_phi, h->arow, h->fft_res, h->max_part);
-    hipError_t e = hipGetLastError();
-    return e != hipSuccess ? e : launch_max_final(h, blocks);
+    const Dims d = h->d;
+    int jm = 16;   // rows per workgroup, fewer while that leaves CUs without four workgroups
+    auto groups = [&](int m) { return (unsigned)((d.nx + 63) / 64 * ((d.nz + 3) / 4) * ((d.ny + m - 1) / m)); };
+    while (jm > FR_CH && groups(jm) < 1024) jm /= 2;
+    const dim3 grd((d.nx + 63) / 64, (d.nz + 3) / 4, (d.ny + jm - 1) / jm);
+#define MDX_RES(S, T)                                                                                           \
+    hipLaunchKernelGGL((fft_residual_kernel<S, T>), grd, dim3(64, 4), 0, h->stream, g, h->fft_rhs, h->fft_phi,  \
+                       h->arow, jm, h->fft_res, h->max_part)
+    if (h->stretched) { if (store) MDX_RES(true, true); else MDX_RES(true, false); }
+    else { if (store) MDX_RES(false, true); else MDX_RES(false, false); }
+#undef MDX_RES
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess || store ? e : launch_max_final(h, groups(jm), host_slot, seq);
 }
 
 // the FP32 x-transforms of the defect solves
-static hipError_t launch_xfft32(mdx_handle *h) {
+static hipError_t launch_xfft32(mdx_handle *h, const double *res) {
     const Dims d = h->d;
     const int stride = fft_stride_t<float2>(d.nx);
 #define XF_(N, TH)                                                                                               \
     return rf_launch<float2, N, TH, xfft32_reg_kernel<N, TH>>(h->stream, rf_row_blocks<N, TH>(d, 1), d,          \
-                                                              (const double *)h->fft_res,                        \
+                                                              res,                                               \
                                                               (const float2 *)h->tw_x32, stride, (float2 *)h->hat32)
 #define XF(N)                                                \
     if (rf_small(rf_row_blocks<N, 256>(d, 1))) XF_(N, 64);   \
@@ -1806,44 +1823,49 @@ static hipError_t launch_xfft32(mdx_handle *h) {
 #undef XF_
     const int lines = rows_per_block(d.nx), nrows = d.ny * d.nz;
     hipLaunchKernelGGL(xfft32_kernel, dim3((nrows + lines - 1) / lines), dim3(FFT_THREADS),
-                       fft_lds<float2>(lines, d.nx, d.nx), h->stream, d, h->fft_res, (const float2 *)h->tw_x32, lines,
+                       fft_lds<float2>(lines, d.nx, d.nx), h->stream, d, res, (const float2 *)h->tw_x32, lines,
                        stride, (float2 *)h->hat32);
     return hipGetLastError();
 }
 
-static hipError_t launch_ixfft32_add(mdx_handle *h) {
+static hipError_t launch_ixfft32_add(mdx_handle *h, const double *mean, bool first) {
     const Dims d = h->d;
     const int stride = fft_stride_t<float2>(d.nx);
     const float scale = 1.0f / (float)(d.nx * d.nz);
-#define IX_(N, TH)                                                                                               \
-    return rf_launch<float2, N, TH, ixfft32_add_reg_kernel<N, TH>>(h->stream, rf_row_blocks<N, TH>(d, 1), d,     \
-                                                                   (const float2 *)h->hat32,                     \
-                                                                   (const float2 *)h->tw_x32, stride, scale, h->fft_phi)
+#define IX_(N, TH, FIRST)                                                                                        \
+    return rf_launch<float2, N, TH, ixfft32_add_reg_kernel<N, TH, FIRST>>(h->stream, rf_row_blocks<N, TH>(d, 1), \
+                                                                          d, (const float2 *)h->hat32,           \
+                                                                          (const float2 *)h->tw_x32, stride,     \
+                                                                          scale, mean, h->fft_phi)
 #define IX(N)                                                \
-    if (rf_small(rf_row_blocks<N, 256>(d, 1))) IX_(N, 64);   \
-    IX_(N, 256)
+    if (rf_small(rf_row_blocks<N, 256>(d, 1))) {             \
+        if (first) IX_(N, 64, true);                         \
+        IX_(N, 64, false);                                   \
+    }                                                        \
+    if (first) IX_(N, 256, true);                            \
+    IX_(N, 256, false)
     RF_SIZES(d.nx, IX)
 #undef IX
 #undef IX_
     const int lines = rows_per_block(d.nx), nrows = d.ny * d.nz;
     hipLaunchKernelGGL(ixfft32_add_kernel, dim3((nrows + lines - 1) / lines), dim3(FFT_THREADS),
                        fft_lds<float2>(lines, d.nx, d.nx), h->stream, d, (const float2 *)h->hat32,
-                       (const float2 *)h->tw_x32, lines, stride, scale, h->fft_phi);
+                       (const float2 *)h->tw_x32, lines, stride, scale, mean, (int)first, h->fft_phi);
     return hipGetLastError();
 }
 
-// one defect-correction pass on res = rhs - L phi: the mean mode in FP64 (plane sums, pinned
-// Thomas), the other modes by FP32 transforms and Thomas; both corrections added to h->fft_phi
-hipError_t launch_fft32_solve_add(mdx_handle *h) {
+// one defect-correction pass on res = rhs - L phi (first: phi = 0 and res = rhs): the mean mode in FP64
+// (plane sums, pinned Thomas), the other modes by FP32 transforms and Thomas; both corrections added
+// to h->fft_phi
+hipError_t launch_fft32_solve_add(mdx_handle *h, bool first) {
     const Dims d = h->d;
     if (d.ny > MEAN_MAX_NY) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(fft_plane_sum_kernel, dim3(d.ny * PLANE_CHUNKS), dim3(256), 0, h->stream, d, h->fft_res,
-                       h->fft_mean);
+    const double *res = first ? h->fft_rhs : h->fft_res;
+    hipLaunchKernelGGL(fft_plane_sum_kernel, dim3(d.ny * PLANE_CHUNKS), dim3(256), 0, h->stream, d, res, h->fft_mean);
     double *mean = h->fft_mean + (size_t)d.ny * PLANE_CHUNKS;
     hipLaunchKernelGGL(fft_mean_mode_kernel, dim3(1), dim3(256), 0, h->stream, d, h->fft_mean, h->cp, h->den_inv,
                        h->arow, 1.0 / (double)(d.nx * d.nz), mean);
-    hipLaunchKernelGGL(fft_add_mean_kernel, dim3(4096), dim3(256), 0, h->stream, d, mean, h->fft_phi);
-    hipError_t e = launch_xfft32(h);
+    hipError_t e = launch_xfft32(h, res);
     if (e != hipSuccess) return e;
     if ((e = launch_zfft<float2, false>(h->stream, d, (float2 *)h->hat32, (const float2 *)h->tw_z32)) != hipSuccess)
         return e;
@@ -1857,17 +1879,20 @@ hipError_t launch_fft32_solve_add(mdx_handle *h) {
                            fft_stride_t<float2>(d.nx), (float2 *)h->hat32, h->cp32, h->den32, h->arow32);
     if ((e = launch_zfft<float2, true>(h->stream, d, (float2 *)h->hat32, (const float2 *)h->tw_z32)) != hipSuccess)
         return e;
-    return launch_ixfft32_add(h);
+    return launch_ixfft32_add(h, mean, first);
 }
 
+// the plane sums of phi in plane 1: the mean that launch_fft_correct takes off phi, which re-imposes the
+// pin phi_hat(y_1) = 0 exactly (the FP32 inverse transforms leave plane means of the order of their
+// rounding, and a constant is invisible to the residual; velocities see only differences)
 hipError_t launch_fft_pin(mdx_handle *h) {
-    const Dims d = h->d;
-    hipLaunchKernelGGL(fft_plane_sum_kernel, dim3(PLANE_CHUNKS), dim3(256), 0, h->stream, d, h->fft_phi, h->fft_mean);
-    hipLaunchKernelGGL(fft_pin_kernel, dim3(4096), dim3(256), 0, h->stream, d, h->fft_mean, h->fft_phi);
+    hipLaunchKernelGGL(fft_plane_sum_kernel, dim3(PLANE_CHUNKS), dim3(256), 0, h->stream, h->d, h->fft_phi, h->fft_mean);
     return hipGetLastError();
 }
 
-// the projection with a given FP64 phi in (nx, nz, ny) layout (step 6)
-hipError_t launch_fft_correct(mdx_handle *h, const double *phi, double dtg) { return launch_correct(h, phi, dtg, nullptr); }
+// the projection with the FP64 phi of the defect correction (step 6); pin: less its mean in plane 1
+hipError_t launch_fft_correct(mdx_handle *h, double dtg, bool pin) {
+    return launch_correct(h, h->fft_phi, dtg, pin ? h->fft_mean : nullptr);
+}
 
 }  // namespace mdx

@@ -482,11 +482,11 @@ bool fft_sums(const mdx_handle *h);   // a step's right-hand side forms the flow
 hipError_t launch_fft_forward(mdx_handle *h, double dtg);
 hipError_t launch_tridiag(mdx_handle *h);
 hipError_t launch_fft_backward_correct(mdx_handle *h, double dtg);
-hipError_t launch_fft_mixed_setup(mdx_handle *h, double dtg);
-hipError_t launch_fft_residual(mdx_handle *h);
-hipError_t launch_fft32_solve_add(mdx_handle *h);
+hipError_t launch_fft_mixed_setup(mdx_handle *h, double dtg, double *host_slot, unsigned long long seq);
+hipError_t launch_fft_residual(mdx_handle *h, bool store, double *host_slot, unsigned long long seq);
+hipError_t launch_fft32_solve_add(mdx_handle *h, bool first);
 hipError_t launch_fft_pin(mdx_handle *h);
-hipError_t launch_fft_correct(mdx_handle *h, const double *phi, double dtg);
+hipError_t launch_fft_correct(mdx_handle *h, double dtg, bool pin);
 }  // namespace mdx
 
 // error helpers

@@ -66,3 +66,29 @@ def test_mixed_solve_matches_fp64(shape):
         ch.close()
     for k in got[0]:
         assert _rel(got[1][k], got[0][k]) < 1e-7, (k, _rel(got[1][k], got[0][k]))
+
+
+@pytest.mark.parametrize("shape", [(16, 6, 16), (8, 7, 64), (96 + 32, 33, 32), (64, 257, 256)])
+@pytest.mark.parametrize("tol,passes", [(1e-2, 1), (1e-9, 2)])
+def test_mixed_passes(shape, tol, passes):
+    """One pass, several, and none: a predictor that is divergence-free within the tolerance already
+    (the projected field again, its ghosts filled) stays as it is."""
+    print(shape, tol, flush=True)
+    g = O.Grid(*shape, lx=2.0, ly=2.0, lz=1.0, periodic=(1, 0, 1), beta=1.5)
+    f = O.random_fields(g, np.random.default_rng(33))
+    ch = _channel(g, f, precision=M.PREC_MIXED, tol=tol)
+    ch.apply_bc()
+    st = ch.pressure_projection(0.07)
+    assert st.converged == 1 and st.checks == st.iterations + 1 and st.div0_inf > 1.0 and st.div_inf < tol
+    assert st.iterations == 1 if passes == 1 else st.iterations >= 1
+    ch.apply_bc()
+    out = ch.download()
+    ch.upload(us=out["un"], vs=out["vn"], ws=out["wn"])
+    again = ch.pressure_projection(0.07)
+    assert again.converged == 1 and again.iterations == 0 and again.checks == 1
+    assert again.div_inf == again.div0_inf
+    ch.apply_bc()
+    new = ch.download()
+    for k in ("un", "vn", "wn", "pn"):
+        assert np.array_equal(new[k], out[k]), k
+    ch.close()

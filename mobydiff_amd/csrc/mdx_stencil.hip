@@ -21,11 +21,13 @@ struct MomOld {
     double ru, rv, rw, cu, cv, cw;
 };
 
-template <bool IBM>
+// NT: the old right-hand sides are loaded and stored past the caches (launch_momentum)
+template <bool IBM, bool NT>
 __device__ inline MomOld mom_old(const double *__restrict__ oru, const double *__restrict__ orv,
                                  const double *__restrict__ orw, const double *__restrict__ cu,
                                  const double *__restrict__ cv, const double *__restrict__ cw, size_t o, size_t cc) {
-    MomOld m{oru[o], orv[o], orw[o], 0.0, 0.0, 0.0};
+    MomOld m{NT ? __builtin_nontemporal_load(oru + o) : oru[o], NT ? __builtin_nontemporal_load(orv + o) : orv[o],
+             NT ? __builtin_nontemporal_load(orw + o) : orw[o], 0.0, 0.0, 0.0};
     if (IBM) {
         m.cu = cu[cc];
         m.cv = cv[cc];
@@ -34,8 +36,13 @@ __device__ inline MomOld mom_old(const double *__restrict__ oru, const double *_
     return m;
 }
 
+template <bool NT> __device__ inline void put_old(double *p, double v) {
+    if (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+
 // returns the u* it stores (0 where the cell's u is a boundary value it does not update)
-template <bool STRETCH, bool IBM, class Acc>
+template <bool STRETCH, bool IBM, bool NT, class Acc>
 __device__ inline double momentum_cell(const GridK &g, const Acc &L, int i, int j, int k, size_t c, size_t o,
                                      const MomOld &m, double *__restrict__ us, double *__restrict__ vs,
                                      double *__restrict__ ws, double *__restrict__ oru, double *__restrict__ orv,
@@ -71,7 +78,7 @@ __device__ inline double momentum_cell(const GridK &g, const Acc &L, int i, int 
         double s = u0 + dta * rhsu + dtb * m.ru - dtg * dpx;
         if (IBM) s = s * (1.0 / (1.0 + dtg * m.cu));
         us[c] = s;
-        oru[o] = rhsu;
+        put_old<NT>(oru + o, rhsu);
         ustar = s;
     }
     if (j >= ny0) {
@@ -101,7 +108,7 @@ __device__ inline double momentum_cell(const GridK &g, const Acc &L, int i, int 
         double s = v0 + dta * rhsv + dtb * m.rv - dtg * dpy;
         if (IBM) s = s * (1.0 / (1.0 + dtg * m.cv));
         vs[c] = s;
-        orv[o] = rhsv;
+        put_old<NT>(orv + o, rhsv);
     }
     if (k >= nz0) {
         const double w0 = L.w(0, 0, 0), wip = L.w(1, 0, 0), wim = L.w(-1, 0, 0);
@@ -129,7 +136,7 @@ __device__ inline double momentum_cell(const GridK &g, const Acc &L, int i, int 
         double s = w0 + dta * rhsw + dtb * m.rw - dtg * dpz;
         if (IBM) s = s * (1.0 / (1.0 + dtg * m.cw));
         ws[c] = s;
-        orw[o] = rhsw;
+        put_old<NT>(orw + o, rhsw);
     }
     return ustar;
 }
@@ -165,8 +172,8 @@ __global__ __launch_bounds__(BX * BY) void momentum_kernel(
     const MomGlobal L{un, vn, wn, pn, d, i, j, k};
     // coefficient index: z-invariant geometries keep one x-y plane (coef_kstride 0)
     const size_t o = d.in(i, j, k);
-    const MomOld m = mom_old<IBM>(oru, orv, orw, cu, cv, cw, o, d.g(i, j, k * coef_kstride));
-    momentum_cell<STRETCH, IBM>(g, L, i, j, k, d.g(i, j, k), o, m, us, vs, ws, oru, orv, orw, dta, dtb, dtg, idx, idy,
+    const MomOld m = mom_old<IBM, false>(oru, orv, orw, cu, cv, cw, o, d.g(i, j, k * coef_kstride));
+    momentum_cell<STRETCH, IBM, false>(g, L, i, j, k, d.g(i, j, k), o, m, us, vs, ws, oru, orv, orw, dta, dtb, dtg, idx, idy,
                                 idz, idx2, idy2, idz2, ire);
 }
 
@@ -195,7 +202,7 @@ struct MomTile {
     __device__ inline double p(int a, int b, int c) const { return c == 0 ? sp[t + a + MTW * b] : pkm; }
 };
 
-template <bool STRETCH, bool IBM, int TY, bool FR>
+template <bool STRETCH, bool IBM, int TY, bool FR, bool NT>
 __global__ __launch_bounds__(MTX * TY) void momentum_tiled_kernel(
     GridK g, const double *__restrict__ un, const double *__restrict__ vn,
     const double *__restrict__ wn, const double *__restrict__ pn, double *__restrict__ us,
@@ -239,7 +246,7 @@ __global__ __launch_bounds__(MTX * TY) void momentum_tiled_kernel(
     double pkm = active ? pn[d.g(i, j, k0 - 1)] : 0.0;
     // the per-cell operands of plane k0 (the next plane's are fetched while a plane is computed)
     MomOld m{};
-    if (active) m = mom_old<IBM>(oru, orv, orw, cu, cv, cw, d.in(i, j, k0), d.g(i, j, k0 * coef_kstride));
+    if (active) m = mom_old<IBM, NT>(oru, orv, orw, cu, cv, cw, d.in(i, j, k0), d.g(i, j, k0 * coef_kstride));
     const double hj = (FR && active) ? (g.ihc ? 1.0 / g.ihc[j] : g.dy) : 0.0;
     double fa = 0.0, fb = 0.0;
     __syncthreads();
@@ -249,7 +256,7 @@ __global__ __launch_bounds__(MTX * TY) void momentum_tiled_kernel(
         // values enter LDS after it
         double ru[PER], rv[PER], rw[PER], rp[PER];
         MomOld mn{};
-        if (active && k < k1) mn = mom_old<IBM>(oru, orv, orw, cu, cv, cw, d.in(i, j, k + 1), d.g(i, j, (k + 1) * coef_kstride));
+        if (active && k < k1) mn = mom_old<IBM, NT>(oru, orv, orw, cu, cv, cw, d.in(i, j, k + 1), d.g(i, j, (k + 1) * coef_kstride));
         if (k < k1) {
 #pragma unroll
             for (int c = 0; c < PER; ++c) {
@@ -268,7 +275,7 @@ __global__ __launch_bounds__(MTX * TY) void momentum_tiled_kernel(
         double pnext = 0.0;
         if (active) {
             const MomTile L{su, sv, sw, sp, {s0 * MPL, ((s0 + 1) % 3) * MPL, ((s0 + 2) % 3) * MPL}, t, pkm};
-            const double uw = momentum_cell<STRETCH, IBM>(g, L, i, j, k, d.g(i, j, k), d.in(i, j, k), m, us, vs, ws,
+            const double uw = momentum_cell<STRETCH, IBM, NT>(g, L, i, j, k, d.g(i, j, k), d.in(i, j, k), m, us, vs, ws,
                                                           oru, orv, orw, dta, dtb, dtg, idx, idy, idz, idx2, idy2,
                                                           idz2, ire);
             if (FR) {   // x is periodic (the launcher checks), so uw is the u* of every cell
@@ -352,14 +359,23 @@ hipError_t launch_momentum(mdx_handle *h, double dta, double dtb, double dtg, do
         }
         tiled = momentum_groups(h->d, ty, mkz) >= 256;
     }
+    // Where the 13 arrays a launch streams are well past the 256 MB of the last-level cache, the old
+    // right-hand sides, which the projection does not touch, only push out the predictor that it reads
+    // next: they go past the caches.  256 x 192 x 256 (1.3 GB): 339 -> 329 us, and the FFT's first launch
+    // after it 115 -> 102; 192 x 160 x 128 (409 MB): 96 -> 92, and a SOLA iteration after it 83 -> 62.
+    // Below, they are read back from the cache: 160 x 128 x 128 (273 MB) 54 us, 74 past it, 128^3 40 and 48.
+    const bool nt = 13.0 * 8.0 * (double)h->ni > 300e6;
     const int nseg = (h->d.nz + mkz - 1) / mkz;
     dim3 blk = tiled ? dim3(MTX, ty, 1) : dim3(BX, BY, 1);
     dim3 grd(tiled ? xcd_grid(h->d.nx, h->d.ny, nseg, MTX, ty) : xcd_grid(h->d.nx, h->d.ny, h->d.nz, BX, BY));
     // the partials come from the tiled kernel, over a periodic x (as constant flow rate requires)
     if (frpart && (!tiled || !h->cfg.periodic[0])) return hipErrorInvalidValue;
 #define MDX_MOM_(S, I, FR)                                                                                     \
-    hipLaunchKernelGGL((tiled ? (ty == 4 ? momentum_tiled_kernel<S, I, 4, FR> : momentum_tiled_kernel<S, I, 8, FR>) \
-                              : momentum_kernel<S, I>),                                                        \
+    hipLaunchKernelGGL((!tiled ? momentum_kernel<S, I>                                                              \
+                        : nt ? (ty == 4 ? momentum_tiled_kernel<S, I, 4, FR, true>                                  \
+                                        : momentum_tiled_kernel<S, I, 8, FR, true>)                                 \
+                             : (ty == 4 ? momentum_tiled_kernel<S, I, 4, FR, false>                                 \
+                                        : momentum_tiled_kernel<S, I, 8, FR, false>)),                              \
                        grd, blk, 0, h->stream,                                                               \
                        g, h->un, h->vn, h->wn,                                                   \
                        h->pn, h->us, h->vs, h->ws, h->oru, h->orv, h->orw, h->cu, h->cv, h->cw,  \

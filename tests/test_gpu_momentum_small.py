@@ -1,5 +1,5 @@
-"""Momentum on grids of few tiles: marches of one, two and four planes and the per-cell kernel give the
-oracle-checked tiled kernel's bits, with and without body and stretching, remainders in every
+"""Momentum on grids of few tiles (marches of one, two and four planes, the per-cell kernel) and past the
+last-level cache gives the bits of the oracle and of the long march, with and without body and stretching, remainders in every
 direction."""
 import numpy as np
 import pytest
@@ -9,8 +9,8 @@ from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
-# per cell; one plane (tile remainders; exactly 256 workgroups); two; four; the default march
-SHAPES = [(2, 2, 2), (32, 24, 16), (66, 35, 31), (64, 64, 16), (100, 70, 54), (128, 97, 64), (130, 129, 70)]
+# per cell; one plane (tile remainders; exactly 256 workgroups); two; four; the default march, past the cache
+SHAPES = [(2, 2, 2), (32, 24, 16), (66, 35, 31), (64, 64, 16), (100, 70, 54), (128, 97, 64), (130, 129, 70), (190, 130, 126)]
 
 
 @pytest.mark.parametrize("shape", SHAPES)

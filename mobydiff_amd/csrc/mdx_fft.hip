@@ -865,19 +865,23 @@ __global__ __launch_bounds__(64 * TW_WAVES) void tridiag_wave_kernel(int nlines,
 }
 
 // 3''. The same solves as a partitioned Thomas recurrence, for ny >= 64.  A workgroup of 256 threads
-//     stages 16 consecutive lines through LDS (as above) and gives each line 16 threads, one per
-//     segment of M consecutive rows (rows past ny are identity rows).  A segment's interior rows
-//     (1 .. M-2) are eliminated by the Thomas recurrence with three right-hand sides: the data, and
-//     the couplings to the segment's first row F (through a_1) and last row E (through c_(M-2)), so
-//     every interior value is p + q F + s E.  Substituted into the first and last rows, that leaves
-//     a tridiagonal system in F_0, E_0, F_1, E_1, ... (32 unknowns per line), which one thread per
-//     line solves by the Thomas recurrence; the segments then form their interior values.  The
-//     serial chain per line is 2 (M - 2) + 64 steps instead of 2 ny, the work about twice the plain
-//     recurrence's, and the data stay in LDS: the kernel moves the spectrum once each way.  The
-//     mean mode pins row 1 as the wave solve does; MEAN_ZERO zeroes that line.
-static constexpr int TP_LINES = 16, TP_SEGS = 16;
+//     takes 16 consecutive lines and gives each line 16 threads, one per segment of M consecutive
+//     rows, which stay in the thread's registers (rows past ny are identity rows; a row of the 16
+//     lines is 256 contiguous bytes, so loads and stores move whole cache lines without staging).
+//     A segment's interior rows (1 .. M-2) are eliminated by the Thomas recurrence with three
+//     right-hand sides: the data, and the couplings to the segment's first row F (through a_1) and
+//     last row E (through c_(M-2)), so every interior value is p + q F + s E.  Substituted into the
+//     first and last rows, that leaves a tridiagonal system in F_0, E_0, F_1, E_1, ... (32 unknowns
+//     per line), which one thread per line solves by the Thomas recurrence, TP_CH rows' operands
+//     read ahead of the chain; the segments then form their interior values.  The serial chain per
+//     line is 2 (M - 2) + 64 steps instead of 2 ny, the work about twice the plain recurrence's, and
+//     the spectrum moves once each way.  The mean mode pins row 1 as the wave solve does; MEAN_ZERO
+//     zeroes that line.  256 x 192 x 256 in FP64: 92 us with the lines staged in LDS (70 KB, two
+//     workgroups per CU) and the reduced system's operands read step by step; 57 now (FP32: 50 and
+//     31), 64^3 13.1 and 7.8.
+static constexpr int TP_LINES = 16, TP_SEGS = 16, TP_CH = 8;
 template <typename C, int M, bool MEAN_ZERO>
-__global__ __launch_bounds__(TP_LINES * TP_SEGS) void tridiag_part_kernel(int nlines, int stride, int nxh, int ny,
+__global__ __launch_bounds__(TP_LINES * TP_SEGS, M <= 12 ? 3 : 2) void tridiag_part_kernel(int nlines, int stride, int nxh, int ny,
                                                                         size_t plane, C *hat,
                                                                         const typename Cx<C>::R *__restrict__ lamx,
                                                                         const typename Cx<C>::R *__restrict__ lamz,
@@ -885,27 +889,28 @@ __global__ __launch_bounds__(TP_LINES * TP_SEGS) void tridiag_part_kernel(int nl
                                                                         const typename Cx<C>::R *__restrict__ bdrow,
                                                                         const typename Cx<C>::R *__restrict__ crow) {
     using R = typename Cx<C>::R;
+    static_assert(M >= 3, "a segment has interior rows");
     constexpr int NR = 2 * TP_SEGS;   // reduced rows per line
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    C *tile = reinterpret_cast<C *>(lds_raw);   // [TP_LINES][ny + 1]
-    __shared__ R ra[TP_LINES][NR], rb[TP_LINES][NR], rc[TP_LINES][NR];
-    __shared__ C rd[TP_LINES][NR];
-    const int ldt = ny + 1;
+    __shared__ R ra[NR][TP_LINES], rb[NR][TP_LINES], rc[NR][TP_LINES];
+    __shared__ C rd[NR][TP_LINES];
     const int tt = threadIdx.x % TP_LINES, sg = threadIdx.x / TP_LINES;
     const int t = blockIdx.x * TP_LINES + tt;
-    const C zero2 = Cx<C>::mk(R(0), R(0));
-    for (int j = sg; j < ny; j += TP_SEGS) tile[tt * ldt + j] = t < nlines ? hat[(size_t)t + plane * j] : zero2;
-    __syncthreads();
-    C *line = tile + (size_t)tt * ldt;
-    R k = R(0);
     const bool live = t < nlines && t % stride < nxh;   // a line, not the padding of a kx row
-    if (live) k = lamx[t % stride] + lamz[t / stride];
     const bool ident_line = !live || (MEAN_ZERO && t == 0);
     const int j0 = sg * M;
-    // row r of the segment: (a, b, c); the data row is line[j0 + r]
+    // row r of the segment: (a, b, c) and the data
+    auto solved = [&](int r) { return !ident_line && j0 + r < ny && !(t == 0 && j0 + r == 0); };
+    C p[M];
+    C *h = hat + (size_t)(t < nlines ? t : 0) + plane * j0;
+#pragma unroll
+    for (int r = 0; r < M; ++r) {
+        p[r] = Cx<C>::mk(R(0), R(0));
+        if (solved(r)) p[r] = h[plane * r];
+    }
+    const R k = live ? lamx[t % stride] + lamz[t / stride] : R(0);
     auto coef = [&](int r, R &a, R &b, R &c) {
         const int j = j0 + r;
-        if (!ident_line && j < ny && !(t == 0 && j == 0)) {
+        if (solved(r)) {
             a = arow[j];
             b = bdrow[j] - k;
             c = crow[j];
@@ -915,109 +920,90 @@ __global__ __launch_bounds__(TP_LINES * TP_SEGS) void tridiag_part_kernel(int nl
             c = R(0);
         }
     };
-    auto data = [&](int r) {
-        const int j = j0 + r;
-        return (!ident_line && j < ny && !(t == 0 && j == 0)) ? line[j] : zero2;
-    };
-    // ---- interior rows 1 .. M-2: forward elimination with the three right-hand sides; the data's
-    // eliminated values go back into LDS, the couplings' stay in registers
+    // ---- interior rows 1 .. M-2: forward elimination with the three right-hand sides
     R cp[M], qq[M], ss[M];
-#pragma unroll
-    for (int r = 0; r < M; ++r) cp[r] = qq[r] = ss[r] = R(0);
     R a0, b0, c0, aL, bL, cL;
     coef(0, a0, b0, c0);
     coef(M - 1, aL, bL, cL);
-    const C d0 = data(0), dL = data(M - 1);
-    C pprev = zero2;
 #pragma unroll
     for (int r = 1; r <= M - 2; ++r) {
         R a, b, c;
         coef(r, a, b, c);
-        const C d = data(r);
         const R den = r > 1 ? b - a * cp[r - 1] : b;
         const R rden = R(1) / den;
         cp[r] = r < M - 2 ? c * rden : R(0);
-        const C p = r > 1 ? Cx<C>::mk((d.x - a * pprev.x) * rden, (d.y - a * pprev.y) * rden)
-                          : Cx<C>::mk(d.x * rden, d.y * rden);
+        p[r] = r > 1 ? Cx<C>::mk((p[r].x - a * p[r - 1].x) * rden, (p[r].y - a * p[r - 1].y) * rden)
+                     : Cx<C>::mk(p[r].x * rden, p[r].y * rden);
         qq[r] = (r == 1 ? -a : -a * qq[r - 1]) * rden;
         ss[r] = ((r == M - 2 ? -c : R(0)) - (r > 1 ? a * ss[r - 1] : R(0))) * rden;
-        if (j0 + r < ny) line[j0 + r] = p;
-        pprev = p;
     }
     // back substitution of the three right-hand sides
-    C pnext = zero2;
 #pragma unroll
-    for (int r = M - 2; r >= 1; --r) {
-        C p = j0 + r < ny ? line[j0 + r] : zero2;
-        if (r < M - 2) {
-            p = Cx<C>::mk(p.x - cp[r] * pnext.x, p.y - cp[r] * pnext.y);
-            qq[r] -= cp[r] * qq[r + 1];
-            ss[r] -= cp[r] * ss[r + 1];
-        }
-        if (j0 + r < ny) line[j0 + r] = p;
-        pnext = p;
+    for (int r = M - 3; r >= 1; --r) {
+        p[r] = Cx<C>::mk(p[r].x - cp[r] * p[r + 1].x, p[r].y - cp[r] * p[r + 1].y);
+        qq[r] -= cp[r] * qq[r + 1];
+        ss[r] -= cp[r] * ss[r + 1];
     }
     // ---- the segment's two rows of the reduced system: F (row 0) and E (row M-1)
-    {
-        const C p1 = M > 2 ? (j0 + 1 < ny ? line[j0 + 1] : zero2) : zero2;
-        const C pl = M > 2 ? (j0 + M - 2 < ny ? line[j0 + M - 2] : zero2) : zero2;
-        if (M > 2) {
-            ra[tt][2 * sg] = a0;
-            rb[tt][2 * sg] = b0 + c0 * qq[1];
-            rc[tt][2 * sg] = c0 * ss[1];
-            rd[tt][2 * sg] = Cx<C>::mk(d0.x - c0 * p1.x, d0.y - c0 * p1.y);
-            ra[tt][2 * sg + 1] = aL * qq[M - 2];
-            rb[tt][2 * sg + 1] = bL + aL * ss[M - 2];
-            rc[tt][2 * sg + 1] = cL;
-            rd[tt][2 * sg + 1] = Cx<C>::mk(dL.x - aL * pl.x, dL.y - aL * pl.y);
-        } else {
-            ra[tt][2 * sg] = a0;
-            rb[tt][2 * sg] = b0;
-            rc[tt][2 * sg] = c0;
-            rd[tt][2 * sg] = d0;
-            ra[tt][2 * sg + 1] = aL;
-            rb[tt][2 * sg + 1] = bL;
-            rc[tt][2 * sg + 1] = cL;
-            rd[tt][2 * sg + 1] = dL;
-        }
-    }
+    ra[2 * sg][tt] = a0;
+    rb[2 * sg][tt] = b0 + c0 * qq[1];
+    rc[2 * sg][tt] = c0 * ss[1];
+    rd[2 * sg][tt] = Cx<C>::mk(p[0].x - c0 * p[1].x, p[0].y - c0 * p[1].y);
+    ra[2 * sg + 1][tt] = aL * qq[M - 2];
+    rb[2 * sg + 1][tt] = bL + aL * ss[M - 2];
+    rc[2 * sg + 1][tt] = cL;
+    rd[2 * sg + 1][tt] = Cx<C>::mk(p[M - 1].x - aL * p[M - 2].x, p[M - 1].y - aL * p[M - 2].y);
     __syncthreads();
     // ---- the reduced system of each line, one thread per line (Thomas; solution into rd)
     if (sg == 0) {
         R cprev = R(0);
-        C dprev = zero2;
-        for (int r = 0; r < NR; ++r) {
-            const R a = ra[tt][r], den = rb[tt][r] - a * cprev, rden = R(1) / den;
-            const C d = rd[tt][r];
-            cprev = rc[tt][r] * rden;
-            dprev = Cx<C>::mk((d.x - a * dprev.x) * rden, (d.y - a * dprev.y) * rden);
-            rc[tt][r] = cprev;
-            rd[tt][r] = dprev;
+        C dprev = Cx<C>::mk(R(0), R(0));
+        for (int r0 = 0; r0 < NR; r0 += TP_CH) {
+            R a[TP_CH], b[TP_CH], c[TP_CH];
+            C d[TP_CH];
+#pragma unroll
+            for (int u = 0; u < TP_CH; ++u) {
+                a[u] = ra[r0 + u][tt];
+                b[u] = rb[r0 + u][tt];
+                c[u] = rc[r0 + u][tt];
+                d[u] = rd[r0 + u][tt];
+            }
+#pragma unroll
+            for (int u = 0; u < TP_CH; ++u) {
+                const R den = b[u] - a[u] * cprev, rden = R(1) / den;
+                cprev = c[u] * rden;
+                dprev = Cx<C>::mk((d[u].x - a[u] * dprev.x) * rden, (d[u].y - a[u] * dprev.y) * rden);
+                rc[r0 + u][tt] = cprev;
+                rd[r0 + u][tt] = dprev;
+            }
         }
-        C xn = rd[tt][NR - 1];
-        for (int r = NR - 2; r >= 0; --r) {
-            const C d = rd[tt][r];
-            xn = Cx<C>::mk(d.x - rc[tt][r] * xn.x, d.y - rc[tt][r] * xn.y);
-            rd[tt][r] = xn;
+        C xn = dprev;
+        for (int r0 = NR - TP_CH; r0 >= 0; r0 -= TP_CH) {
+            R c[TP_CH];
+            C d[TP_CH];
+#pragma unroll
+            for (int u = 0; u < TP_CH; ++u) {
+                c[u] = rc[r0 + u][tt];
+                d[u] = rd[r0 + u][tt];
+            }
+#pragma unroll
+            for (int u = TP_CH - 1; u >= 0; --u) {
+                if (r0 + u == NR - 1) continue;
+                xn = Cx<C>::mk(d[u].x - c[u] * xn.x, d[u].y - c[u] * xn.y);
+                rd[r0 + u][tt] = xn;
+            }
         }
     }
     __syncthreads();
     // ---- every row of the segment from F and E
-    {
-        const C F = rd[tt][2 * sg], E = rd[tt][2 * sg + 1];
-        if (j0 < ny) line[j0] = F;
+    if (!live) return;
+    const C F = rd[2 * sg][tt], E = rd[2 * sg + 1][tt];
 #pragma unroll
-        for (int r = 1; r <= M - 2; ++r) {
-            if (j0 + r < ny) {
-                const C p = line[j0 + r];
-                line[j0 + r] = Cx<C>::mk(p.x + qq[r] * F.x + ss[r] * E.x, p.y + qq[r] * F.y + ss[r] * E.y);
-            }
-        }
-        if (j0 + M - 1 < ny) line[j0 + M - 1] = E;
+    for (int r = 0; r < M; ++r) {
+        if (j0 + r < ny)
+            h[plane * r] = r == 0 ? F : r == M - 1 ? E
+                           : Cx<C>::mk(p[r].x + qq[r] * F.x + ss[r] * E.x, p[r].y + qq[r] * F.y + ss[r] * E.y);
     }
-    __syncthreads();
-    if (live)
-        for (int j = sg; j < ny; j += TP_SEGS) hat[(size_t)t + plane * j] = tile[tt * ldt + j];
 }
 
 // launches the partitioned solve for 64 <= ny <= 256 (false: the caller takes another solver)
@@ -1029,14 +1015,9 @@ static bool launch_tridiag_part(hipStream_t st, const Dims &d, C *hat, const typ
     const int nxh = d.nx / 2 + 1, stride = fft_stride_t<C>(d.nx), nlines = stride * d.nz, m = (d.ny + TP_SEGS - 1) / TP_SEGS;
     const size_t plane = (size_t)nlines;
     const dim3 grid((nlines + TP_LINES - 1) / TP_LINES), blk(TP_LINES * TP_SEGS);
-    const size_t lds = (size_t)TP_LINES * (d.ny + 1) * sizeof(C);   // <= 66 KB
 #define TP_CASE(MM)                                                                                            \
     if (m <= MM) {                                                                                             \
-        static const hipError_t attr = hipFuncSetAttribute(                                                    \
-            reinterpret_cast<const void *>(&tridiag_part_kernel<C, MM, MEAN_ZERO>),                            \
-            hipFuncAttributeMaxDynamicSharedMemorySize, 16 * 257 * (int)sizeof(C));                            \
-        if (attr != hipSuccess) return false;                                                                  \
-        hipLaunchKernelGGL((tridiag_part_kernel<C, MM, MEAN_ZERO>), grid, blk, lds, st, nlines, stride, nxh, d.ny, plane, \
+        hipLaunchKernelGGL((tridiag_part_kernel<C, MM, MEAN_ZERO>), grid, blk, 0, st, nlines, stride, nxh, d.ny, plane, \
                            hat, lamx, lamz, a, bd, c);                                                         \
         return true;                                                                                           \
     }

@@ -864,7 +864,7 @@ __global__ __launch_bounds__(64 * TW_WAVES) void tridiag_wave_kernel(int nlines,
     }
 }
 
-// 3''. The same solves as a partitioned Thomas recurrence, for ny >= 64.  A workgroup of 256 threads
+// 3''. The same solves as a partitioned Thomas recurrence.  A workgroup of 256 threads
 //     takes 16 consecutive lines and gives each line 16 threads, one per segment of M consecutive
 //     rows, which stay in the thread's registers (rows past ny are identity rows; a row of the 16
 //     lines is 256 contiguous bytes, so loads and stores move whole cache lines without staging).
@@ -1006,12 +1006,15 @@ __global__ __launch_bounds__(TP_LINES * TP_SEGS, M <= 12 ? 3 : 2) void tridiag_p
     }
 }
 
-// launches the partitioned solve for 64 <= ny <= 256 (false: the caller takes another solver)
+// launches the partitioned solve for ny <= 256, in FP32 for ny >= 64 (false: the caller takes another
+// solver).  Below 64 rows a line's segments past ny idle, and still FP64 takes 7.4 us at 64 x 24 x 64
+// and 9.8 at 128 x 33 x 128 where a wave per line took 14.2 and 28.8; the FP32 passes of the defect
+// correction keep the wave's rounding there.
 template <typename C, bool MEAN_ZERO>
 static bool launch_tridiag_part(hipStream_t st, const Dims &d, C *hat, const typename Cx<C>::R *lamx,
                                 const typename Cx<C>::R *lamz, const typename Cx<C>::R *a,
                                 const typename Cx<C>::R *bd, const typename Cx<C>::R *c) {
-    if (d.ny < 64 || d.ny > 256) return false;
+    if ((sizeof(C) == 8 && d.ny < 64) || d.ny > 256) return false;
     const int nxh = d.nx / 2 + 1, stride = fft_stride_t<C>(d.nx), nlines = stride * d.nz, m = (d.ny + TP_SEGS - 1) / TP_SEGS;
     const size_t plane = (size_t)nlines;
     const dim3 grid((nlines + TP_LINES - 1) / TP_LINES), blk(TP_LINES * TP_SEGS);

@@ -874,10 +874,10 @@ static int rb_prepare(mdx_handle *h) {
     for (int **xl : {&h->rb_xl32, &h->rb_xl64})
         if (*xl) { (void)hipFree(*xl); *xl = nullptr; }
     MDX_HIP(hipMalloc(&h->rb_xl32, rb_xlist_bytes(p32)));
-    MDX_HIP(rb_build_xlists(h, p32, h->rb_xl32));
+    MDX_HIP(rb_build_xlists(h, p32, true, h->rb_xl32));
     if (h->lds_sor_mode == 2) {
         MDX_HIP(hipMalloc(&h->rb_xl64, rb_xlist_bytes(p64)));
-        MDX_HIP(rb_build_xlists(h, p64, h->rb_xl64));
+        MDX_HIP(rb_build_xlists(h, p64, false, h->rb_xl64));
     }
     h->rb_tag = 0;
     h->rb_plan64 = p64;

@@ -474,7 +474,7 @@ struct RbDefect {
 hipError_t launch_rb_lds(mdx_handle *h, bool fp32, int iters, int zero_init, const RbDefect *df = nullptr);
 size_t rb_faces_bytes(const RbPlanOut &p, bool fp32);
 size_t rb_xlist_bytes(const RbPlanOut &p);
-hipError_t rb_build_xlists(mdx_handle *h, const RbPlanOut &p, int *xl);
+hipError_t rb_build_xlists(mdx_handle *h, const RbPlanOut &p, bool fp32, int *xl);
 
 // FFT path
 int fft_stride(int nx, bool fp32);   // complex elements per kx row of the spectrum

@@ -9,6 +9,7 @@
 //   4. inverse z-FFT                                                         hat -> hat
 //   5. inverse real x-FFT with the 1/(nx nz) scaling per row                 hat -> phi
 //   6. projection u = (u* - dtg grad phi)/(1 + dtg coef), p += phi
+// (2. to 4. are one launch on small grids, column_solve_kernel).
 // Transforms of 16 to 1024 points hold 16 points per thread in registers (fft_line: one LDS
 // exchange for 32 to 256 points, two above); shorter ones are radix-4 Stockham (self-sorting) in
 // LDS.  hat keeps the reference's half-spectrum layout plane_hat(nxh, nz, ny), kx fastest, each kx
@@ -251,7 +252,8 @@ __device__ inline void rf_split(const C *line, int m, C &a, C &b) {
 }
 // rows 2 P and 2 P + 1 of the thread's line from its transform e to hat; every thread of the
 // workgroup calls it (barriers)
-template <typename C, int N, int TH, int W = 1>
+// (TR: into the transposed spectrum of the column solves, kx slowest, `stride` values to a kx)
+template <typename C, int N, int TH, int W = 1, bool TR = false>
 __device__ inline void rf_store_rows(C (&e)[16], int t, C *lds, int l, int P0, int npairs, int stride, C *hat) {
     using F = RFft<N, TH>;
     C *line = lds + (size_t)l * F::LS;
@@ -263,12 +265,20 @@ __device__ inline void rf_store_rows(C (&e)[16], int t, C *lds, int l, int P0, i
     __syncthreads();
     constexpr int H = N / 2 + 1;
     for (int q = threadIdx.x; q < F::LPW * H; q += TH * W) {
-        const int ll = q / H, m = q - ll * H, P = P0 + ll;
-        if (P >= npairs) break;
+        const int ll = TR ? q % F::LPW : q / H, m = TR ? q / F::LPW : q - ll * H, P = P0 + ll;
+        if (P >= npairs) {
+            if (TR) continue;
+            break;
+        }
         C a, b;
         rf_split<C, N>(lds + (size_t)ll * F::LS, m, a, b);
-        hat[(size_t)stride * (2 * P) + m] = a;
-        hat[(size_t)stride * (2 * P + 1) + m] = b;
+        if (TR) {
+            hat[(size_t)stride * m + 2 * P] = a;
+            hat[(size_t)stride * m + 2 * P + 1] = b;
+        } else {
+            hat[(size_t)stride * (2 * P) + m] = a;
+            hat[(size_t)stride * (2 * P + 1) + m] = b;
+        }
     }
 }
 // the thread's points of the inverse line of rows 2 P and 2 P + 1, from their half spectra (the real
@@ -336,7 +346,7 @@ __device__ inline void flow_sum_tile(const GridK &g, const double *__restrict__ 
     }
     flow_tile_sum<4>(fa, fb, threadIdx.x, s, f.part, (size_t)wg);
 }
-template <int N, int TH, int W, bool STRETCH>
+template <int N, int TH, int W, bool STRETCH, bool TR>
 __global__ __launch_bounds__(TH * W) void rhs_xfft_reg_kernel(GridK g, const double *__restrict__ us,
                                                               const double *__restrict__ vs,
                                                               const double *__restrict__ ws, double dtg, int wrap,
@@ -387,7 +397,7 @@ __global__ __launch_bounds__(TH * W) void rhs_xfft_reg_kernel(GridK g, const dou
     if (on) rf_gather<double2, N>(e, t, line);
     if constexpr (!F::TW0) __syncthreads();   // the lines are read before they are written again
     fft_line<double2, N, false>(e, t, twl, line, on);
-    rf_store_rows<double2, N, TH, W>(e, t, lds, l, P0, npairs, stride, hat);
+    rf_store_rows<double2, N, TH, W, TR>(e, t, lds, l, P0, npairs, stride, hat);
 }
 
 // 1. (FP32) forward x-transform of a real FP64 field in (nx, nz, ny) layout, a row per line (two rows
@@ -433,6 +443,54 @@ __global__ __launch_bounds__(TH) void ixfft_reg_kernel(Dims d, const double2 *__
     for (int s = 0; s < 16; ++s) {
         p[F::M * s] = e[s].x * scale;
         p[N + F::M * s] = e[s].y * scale;
+    }
+}
+// The same from the transposed spectrum (column_solve_kernel) for its small grids: 64 threads hold the
+// lines, and 256 load them (neighbouring lanes on neighbouring lines, 32 bytes each) and store phi's
+// rows, through LDS.  64^3: 4.0 us above, 5.2 here (6.6 with the 64 threads alone).
+template <int N, int TH, int W>
+__global__ __launch_bounds__(TH * W) void ixfft_columns_kernel(Dims d, const double2 *__restrict__ hat,
+                                                               const double2 *__restrict__ tw, int stride,
+                                                               double scale, double *__restrict__ phi) {
+    using F = RFft<N, TH>;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    double2 *lds = reinterpret_cast<double2 *>(lds_raw), *twl = lds + F::LPW * F::LS;
+    const int npairs = d.ny * d.nz / 2, t = threadIdx.x % F::M, l = threadIdx.x / F::M, P0 = blockIdx.x * F::LPW;
+    rf_stage<double2, N, TH, W>(twl, tw);
+    for (int q = threadIdx.x; q < F::LPW * (N / 2 + 1); q += TH * W) {
+        const int ll = q % F::LPW, m = q / F::LPW;
+        double2 *line = lds + ll * F::LS;
+        double2 a = make_double2(0.0, 0.0), b = a;
+        if (P0 + ll < npairs) {
+            const double2 *h = hat + (size_t)stride * m + 2 * (P0 + ll);
+            a = h[0];
+            b = h[1];
+        }
+        if (m == 0 || 2 * m == N) {   // real
+            line[rf_pad(m)] = make_double2(a.x, b.x);
+        } else {
+            line[rf_pad(m)] = make_double2(a.x - b.y, a.y + b.x);
+            line[rf_pad(N - m)] = make_double2(a.x + b.y, b.x - a.y);
+        }
+    }
+    __syncthreads();
+    const bool on = l < F::LPW;
+    double2 *line = lds + (on ? l : 0) * F::LS;
+    double2 e[16];
+    if (on) rf_gather<double2, N>(e, t, line);
+    if constexpr (!F::TW0) __syncthreads();   // the lines are read before they are written again
+    fft_line<double2, N, true>(e, t, twl, line, on);
+    __syncthreads();
+    if (on) {
+#pragma unroll
+        for (int s = 0; s < 16; ++s) line[rf_pad(t + F::M * s)] = e[s];
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < 2 * F::LPW * N; q += TH * W) {
+        const int r = q / N, x = q % N;
+        if (2 * P0 + r >= 2 * npairs) break;
+        const double2 v = lds[r / 2 * F::LS + rf_pad(x)];
+        phi[(size_t)N * (2 * P0 + r) + x] = (r % 2 ? v.y : v.x) * scale;
     }
 }
 // 5. (FP32) inverse x-transform of each row, scaled, and the mean mode's solution added to the FP64 phi
@@ -1006,6 +1064,149 @@ __global__ __launch_bounds__(TP_LINES * TP_SEGS, M <= 12 ? 3 : 2) void tridiag_p
     }
 }
 
+// 2. - 4. in one launch, where a kx column of the spectrum (all planes and kz, transposed: kx slowest)
+//     fits a CU's LDS and the launches are short: z-transforms of the column's lines, its tridiagonal
+//     solves as tridiag_part_kernel does them (CS_SEGS segments of M rows; the reduced rows' data in the
+//     tile, at the rows they stand for), and the transforms back, one workgroup per kx.  Bound by
+//     latency: 64^3 18.2 us in three launches, 13.4 in one; 128 x 97 x 64 26.2 and 18.0.
+static constexpr int CS_T = 512, CS_SEGS = 8;
+template <int N, int M> constexpr size_t column_lds() {
+    return (size_t)CS_SEGS * M * RFft<N, CS_T>::LS * 16 + RFft<N, CS_T>::TW * 16 + 3 * 2 * CS_SEGS * (N < 64 ? N : 64) * 8;
+}
+template <int N, int M>
+__global__ __launch_bounds__(CS_T) void column_solve_kernel(int ny, const double2 *__restrict__ tw,
+                                                            const double *__restrict__ lamx,
+                                                            const double *__restrict__ lamz,
+                                                            const double *__restrict__ arow,
+                                                            const double *__restrict__ bdrow,
+                                                            const double *__restrict__ crow, double2 *__restrict__ hat) {
+    using F = RFft<N, CS_T>;
+    using C2 = Cx<double2>;
+    constexpr int NK = N < 64 ? N : 64, NR = 2 * CS_SEGS;   // kz at a time, reduced rows
+    static_assert(M >= 3 && NK * CS_SEGS <= CS_T, "a thread per segment");
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    double2 *tile = reinterpret_cast<double2 *>(lds_raw), *twl = tile + CS_SEGS * M * F::LS;
+    double *ra = reinterpret_cast<double *>(twl + F::TW), *rb = ra + NR * NK, *rc = rb + NR * NK;
+    const int kx = blockIdx.x, t = threadIdx.x % F::M, l = threadIdx.x / F::M;
+    double2 *col = hat + (size_t)kx * ny * N;
+    rf_stage<double2, N, CS_T>(twl, tw);
+    if constexpr (!F::TW0) __syncthreads();
+    double2 e[16];
+    for (int j0 = 0; j0 < ny; j0 += F::LPW) {
+        const int j = j0 + l;
+        const bool on = j < ny;
+        double2 *line = tile + (on ? j : 0) * F::LS;
+        if (on) {
+#pragma unroll
+            for (int s = 0; s < 16; ++s) e[s] = col[(size_t)j * N + t + F::M * s];
+        }
+        fft_line<double2, N, false>(e, t, twl, line, on);
+        __syncthreads();
+        if (on) {
+#pragma unroll
+            for (int s = 0; s < 16; ++s) line[rf_pad(t + F::M * s)] = e[s];
+        }
+    }
+    const int tk = threadIdx.x % NK, sg = threadIdx.x / NK, r0 = sg * M;
+    for (int k0 = 0; k0 < N; k0 += NK) {
+        const int kz = k0 + tk;
+        const bool mine = sg < CS_SEGS;
+        double2 *c = tile + rf_pad(kz);
+        const double k = lamx[kx] + lamz[kz];
+        auto solved = [&](int r) { return r0 + r < ny && !(kx == 0 && kz == 0 && r0 + r == 0); };
+        auto coef = [&](int r, double &a, double &b, double &cc) {
+            a = cc = 0.0;
+            b = 1.0;
+            if (solved(r)) {
+                a = arow[r0 + r];
+                b = bdrow[r0 + r] - k;
+                cc = crow[r0 + r];
+            }
+        };
+        double2 p[M];
+        double cp[M], qq[M], ss[M];
+        __syncthreads();
+        if (mine) {
+#pragma unroll
+            for (int r = 0; r < M; ++r) {
+                p[r] = make_double2(0.0, 0.0);
+                if (solved(r)) p[r] = c[(r0 + r) * F::LS];
+            }
+            double a0, b0, c0, aL, bL, cL;
+            coef(0, a0, b0, c0);
+            coef(M - 1, aL, bL, cL);
+#pragma unroll
+            for (int r = 1; r <= M - 2; ++r) {
+                double a, b, cc;
+                coef(r, a, b, cc);
+                const double rden = 1.0 / (r > 1 ? b - a * cp[r - 1] : b);
+                cp[r] = r < M - 2 ? cc * rden : 0.0;
+                p[r] = r > 1 ? C2::mk((p[r].x - a * p[r - 1].x) * rden, (p[r].y - a * p[r - 1].y) * rden)
+                             : C2::mk(p[r].x * rden, p[r].y * rden);
+                qq[r] = (r == 1 ? -a : -a * qq[r - 1]) * rden;
+                ss[r] = ((r == M - 2 ? -cc : 0.0) - (r > 1 ? a * ss[r - 1] : 0.0)) * rden;
+            }
+#pragma unroll
+            for (int r = M - 3; r >= 1; --r) {
+                p[r] = C2::mk(p[r].x - cp[r] * p[r + 1].x, p[r].y - cp[r] * p[r + 1].y);
+                qq[r] -= cp[r] * qq[r + 1];
+                ss[r] -= cp[r] * ss[r + 1];
+            }
+            // the reduced rows F (row 0) and E (row M-1); their data in the tile, at those rows
+            ra[2 * sg * NK + tk] = a0;
+            rb[2 * sg * NK + tk] = b0 + c0 * qq[1];
+            rc[2 * sg * NK + tk] = c0 * ss[1];
+            c[r0 * F::LS] = C2::mk(p[0].x - c0 * p[1].x, p[0].y - c0 * p[1].y);
+            ra[(2 * sg + 1) * NK + tk] = aL * qq[M - 2];
+            rb[(2 * sg + 1) * NK + tk] = bL + aL * ss[M - 2];
+            rc[(2 * sg + 1) * NK + tk] = cL;
+            c[(r0 + M - 1) * F::LS] = C2::mk(p[M - 1].x - aL * p[M - 2].x, p[M - 1].y - aL * p[M - 2].y);
+        }
+        __syncthreads();
+        if (sg == 0) {
+            auto row = [&](int r) -> double2 & { return c[(r / 2 * M + (r % 2 ? M - 1 : 0)) * F::LS]; };
+            double cs[NR], cprev = 0.0;
+            double2 ds[NR], dprev = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int r = 0; r < NR; ++r) ds[r] = row(r);
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const double a = ra[r * NK + tk], rden = 1.0 / (rb[r * NK + tk] - a * cprev);
+                cs[r] = cprev = rc[r * NK + tk] * rden;
+                ds[r] = dprev = C2::mk((ds[r].x - a * dprev.x) * rden, (ds[r].y - a * dprev.y) * rden);
+            }
+            row(NR - 1) = dprev;
+#pragma unroll
+            for (int r = NR - 2; r >= 0; --r) {
+                dprev = C2::mk(ds[r].x - cs[r] * dprev.x, ds[r].y - cs[r] * dprev.y);
+                row(r) = dprev;
+            }
+        }
+        __syncthreads();
+        if (mine) {
+            const double2 f = c[r0 * F::LS], g = c[(r0 + M - 1) * F::LS];
+#pragma unroll
+            for (int r = 1; r <= M - 2; ++r)
+                if (r0 + r < ny)
+                    c[(r0 + r) * F::LS] = C2::mk(p[r].x + qq[r] * f.x + ss[r] * g.x, p[r].y + qq[r] * f.y + ss[r] * g.y);
+        }
+    }
+    __syncthreads();
+    for (int j0 = 0; j0 < ny; j0 += F::LPW) {
+        const int j = j0 + l;
+        const bool on = j < ny;
+        double2 *line = tile + (on ? j : 0) * F::LS;
+        if (on) rf_gather<double2, N>(e, t, line);
+        if constexpr (!F::TW0) __syncthreads();
+        fft_line<double2, N, true>(e, t, twl, line, on);
+        if (on) {
+#pragma unroll
+            for (int s = 0; s < 16; ++s) col[(size_t)j * N + t + F::M * s] = e[s];
+        }
+        __syncthreads();
+    }
+}
+
 // launches the partitioned solve for ny <= 256, in FP32 for ny >= 64 (false: the caller takes another
 // solver).  Below 64 rows a line's segments past ny idle, and still FP64 takes 7.4 us at 64 x 24 x 64
 // and 9.8 at 128 x 33 x 128 where a wave per line took 14.2 and 28.8; the FP32 passes of the defect
@@ -1375,7 +1576,7 @@ static hipError_t launch_zfft(hipStream_t st, const Dims &d, C *hat, const C *tw
     return hipGetLastError();
 }
 
-static hipError_t launch_rhs_xfft(mdx_handle *h, double dtg) {
+template <bool TRK> static hipError_t launch_rhs_xfft(mdx_handle *h, double dtg) {
     GridK g = grid_k(h);
     const Dims d = h->d;
     const int stride = fft_stride_t<double2>(d.nx);
@@ -1383,9 +1584,10 @@ static hipError_t launch_rhs_xfft(mdx_handle *h, double dtg) {
     do {                                                                                                              \
         const unsigned nb = rf_row_blocks<N, TH>(d);                                                                  \
         const FlowSum fsum{(int)nb, h->mom_kz, h->fr_part};                                                           \
-        return rf_launch<double2, N, TH, rhs_xfft_reg_kernel<N, TH, W, S>, W>(                                        \
+        return rf_launch<double2, N, TH, rhs_xfft_reg_kernel<N, TH, W, S, W == 4 && TRK>, W>(                         \
             h->stream, nb + (h->step_sum ? momentum_tiles(h) : 0), g, (const double *)h->us, (const double *)h->vs,   \
-            (const double *)h->ws, dtg, fft_wrap(h), fsum, (const double2 *)h->tw_x, stride, (double2 *)h->hat);      \
+            (const double *)h->ws, dtg, fft_wrap(h), fsum, (const double2 *)h->tw_x, TRK ? d.ny * d.nz : stride,       \
+            (double2 *)h->hat);                                                                                       \
     } while (0)
 #define XF(N)                                                  \
     if (rf_small(rf_row_blocks<N, 256>(d))) {                  \
@@ -1416,10 +1618,9 @@ static hipError_t launch_ixfft(mdx_handle *h, double *phi) {
     const int stride = fft_stride_t<double2>(d.nx);
     const double scale = 1.0 / (double)(d.nx * d.nz);
 #define IX_(N, TH)                                                                                                  \
-    return rf_launch<double2, N, TH, ixfft_reg_kernel<N, TH>>(h->stream, rf_row_blocks<N, TH>(d), d, \
-                                                                              (const double2 *)h->hat,              \
-                                                                              (const double2 *)h->tw_x, stride,    \
-                                                                              scale, phi)
+    return rf_launch<double2, N, TH, ixfft_reg_kernel<N, TH>>(h->stream, rf_row_blocks<N, TH>(d), d,                 \
+                                                              (const double2 *)h->hat, (const double2 *)h->tw_x,    \
+                                                              stride, scale, phi)
 #define IX(N)                                                \
     if (rf_small(rf_row_blocks<N, 256>(d))) IX_(N, 64);      \
     IX_(N, 256)
@@ -1434,13 +1635,91 @@ static hipError_t launch_ixfft(mdx_handle *h, double *phi) {
     return hipGetLastError();
 }
 
+// the LDS a column may take
+static constexpr size_t COLUMN_LDS = 160 * 1024 - 1024;
+// Whether (2.) to (4.) go column by column in one launch: FP64 grids whose x-transforms take the
+// small workgroups, with a kx column in LDS.  A step against the three launches: 149 and 163 us at
+// 64^3, 227 and 250 at 128 x 97 x 64, 224 and 264 at 256 x 60 x 64, 110 and 129 at 32 x 24 x 32, 154 and
+// 160 at 16 x 96 x 64 (nine columns).
+template <int N, int M> static hipError_t column_solve(mdx_handle *h) {
+    const Dims d = h->d;
+    constexpr size_t lds = column_lds<N, M>();
+    const hipError_t e = rf_allow<column_solve_kernel<N, M>>(lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((column_solve_kernel<N, M>), dim3(d.nx / 2 + 1), dim3(CS_T), lds, h->stream, d.ny,
+                       (const double2 *)h->tw_z, h->lamx, h->lamz, h->tw_a, h->bdrow, h->crow, (double2 *)h->hat);
+    return hipGetLastError();
+}
+#define CS_ROWS(N, CALL)                                  \
+    do {                                                  \
+        const int m = (d.ny + CS_SEGS - 1) / CS_SEGS;     \
+        if (m <= 4) CALL(N, 4);                           \
+        if (m <= 8) CALL(N, 8);                           \
+        if (m <= 12) CALL(N, 12);                         \
+        if (m <= 13) CALL(N, 13);                         \
+        if (m <= 16) CALL(N, 16);                         \
+    } while (0)
+static bool columns_fit(const mdx_handle *h) {
+    const Dims d = h->d;
+    if (!h->wave_tridiag || !h->part_tridiag || d.nx < 16 || d.nx > 256) return false;
+    bool small = false;
+#define CALL(N) { small = rf_small(rf_row_blocks<N, 256>(d)); break; }
+    switch (d.nx) {
+    case 16: CALL(16)
+    case 32: CALL(32)
+    case 64: CALL(64)
+    case 128: CALL(128)
+    default: CALL(256)
+    }
+#undef CALL
+    if (!small) return false;
+#define CALL(N, M) return column_lds<N, M>() <= COLUMN_LDS
+    switch (d.nz) {
+    case 32: CS_ROWS(32, CALL); break;
+    case 64: CS_ROWS(64, CALL); break;
+    case 128: CS_ROWS(128, CALL); break;
+    default: break;
+    }
+#undef CALL
+    return false;
+}
+static hipError_t launch_columns(mdx_handle *h) {
+    const Dims d = h->d;
+#define CALL(N, M)                                                                       \
+    if constexpr (column_lds<N, M>() <= COLUMN_LDS) return column_solve<N, M>(h); \
+    else return hipErrorInvalidValue
+    switch (d.nz) {
+    case 32: CS_ROWS(32, CALL); break;
+    case 64: CS_ROWS(64, CALL); break;
+    case 128: CS_ROWS(128, CALL); break;
+    default: break;
+    }
+#undef CALL
+    return hipErrorInvalidValue;
+}
+
+static hipError_t launch_ixfft_columns(mdx_handle *h, double *phi) {
+    const Dims d = h->d;
+    const double scale = 1.0 / (double)(d.nx * d.nz);
+#define IX(N)                                                                                                       \
+    return rf_launch<double2, N, 64, ixfft_columns_kernel<N, 64, 4>, 4>(h->stream, rf_row_blocks<N, 64>(d), d,      \
+                                                                        (const double2 *)h->hat,                    \
+                                                                        (const double2 *)h->tw_x, d.ny * d.nz,      \
+                                                                        scale, phi)
+    RF_SIZES(d.nx, IX)
+#undef IX
+    return hipErrorInvalidValue;
+}
+
 hipError_t launch_fft_forward(mdx_handle *h, double dtg) {
-    const hipError_t e = launch_rhs_xfft(h, dtg);
+    if (columns_fit(h)) return launch_rhs_xfft<true>(h, dtg);
+    const hipError_t e = launch_rhs_xfft<false>(h, dtg);
     return e != hipSuccess ? e
                            : launch_zfft<double2, false>(h->stream, h->d, (double2 *)h->hat, (const double2 *)h->tw_z);
 }
 
 hipError_t launch_tridiag(mdx_handle *h) {
+    if (columns_fit(h)) return launch_columns(h);   // with both z-transforms
     const Dims d = h->d;
     const int nlines = (d.nx / 2 + 1) * d.nz;
     if (h->wave_tridiag && h->part_tridiag &&
@@ -1456,11 +1735,14 @@ hipError_t launch_tridiag(mdx_handle *h) {
 }
 
 hipError_t launch_fft_backward_correct(mdx_handle *h, double dtg) {
-    const Dims d = h->d;
-    hipError_t e = launch_zfft<double2, true>(h->stream, d, (double2 *)h->hat, (const double2 *)h->tw_z);
-    if (e != hipSuccess) return e;
-    if ((e = launch_ixfft(h, h->fft_rhs)) != hipSuccess) return e;
-    return launch_correct(h, h->fft_rhs, dtg, nullptr);
+    hipError_t e;
+    if (columns_fit(h)) {
+        e = launch_ixfft_columns(h, h->fft_rhs);
+    } else {
+        e = launch_zfft<double2, true>(h->stream, h->d, (double2 *)h->hat, (const double2 *)h->tw_z);
+        if (e == hipSuccess) e = launch_ixfft(h, h->fft_rhs);
+    }
+    return e != hipSuccess ? e : launch_correct(h, h->fft_rhs, dtg, nullptr);
 }
 
 // ------------------------------------------------------------------------------- mixed precision

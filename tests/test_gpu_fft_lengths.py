@@ -1,7 +1,7 @@
 """The FFT projection at every transform length: 16 to 1024 points in x and in z (the register
 transforms: one pass, two passes with each first radix, three passes), 2 to 8 (the LDS kernels),
 numbers of rows and of spectrum columns that leave workgroups partly empty, both workgroup sizes, ny at
-the edges of the tridiagonal solves' segments,
+the edges of the tridiagonal solves' segments and of the column solves,
 against the oracle's FFT projection (bound as for the other FFT tests: 1e-12 of each field), and the FP32 transforms
 inside the defect correction against the FP64 solve."""
 import numpy as np
@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [(n, 5, 16) for n in (16, 32, 64, 128, 256, 512, 1024)] + [(16, 3, n) for n in (32, 64, 128, 256, 512, 1024)] \
     + [(2, 4, 32), (32, 4, 2), (8, 7, 64), (64, 70, 4), (128, 33, 32), (32, 17, 128)] \
-    + [(32, ny, 16) for ny in (2, 63, 64, 65, 128, 129, 192, 193, 256, 257)]
+    + [(32, ny, 16) for ny in (2, 63, 64, 65, 128, 129, 192, 193, 256, 257)] \
+    + [(32, ny, 64) for ny in (2, 32, 33, 64, 65, 96, 97, 104, 105)] + [(16, 32, 128), (16, 33, 128), (64, 128, 32), (64, 129, 32)]
 # enough lines for workgroups of 256 threads (the ones above take 64)
 LARGE = [(256, 65, 256), (64, 257, 256), (1024, 65, 64)]
 

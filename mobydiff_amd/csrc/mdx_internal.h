@@ -314,6 +314,7 @@ struct mdx_handle {
     // z-planes each workgroup of the tiled momentum kernel marches (momentum_default_planes, 8 or
     // 12; MOBYDIFF_MOM_KZ)
     int mom_kz = 8;
+    bool mom_fixed = false;   // MOBYDIFF_MOM_KZ: on every grid
     int rb_state = 0;              // 0 not planned, 1 ready, -1 unavailable
     // polls of a neighbour wait before it gives up (MOBYDIFF_LDS_SPIN_LIMIT; a test hook); a wait
     // that gives up sets the error word, the batch drains, and the solve restarts on the

@@ -337,7 +337,7 @@ int momentum_tiles(const mdx_handle *h) { return (int)momentum_groups(h->d, mome
 static constexpr long MOM_FULL = 768;   // workgroups from which the long march wins (launch_momentum)
 // (64^3 with sums, in a step: 22.6 us; without 12.0, and the sums ride in the FFT's first launch)
 bool momentum_sums_apart(const mdx_handle *h) {
-    return h->tiled_momentum && momentum_rows(h) == 4 && momentum_tiles(h) < MOM_FULL;
+    return h->tiled_momentum && !h->mom_fixed && momentum_rows(h) == 4 && momentum_tiles(h) < MOM_FULL;
 }
 
 hipError_t launch_momentum(mdx_handle *h, double dta, double dtb, double dtg, double *frpart) {
@@ -346,7 +346,7 @@ hipError_t launch_momentum(mdx_handle *h, double dta, double dtb, double dtg, do
     const double dx2 = dx * dx, dy2 = dy * dy, dz2 = dz * dz;
     int mkz = h->mom_kz, ty = momentum_rows(h);
     bool tiled = h->tiled_momentum;
-    if (tiled && !frpart) {
+    if (tiled && !frpart && !h->mom_fixed) {
         // Without the sums, which follow the tiling, a workgroup marches fewer planes where that many
         // give every CU less than three of them, and the smallest grids go a thread per cell (a march
         // is a chain of loads and barriers; hot caches, 8 planes against these): 14.9 -> 4.0 us at

@@ -1828,8 +1828,9 @@ extern "C" int mdx_step(mdx_handle *h, double dt, mdx_step_stats *stats) {
         if (h->cfg.flowrate && h->fr_part) {
             // momentum forms the flow-rate partial sums of u*; one launch folds them, shifts u* and
             // builds the stage's face-coefficient tables if the solve needs new ones (with the FFT
-            // and no body the shift is uniform, and the projection's last pass makes it)
-            const bool late = h->cfg.solver == MDX_SOLVER_FFT && !h->ibm_on;
+            // and no body the shift is uniform, and the projection's last pass makes it, before the
+            // predictor's fill: a separate fill needs it shifted)
+            const bool late = h->cfg.solver == MDX_SOLVER_FFT && !h->ibm_on && h->fused_bc;
             h->step_sum = late && fft_sums(h);
             MDX_HIP(launch_momentum(h, dta, dtb, dtg, h->step_sum ? nullptr : h->fr_part));
             ev_record(h, 5);

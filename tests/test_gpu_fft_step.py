@@ -19,6 +19,21 @@ NAMES = ("un", "vn", "wn", "pn", "us", "vs", "ws", "oru", "orv", "orw")
 @pytest.mark.parametrize("flow,body,beta,prec", [(True, False, 1.5, "fp64"), (False, False, None, "fp64"),
                                                  (True, True, None, "fp64"), (True, False, None, "mixed")])
 def test_step_equals_the_calls(shape, flow, body, beta, prec):
+    _compare(shape, flow, body, beta, prec)
+
+
+# the routes that the switches leave: separate fills, sums and shift, other marches, other solves
+@pytest.mark.parametrize("env", ["FUSED_BC=0", "FUSED_FLOWRATE=0", "MOMENTUM_DIRECT=1", "MOM_KZ=4", "PART_TRIDIAG=0",
+                                 "WAVE_TRIDIAG=0"])
+@pytest.mark.parametrize("shape", [(2, 2, 2), (32, 66, 8), (64, 20, 32)])
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_switches(env, shape, prec, monkeypatch):
+    name, value = env.split("=")
+    monkeypatch.setenv("MOBYDIFF_" + name, value)
+    _compare(shape, True, False, 1.5, prec)
+
+
+def _compare(shape, flow, body, beta, prec):
     print(shape, flow, body, beta, prec, flush=True)
     rng = np.random.default_rng(5)
     g = O.Grid(*shape, lx=2.0, ly=2.0, lz=1.0, periodic=(1, 0, 1), beta=beta)

@@ -14,6 +14,8 @@
 // exchange for 32 to 256 points, two above); shorter ones are radix-4 Stockham (self-sorting) in
 // LDS.  hat keeps the reference's half-spectrum layout plane_hat(nxh, nz, ny), kx fastest, each kx
 // row padded to whole 128-byte lines (fft_stride).
+#include <type_traits>
+
 #include "mdx_internal.h"
 
 namespace mdx {
@@ -922,23 +924,107 @@ __global__ __launch_bounds__(64 * TW_WAVES) void tridiag_wave_kernel(int nlines,
     }
 }
 
-// 3''. The same solves as a partitioned Thomas recurrence.  A workgroup of 256 threads
-//     takes 16 consecutive lines and gives each line 16 threads, one per segment of M consecutive
-//     rows, which stay in the thread's registers (rows past ny are identity rows; a row of the 16
-//     lines is 256 contiguous bytes, so loads and stores move whole cache lines without staging).
-//     A segment's interior rows (1 .. M-2) are eliminated by the Thomas recurrence with three
-//     right-hand sides: the data, and the couplings to the segment's first row F (through a_1) and
-//     last row E (through c_(M-2)), so every interior value is p + q F + s E.  Substituted into the
-//     first and last rows, that leaves a tridiagonal system in F_0, E_0, F_1, E_1, ... (32 unknowns
-//     per line), which one thread per line solves by the Thomas recurrence, TP_CH rows' operands
-//     read ahead of the chain; the segments then form their interior values.  The serial chain per
+// The partitioned Thomas recurrence: a line's rows are cut into segments of M consecutive rows, a
+// thread each, whose rows stay in its registers (rows past ny are identity rows).  A segment's
+// interior rows (1 .. M-2) are eliminated by the Thomas recurrence with three right-hand sides: the
+// data, and the couplings to the segment's first row F (through a_1) and last row E (through
+// c_(M-2)), so every interior value is p + q F + s E.  Substituted into the first and last rows,
+// that leaves a tridiagonal system in F_0, E_0, F_1, E_1, ... of two rows per segment.
+// KEEP: what the elimination of another right-hand side needs stays too.
+template <typename C, int M, bool KEEP> struct TriSegment {
+    using R = typename Cx<C>::R;
+    static_assert(M >= 3, "a segment has interior rows");
+    R cp[M], qq[M], ss[M], rd[KEEP ? M : 1];
+    R a0, b0, c0, aL, bL, cL;
+    // coef(r, a, b, c): row r of the segment; p: the data
+    template <typename F> __device__ inline void eliminate(const F &coef, C (&p)[M]) {
+        coef(0, a0, b0, c0);
+        coef(M - 1, aL, bL, cL);
+#pragma unroll
+        for (int r = 1; r <= M - 2; ++r) {
+            R a, b, c;
+            coef(r, a, b, c);
+            const R rden = R(1) / (r > 1 ? b - a * cp[r - 1] : b);
+            if (KEEP) rd[KEEP ? r : 0] = rden;
+            cp[r] = r < M - 2 ? c * rden : R(0);
+            p[r] = r > 1 ? Cx<C>::mk((p[r].x - a * p[r - 1].x) * rden, (p[r].y - a * p[r - 1].y) * rden)
+                         : Cx<C>::mk(p[r].x * rden, p[r].y * rden);
+            qq[r] = (r == 1 ? -a : -a * qq[r - 1]) * rden;
+            ss[r] = ((r == M - 2 ? -c : R(0)) - (r > 1 ? a * ss[r - 1] : R(0))) * rden;
+        }
+#pragma unroll
+        for (int r = M - 3; r >= 1; --r) {
+            p[r] = Cx<C>::mk(p[r].x - cp[r] * p[r + 1].x, p[r].y - cp[r] * p[r + 1].y);
+            qq[r] -= cp[r] * qq[r + 1];
+            ss[r] -= cp[r] * ss[r + 1];
+        }
+    }
+    // the same elimination of another right-hand side
+    template <typename F> __device__ inline void again(const F &coef, C (&p)[M]) const {
+#pragma unroll
+        for (int r = 1; r <= M - 2; ++r) {
+            R a, b, c;
+            coef(r, a, b, c);
+            const R rden = rd[KEEP ? r : 0];
+            p[r] = r > 1 ? Cx<C>::mk((p[r].x - a * p[r - 1].x) * rden, (p[r].y - a * p[r - 1].y) * rden)
+                         : Cx<C>::mk(p[r].x * rden, p[r].y * rden);
+        }
+#pragma unroll
+        for (int r = M - 3; r >= 1; --r) p[r] = Cx<C>::mk(p[r].x - cp[r] * p[r + 1].x, p[r].y - cp[r] * p[r + 1].y);
+    }
+    // the two rows of the reduced system (a, b, c) and their data
+    __device__ inline void first(R &a, R &b, R &c) const {
+        a = a0;
+        b = b0 + c0 * qq[1];
+        c = c0 * ss[1];
+    }
+    __device__ inline void last(R &a, R &b, R &c) const {
+        a = aL * qq[M - 2];
+        b = bL + aL * ss[M - 2];
+        c = cL;
+    }
+    __device__ inline C first(const C (&p)[M]) const { return Cx<C>::mk(p[0].x - c0 * p[1].x, p[0].y - c0 * p[1].y); }
+    __device__ inline C last(const C (&p)[M]) const {
+        return Cx<C>::mk(p[M - 1].x - aL * p[M - 2].x, p[M - 1].y - aL * p[M - 2].y);
+    }
+    // row r of the solution
+    __device__ inline C row(const C (&p)[M], int r, C F, C E) const {
+        return r == 0 ? F : r == M - 1 ? E
+               : Cx<C>::mk(p[r].x + qq[r] * F.x + ss[r] * E.x, p[r].y + qq[r] * F.y + ss[r] * E.y);
+    }
+};
+// the residual of a segment's rows into r: data(q) less the rows (coef) applied to x, whose neighbours
+// past the segment's ends are xm and xp
+template <typename C, int M, typename F, typename G>
+__device__ inline void tri_residual(const F &coef, const G &data, const C (&x)[M], C xm, C xp, C (&r)[M]) {
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        typename Cx<C>::R a, b, c;
+        coef(q, a, b, c);
+        C l = xm, u = xp;
+        if (q > 0) l = x[q > 0 ? q - 1 : 0];
+        if (q < M - 1) u = x[q < M - 1 ? q + 1 : q];
+        const C d = data(q);
+        r[q] = Cx<C>::mk(d.x - (a * l.x + b * x[q].x + c * u.x), d.y - (a * l.y + b * x[q].y + c * u.y));
+    }
+}
+
+// 3''. The same solves as a partitioned Thomas recurrence (TriSegment).  A workgroup of 256 threads
+//     takes 16 consecutive lines and gives each line 16 segments; a row of the 16 lines is 256
+//     contiguous bytes, so loads and stores move whole cache lines without staging.  The reduced
+//     system (32 unknowns per line) is solved by one thread per line, TP_CH rows' operands read
+//     ahead of the chain; the segments then form their interior values.  The serial chain per
 //     line is 2 (M - 2) + 64 steps instead of 2 ny, the work about twice the plain recurrence's, and
 //     the spectrum moves once each way.  The mean mode pins row 1 as the wave solve does; MEAN_ZERO
 //     zeroes that line.  256 x 192 x 256 in FP64: 92 us with the lines staged in LDS (70 KB, two
 //     workgroups per CU) and the reduced system's operands read step by step; 57 now (FP32: 50 and
 //     31), 64^3 13.1 and 7.8.
+//     REFINE: one step of iterative refinement, as in the wave solve, which the FP64 lines of fewer
+//     than 64 rows took before.  Over ny = 16 .. 63, uniform spacing in a 4 pi x 2 x 2 pi box, the
+//     slowest modes' rms error is 3.7e-14 without the step, 1.2e-14 with it and 1.2e-14 in the wave
+//     solve; from 64 rows on the recurrence alone is as accurate as it was.
 static constexpr int TP_LINES = 16, TP_SEGS = 16, TP_CH = 8;
-template <typename C, int M, bool MEAN_ZERO>
+template <typename C, int M, bool MEAN_ZERO, bool REFINE>
 __global__ __launch_bounds__(TP_LINES * TP_SEGS, M <= 12 ? 3 : 2) void tridiag_part_kernel(int nlines, int stride, int nxh, int ny,
                                                                         size_t plane, C *hat,
                                                                         const typename Cx<C>::R *__restrict__ lamx,
@@ -947,7 +1033,6 @@ __global__ __launch_bounds__(TP_LINES * TP_SEGS, M <= 12 ? 3 : 2) void tridiag_p
                                                                         const typename Cx<C>::R *__restrict__ bdrow,
                                                                         const typename Cx<C>::R *__restrict__ crow) {
     using R = typename Cx<C>::R;
-    static_assert(M >= 3, "a segment has interior rows");
     constexpr int NR = 2 * TP_SEGS;   // reduced rows per line
     __shared__ R ra[NR][TP_LINES], rb[NR][TP_LINES], rc[NR][TP_LINES];
     __shared__ C rd[NR][TP_LINES];
@@ -956,14 +1041,16 @@ __global__ __launch_bounds__(TP_LINES * TP_SEGS, M <= 12 ? 3 : 2) void tridiag_p
     const bool live = t < nlines && t % stride < nxh;   // a line, not the padding of a kx row
     const bool ident_line = !live || (MEAN_ZERO && t == 0);
     const int j0 = sg * M;
+    const C zero = Cx<C>::mk(R(0), R(0));
     // row r of the segment: (a, b, c) and the data
     auto solved = [&](int r) { return !ident_line && j0 + r < ny && !(t == 0 && j0 + r == 0); };
-    C p[M];
+    C p[M], d[REFINE ? M : 1];
     C *h = hat + (size_t)(t < nlines ? t : 0) + plane * j0;
 #pragma unroll
     for (int r = 0; r < M; ++r) {
-        p[r] = Cx<C>::mk(R(0), R(0));
+        p[r] = zero;
         if (solved(r)) p[r] = h[plane * r];
+        if (REFINE) d[REFINE ? r : 0] = p[r];
     }
     const R k = live ? lamx[t % stride] + lamz[t / stride] : R(0);
     auto coef = [&](int r, R &a, R &b, R &c) {
@@ -978,89 +1065,91 @@ __global__ __launch_bounds__(TP_LINES * TP_SEGS, M <= 12 ? 3 : 2) void tridiag_p
             c = R(0);
         }
     };
-    // ---- interior rows 1 .. M-2: forward elimination with the three right-hand sides
-    R cp[M], qq[M], ss[M];
-    R a0, b0, c0, aL, bL, cL;
-    coef(0, a0, b0, c0);
-    coef(M - 1, aL, bL, cL);
-#pragma unroll
-    for (int r = 1; r <= M - 2; ++r) {
-        R a, b, c;
-        coef(r, a, b, c);
-        const R den = r > 1 ? b - a * cp[r - 1] : b;
-        const R rden = R(1) / den;
-        cp[r] = r < M - 2 ? c * rden : R(0);
-        p[r] = r > 1 ? Cx<C>::mk((p[r].x - a * p[r - 1].x) * rden, (p[r].y - a * p[r - 1].y) * rden)
-                     : Cx<C>::mk(p[r].x * rden, p[r].y * rden);
-        qq[r] = (r == 1 ? -a : -a * qq[r - 1]) * rden;
-        ss[r] = ((r == M - 2 ? -c : R(0)) - (r > 1 ? a * ss[r - 1] : R(0))) * rden;
-    }
-    // back substitution of the three right-hand sides
-#pragma unroll
-    for (int r = M - 3; r >= 1; --r) {
-        p[r] = Cx<C>::mk(p[r].x - cp[r] * p[r + 1].x, p[r].y - cp[r] * p[r + 1].y);
-        qq[r] -= cp[r] * qq[r + 1];
-        ss[r] -= cp[r] * ss[r + 1];
-    }
-    // ---- the segment's two rows of the reduced system: F (row 0) and E (row M-1)
-    ra[2 * sg][tt] = a0;
-    rb[2 * sg][tt] = b0 + c0 * qq[1];
-    rc[2 * sg][tt] = c0 * ss[1];
-    rd[2 * sg][tt] = Cx<C>::mk(p[0].x - c0 * p[1].x, p[0].y - c0 * p[1].y);
-    ra[2 * sg + 1][tt] = aL * qq[M - 2];
-    rb[2 * sg + 1][tt] = bL + aL * ss[M - 2];
-    rc[2 * sg + 1][tt] = cL;
-    rd[2 * sg + 1][tt] = Cx<C>::mk(p[M - 1].x - aL * p[M - 2].x, p[M - 1].y - aL * p[M - 2].y);
+    TriSegment<C, M, REFINE> seg;
+    seg.eliminate(coef, p);
+    seg.first(ra[2 * sg][tt], rb[2 * sg][tt], rc[2 * sg][tt]);
+    rd[2 * sg][tt] = seg.first(p);
+    seg.last(ra[2 * sg + 1][tt], rb[2 * sg + 1][tt], rc[2 * sg + 1][tt]);
+    rd[2 * sg + 1][tt] = seg.last(p);
     __syncthreads();
-    // ---- the reduced system of each line, one thread per line (Thomas; solution into rd)
-    if (sg == 0) {
+    // the reduced system of each line, one thread per line (Thomas; solution into rd); again: with the
+    // factors of the first time (rb: reciprocal denominators)
+    auto reduced = [&](auto again_) {
+        constexpr bool again = decltype(again_)::value;
         R cprev = R(0);
-        C dprev = Cx<C>::mk(R(0), R(0));
+        C dprev = zero;
         for (int r0 = 0; r0 < NR; r0 += TP_CH) {
             R a[TP_CH], b[TP_CH], c[TP_CH];
-            C d[TP_CH];
+            C e[TP_CH];
 #pragma unroll
             for (int u = 0; u < TP_CH; ++u) {
                 a[u] = ra[r0 + u][tt];
                 b[u] = rb[r0 + u][tt];
-                c[u] = rc[r0 + u][tt];
-                d[u] = rd[r0 + u][tt];
+                if (!again) c[u] = rc[r0 + u][tt];
+                e[u] = rd[r0 + u][tt];
             }
 #pragma unroll
             for (int u = 0; u < TP_CH; ++u) {
-                const R den = b[u] - a[u] * cprev, rden = R(1) / den;
-                cprev = c[u] * rden;
-                dprev = Cx<C>::mk((d[u].x - a[u] * dprev.x) * rden, (d[u].y - a[u] * dprev.y) * rden);
-                rc[r0 + u][tt] = cprev;
+                R rden = b[u];
+                if (!again) {
+                    const R den = b[u] - a[u] * cprev;
+                    rden = R(1) / den;
+                    cprev = c[u] * rden;
+                    rc[r0 + u][tt] = cprev;
+                    if (REFINE) rb[r0 + u][tt] = rden;
+                }
+                dprev = Cx<C>::mk((e[u].x - a[u] * dprev.x) * rden, (e[u].y - a[u] * dprev.y) * rden);
                 rd[r0 + u][tt] = dprev;
             }
         }
         C xn = dprev;
         for (int r0 = NR - TP_CH; r0 >= 0; r0 -= TP_CH) {
             R c[TP_CH];
-            C d[TP_CH];
+            C e[TP_CH];
 #pragma unroll
             for (int u = 0; u < TP_CH; ++u) {
                 c[u] = rc[r0 + u][tt];
-                d[u] = rd[r0 + u][tt];
+                e[u] = rd[r0 + u][tt];
             }
 #pragma unroll
             for (int u = TP_CH - 1; u >= 0; --u) {
                 if (r0 + u == NR - 1) continue;
-                xn = Cx<C>::mk(d[u].x - c[u] * xn.x, d[u].y - c[u] * xn.y);
+                xn = Cx<C>::mk(e[u].x - c[u] * xn.x, e[u].y - c[u] * xn.y);
                 rd[r0 + u][tt] = xn;
             }
         }
-    }
+    };
+    if (sg == 0) reduced(std::false_type{});
     __syncthreads();
     // ---- every row of the segment from F and E
-    if (!live) return;
     const C F = rd[2 * sg][tt], E = rd[2 * sg + 1][tt];
+    if constexpr (REFINE) {
+        C x[M];
 #pragma unroll
-    for (int r = 0; r < M; ++r) {
-        if (j0 + r < ny)
-            h[plane * r] = r == 0 ? F : r == M - 1 ? E
-                           : Cx<C>::mk(p[r].x + qq[r] * F.x + ss[r] * E.x, p[r].y + qq[r] * F.y + ss[r] * E.y);
+        for (int r = 0; r < M; ++r) x[r] = seg.row(p, r, F, E);
+        C xm = zero, xp = zero;
+        if (sg > 0) xm = rd[2 * sg - 1][tt];
+        if (sg < TP_SEGS - 1) xp = rd[2 * sg + 2][tt];
+        tri_residual<C, M>(coef, [&](int r) { return d[REFINE ? r : 0]; }, x, xm, xp, p);
+        seg.again(coef, p);
+        __syncthreads();   // the neighbours' ends have been read
+        rd[2 * sg][tt] = seg.first(p);
+        rd[2 * sg + 1][tt] = seg.last(p);
+        __syncthreads();
+        if (sg == 0) reduced(std::true_type{});
+        __syncthreads();
+        const C dF = rd[2 * sg][tt], dE = rd[2 * sg + 1][tt];
+        if (!live) return;
+#pragma unroll
+        for (int r = 0; r < M; ++r) {
+            const C e = seg.row(p, r, dF, dE);
+            if (j0 + r < ny) h[plane * r] = Cx<C>::mk(x[r].x + e.x, x[r].y + e.y);
+        }
+    } else {
+        if (!live) return;
+#pragma unroll
+        for (int r = 0; r < M; ++r)
+            if (j0 + r < ny) h[plane * r] = seg.row(p, r, F, E);
     }
 }
 
@@ -1068,12 +1157,14 @@ __global__ __launch_bounds__(TP_LINES * TP_SEGS, M <= 12 ? 3 : 2) void tridiag_p
 //     fits a CU's LDS and the launches are short: z-transforms of the column's lines, its tridiagonal
 //     solves as tridiag_part_kernel does them (CS_SEGS segments of M rows; the reduced rows' data in the
 //     tile, at the rows they stand for), and the transforms back, one workgroup per kx.  Bound by
-//     latency: 64^3 18.2 us in three launches, 13.4 in one; 128 x 97 x 64 26.2 and 18.0.
+//     latency: 64^3 18.2 us in three launches, 13.0 in one; 128 x 97 x 64 26.2 and 17.1.
+//     REFINE as there (rms error over ny = 16 .. 63 2.3e-14 without the step, 1.2e-14 with it; from 64
+//     rows on, without, 6.4e-14 against 8.0e-14 with 16 segments): 64 x 48 x 64 11.0 us without, 15.2.
 static constexpr int CS_T = 512, CS_SEGS = 8;
 template <int N, int M> constexpr size_t column_lds() {
     return (size_t)CS_SEGS * M * RFft<N, CS_T>::LS * 16 + RFft<N, CS_T>::TW * 16 + 3 * 2 * CS_SEGS * (N < 64 ? N : 64) * 8;
 }
-template <int N, int M>
+template <int N, int M, bool REFINE>
 __global__ __launch_bounds__(CS_T) void column_solve_kernel(int ny, const double2 *__restrict__ tw,
                                                             const double *__restrict__ lamx,
                                                             const double *__restrict__ lamz,
@@ -1083,7 +1174,7 @@ __global__ __launch_bounds__(CS_T) void column_solve_kernel(int ny, const double
     using F = RFft<N, CS_T>;
     using C2 = Cx<double2>;
     constexpr int NK = N < 64 ? N : 64, NR = 2 * CS_SEGS;   // kz at a time, reduced rows
-    static_assert(M >= 3 && NK * CS_SEGS <= CS_T, "a thread per segment");
+    static_assert(NK * CS_SEGS <= CS_T, "a thread per segment");
     extern __shared__ __align__(16) unsigned char lds_raw[];
     double2 *tile = reinterpret_cast<double2 *>(lds_raw), *twl = tile + CS_SEGS * M * F::LS;
     double *ra = reinterpret_cast<double *>(twl + F::TW), *rb = ra + NR * NK, *rc = rb + NR * NK;
@@ -1091,11 +1182,11 @@ __global__ __launch_bounds__(CS_T) void column_solve_kernel(int ny, const double
     double2 *col = hat + (size_t)kx * ny * N;
     rf_stage<double2, N, CS_T>(twl, tw);
     if constexpr (!F::TW0) __syncthreads();
-    double2 e[16];
     for (int j0 = 0; j0 < ny; j0 += F::LPW) {
         const int j = j0 + l;
         const bool on = j < ny;
         double2 *line = tile + (on ? j : 0) * F::LS;
+        double2 e[16];   // (one for both loops would keep idle lanes' values through the solves: spills)
         if (on) {
 #pragma unroll
             for (int s = 0; s < 16; ++s) e[s] = col[(size_t)j * N + t + F::M * s];
@@ -1113,6 +1204,7 @@ __global__ __launch_bounds__(CS_T) void column_solve_kernel(int ny, const double
         const bool mine = sg < CS_SEGS;
         double2 *c = tile + rf_pad(kz);
         const double k = lamx[kx] + lamz[kz];
+        const double2 zero = make_double2(0.0, 0.0);
         auto solved = [&](int r) { return r0 + r < ny && !(kx == 0 && kz == 0 && r0 + r == 0); };
         auto coef = [&](int r, double &a, double &b, double &cc) {
             a = cc = 0.0;
@@ -1123,72 +1215,116 @@ __global__ __launch_bounds__(CS_T) void column_solve_kernel(int ny, const double
                 cc = crow[r0 + r];
             }
         };
-        double2 p[M];
-        double cp[M], qq[M], ss[M];
+        double2 p[M], df = zero, dl = zero;
+        TriSegment<double2, M, REFINE> seg;
         __syncthreads();
         if (mine) {
 #pragma unroll
             for (int r = 0; r < M; ++r) {
-                p[r] = make_double2(0.0, 0.0);
+                p[r] = zero;
                 if (solved(r)) p[r] = c[(r0 + r) * F::LS];
             }
-            double a0, b0, c0, aL, bL, cL;
-            coef(0, a0, b0, c0);
-            coef(M - 1, aL, bL, cL);
-#pragma unroll
-            for (int r = 1; r <= M - 2; ++r) {
-                double a, b, cc;
-                coef(r, a, b, cc);
-                const double rden = 1.0 / (r > 1 ? b - a * cp[r - 1] : b);
-                cp[r] = r < M - 2 ? cc * rden : 0.0;
-                p[r] = r > 1 ? C2::mk((p[r].x - a * p[r - 1].x) * rden, (p[r].y - a * p[r - 1].y) * rden)
-                             : C2::mk(p[r].x * rden, p[r].y * rden);
-                qq[r] = (r == 1 ? -a : -a * qq[r - 1]) * rden;
-                ss[r] = ((r == M - 2 ? -cc : 0.0) - (r > 1 ? a * ss[r - 1] : 0.0)) * rden;
-            }
-#pragma unroll
-            for (int r = M - 3; r >= 1; --r) {
-                p[r] = C2::mk(p[r].x - cp[r] * p[r + 1].x, p[r].y - cp[r] * p[r + 1].y);
-                qq[r] -= cp[r] * qq[r + 1];
-                ss[r] -= cp[r] * ss[r + 1];
-            }
-            // the reduced rows F (row 0) and E (row M-1); their data in the tile, at those rows
-            ra[2 * sg * NK + tk] = a0;
-            rb[2 * sg * NK + tk] = b0 + c0 * qq[1];
-            rc[2 * sg * NK + tk] = c0 * ss[1];
-            c[r0 * F::LS] = C2::mk(p[0].x - c0 * p[1].x, p[0].y - c0 * p[1].y);
-            ra[(2 * sg + 1) * NK + tk] = aL * qq[M - 2];
-            rb[(2 * sg + 1) * NK + tk] = bL + aL * ss[M - 2];
-            rc[(2 * sg + 1) * NK + tk] = cL;
-            c[(r0 + M - 1) * F::LS] = C2::mk(p[M - 1].x - aL * p[M - 2].x, p[M - 1].y - aL * p[M - 2].y);
+            df = p[0];
+            dl = p[M - 1];
+            seg.eliminate(coef, p);
+            const int f = 2 * sg * NK + tk, g = f + NK;
+            seg.first(ra[f], rb[f], rc[f]);
+            c[r0 * F::LS] = seg.first(p);
+            seg.last(ra[g], rb[g], rc[g]);
+            c[(r0 + M - 1) * F::LS] = seg.last(p);
         }
-        __syncthreads();
-        if (sg == 0) {
+        // the reduced rows of a kz, by the first segment's thread; again: with the kept factors
+        auto reduced = [&](auto again_) {
+            constexpr bool again = decltype(again_)::value;
             auto row = [&](int r) -> double2 & { return c[(r / 2 * M + (r % 2 ? M - 1 : 0)) * F::LS]; };
-            double cs[NR], cprev = 0.0;
-            double2 ds[NR], dprev = make_double2(0.0, 0.0);
+            constexpr int CH = REFINE ? 8 : NR;   // rows read ahead of the chain
+            double cs[CH], cprev = 0.0;
+            double2 ds[CH], dprev = zero;
 #pragma unroll
-            for (int r = 0; r < NR; ++r) ds[r] = row(r);
+            for (int q = 0; q < NR; q += CH) {
 #pragma unroll
-            for (int r = 0; r < NR; ++r) {
-                const double a = ra[r * NK + tk], rden = 1.0 / (rb[r * NK + tk] - a * cprev);
-                cs[r] = cprev = rc[r * NK + tk] * rden;
-                ds[r] = dprev = C2::mk((ds[r].x - a * dprev.x) * rden, (ds[r].y - a * dprev.y) * rden);
+                for (int u = 0; u < CH; ++u) ds[u] = row(q + u);
+#pragma unroll
+                for (int u = 0; u < CH; ++u) {
+                    const int o = (q + u) * NK + tk;
+                    const double a = ra[o];
+                    double rden = rb[o];
+                    if (!again) {
+                        rden = 1.0 / (rden - a * cprev);
+                        cs[u] = cprev = rc[o] * rden;
+                        if (REFINE) {
+                            rb[o] = rden;
+                            rc[o] = cprev;
+                        }
+                    }
+                    ds[u] = dprev = C2::mk((ds[u].x - a * dprev.x) * rden, (ds[u].y - a * dprev.y) * rden);
+                    if (REFINE) row(q + u) = dprev;
+                }
+                if (REFINE) __builtin_amdgcn_sched_barrier(0);
             }
-            row(NR - 1) = dprev;
+            if (!REFINE) row(NR - 1) = dprev;
 #pragma unroll
-            for (int r = NR - 2; r >= 0; --r) {
-                dprev = C2::mk(ds[r].x - cs[r] * dprev.x, ds[r].y - cs[r] * dprev.y);
-                row(r) = dprev;
+            for (int q = NR - CH; q >= 0; q -= CH) {
+                if (REFINE) {
+#pragma unroll
+                    for (int u = 0; u < CH; ++u) {
+                        ds[u] = row(q + u);
+                        cs[u] = rc[(q + u) * NK + tk];
+                    }
+                }
+#pragma unroll
+                for (int u = CH - 1; u >= 0; --u) {
+                    if (q + u == NR - 1) continue;
+                    dprev = C2::mk(ds[u].x - cs[u] * dprev.x, ds[u].y - cs[u] * dprev.y);
+                    row(q + u) = dprev;
+                }
+                if (REFINE) __builtin_amdgcn_sched_barrier(0);
             }
-        }
+        };
         __syncthreads();
-        if (mine) {
+        if (sg == 0) reduced(std::false_type{});
+        __syncthreads();
+        if constexpr (REFINE) {
+            double2 x[M];
+            if (mine) {
+                const double2 f = c[r0 * F::LS], g = c[(r0 + M - 1) * F::LS];
+                double2 xm = zero, xp = zero;
+                if (sg > 0) xm = c[(r0 - 1) * F::LS];
+                if (sg < CS_SEGS - 1) xp = c[(r0 + M) * F::LS];
+#pragma unroll
+                for (int r = 0; r < M; ++r) x[r] = seg.row(p, r, f, g);
+                // (the interior rows' data are still in the tile)
+                auto data = [&](int r) {
+                    double2 v = zero;
+                    if (r == 0) v = df;
+                    else if (r == M - 1) v = dl;
+                    else if (solved(r)) v = c[(r0 + r) * F::LS];
+                    return v;
+                };
+                tri_residual<double2, M>(coef, data, x, xm, xp, p);
+                seg.again(coef, p);
+            }
+            __syncthreads();   // the neighbours' ends have been read
+            if (mine) {
+                c[r0 * F::LS] = seg.first(p);
+                c[(r0 + M - 1) * F::LS] = seg.last(p);
+            }
+            __syncthreads();
+            if (sg == 0) reduced(std::true_type{});
+            __syncthreads();
+            if (mine) {
+                const double2 f = c[r0 * F::LS], g = c[(r0 + M - 1) * F::LS];
+#pragma unroll
+                for (int r = 0; r < M; ++r) {
+                    const double2 v = seg.row(p, r, f, g);
+                    if (r0 + r < ny) c[(r0 + r) * F::LS] = C2::mk(x[r].x + v.x, x[r].y + v.y);
+                }
+            }
+        } else if (mine) {
             const double2 f = c[r0 * F::LS], g = c[(r0 + M - 1) * F::LS];
 #pragma unroll
             for (int r = 1; r <= M - 2; ++r)
-                if (r0 + r < ny)
-                    c[(r0 + r) * F::LS] = C2::mk(p[r].x + qq[r] * f.x + ss[r] * g.x, p[r].y + qq[r] * f.y + ss[r] * g.y);
+                if (r0 + r < ny) c[(r0 + r) * F::LS] = seg.row(p, r, f, g);
         }
     }
     __syncthreads();
@@ -1196,6 +1332,7 @@ __global__ __launch_bounds__(CS_T) void column_solve_kernel(int ny, const double
         const int j = j0 + l;
         const bool on = j < ny;
         double2 *line = tile + (on ? j : 0) * F::LS;
+        double2 e[16];
         if (on) rf_gather<double2, N>(e, t, line);
         if constexpr (!F::TW0) __syncthreads();
         fft_line<double2, N, true>(e, t, twl, line, on);
@@ -1208,8 +1345,8 @@ __global__ __launch_bounds__(CS_T) void column_solve_kernel(int ny, const double
 }
 
 // launches the partitioned solve for ny <= 256, in FP32 for ny >= 64 (false: the caller takes another
-// solver).  Below 64 rows a line's segments past ny idle, and still FP64 takes 7.4 us at 64 x 24 x 64
-// and 9.8 at 128 x 33 x 128 where a wave per line took 14.2 and 28.8; the FP32 passes of the defect
+// solver).  Below 64 rows a line's segments past ny idle, and still FP64, with its refinement step,
+// takes 14.1 us at 128 x 33 x 128 where a wave per line took 28.8; the FP32 passes of the defect
 // correction keep the wave's rounding there.
 template <typename C, bool MEAN_ZERO>
 static bool launch_tridiag_part(hipStream_t st, const Dims &d, C *hat, const typename Cx<C>::R *lamx,
@@ -1219,14 +1356,21 @@ static bool launch_tridiag_part(hipStream_t st, const Dims &d, C *hat, const typ
     const int nxh = d.nx / 2 + 1, stride = fft_stride_t<C>(d.nx), nlines = stride * d.nz, m = (d.ny + TP_SEGS - 1) / TP_SEGS;
     const size_t plane = (size_t)nlines;
     const dim3 grid((nlines + TP_LINES - 1) / TP_LINES), blk(TP_LINES * TP_SEGS);
-#define TP_CASE(MM)                                                                                            \
-    if (m <= MM) {                                                                                             \
-        hipLaunchKernelGGL((tridiag_part_kernel<C, MM, MEAN_ZERO>), grid, blk, 0, st, nlines, stride, nxh, d.ny, plane, \
-                           hat, lamx, lamz, a, bd, c);                                                         \
-        return true;                                                                                           \
+#define TP_LAUNCH(MM, REF)                                                                                         \
+    hipLaunchKernelGGL((tridiag_part_kernel<C, MM, MEAN_ZERO, REF>), grid, blk, 0, st, nlines, stride, nxh, d.ny, \
+                       plane, hat, lamx, lamz, a, bd, c)
+    if (d.ny < 64) {
+        if constexpr (sizeof(C) == 16) TP_LAUNCH(4, true);
+        return true;
+    }
+#define TP_CASE(MM)           \
+    if (m <= MM) {            \
+        TP_LAUNCH(MM, false); \
+        return true;          \
     }
     TP_CASE(4) TP_CASE(8) TP_CASE(12) TP_CASE(16)
 #undef TP_CASE
+#undef TP_LAUNCH
     return false;
 }
 
@@ -1644,11 +1788,17 @@ static constexpr size_t COLUMN_LDS = 160 * 1024 - 1024;
 template <int N, int M> static hipError_t column_solve(mdx_handle *h) {
     const Dims d = h->d;
     constexpr size_t lds = column_lds<N, M>();
-    const hipError_t e = rf_allow<column_solve_kernel<N, M>>(lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((column_solve_kernel<N, M>), dim3(d.nx / 2 + 1), dim3(CS_T), lds, h->stream, d.ny,
-                       (const double2 *)h->tw_z, h->lamx, h->lamz, h->tw_a, h->bdrow, h->crow, (double2 *)h->hat);
-    return hipGetLastError();
+    auto launch = [&](auto refine) {
+        constexpr auto FN = column_solve_kernel<N, M, decltype(refine)::value>;
+        const hipError_t e = rf_allow<FN>(lds);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(FN, dim3(d.nx / 2 + 1), dim3(CS_T), lds, h->stream, d.ny, (const double2 *)h->tw_z, h->lamx,
+                           h->lamz, h->tw_a, h->bdrow, h->crow, (double2 *)h->hat);
+        return hipGetLastError();
+    };
+    if constexpr (CS_SEGS * M < 64) return launch(std::true_type{});
+    else if constexpr (CS_SEGS * (M - 1) >= 63) return launch(std::false_type{});
+    else return d.ny < 64 ? launch(std::true_type{}) : launch(std::false_type{});
 }
 #define CS_ROWS(N, CALL)                                  \
     do {                                                  \

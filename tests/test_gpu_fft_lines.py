@@ -1,0 +1,71 @@
+"""Accuracy of the FFT projection's FP64 tridiagonal solves below 64 rows, where a partitioned
+recurrence alone loses the slow modes' digits: phi's (kx, kz) lines against the same systems solved
+in extended precision, over ny = 17 .. 63, through the column solves (nz = 64) and the partitioned
+solves (nz = 16).  Bound: with the refinement step the rms error of these lines is 1.3 to 2.1 times
+the plain Thomas recurrence's in FP64 (formed here), without it 3.2 to 5.4 times; 2.6 lies between."""
+import math
+
+import numpy as np
+import pytest
+
+import mobydiff_amd as M
+
+pytestmark = pytest.mark.gpu
+
+LX, LY, LZ = 4 * math.pi, 2.0, 2 * math.pi
+MODES = [(kx, kz) for kx in (1, 2, 3) for kz in (0, 1, 2)]
+
+
+def _thomas(dt, dyi2, k, d):
+    """Rows a x_(j-1) + (bd - k) x_j + c x_(j+1) = d of uniform spacing, Neumann ends."""
+    ny = len(d)
+    a, c, bd = np.full(ny, dyi2), np.full(ny, dyi2), np.full(ny, -2.0 * dyi2)
+    a[0] = c[-1] = 0.0
+    bd[0] = bd[-1] = -dyi2
+    b = [(x - k).astype(dt) for x in bd]   # rounded in FP64, as every solver's rows are
+    a, c, x = a.astype(dt), c.astype(dt), d.copy()
+    cp = np.zeros((ny,) + k.shape, dt)
+    for j in range(ny):
+        r = dt(1) / (b[j] - (a[j] * cp[j - 1] if j else 0))
+        cp[j] = c[j] * r
+        x[j] = (x[j] - (a[j] * x[j - 1] if j else 0)) * r
+    for j in range(ny - 2, -1, -1):
+        x[j] = x[j] - cp[j] * x[j + 1]
+    return x
+
+
+@pytest.mark.parametrize("nz", [64, 16])
+def test_slow_modes_keep_their_digits(nz):
+    nx, dtg, rng = 64, 0.1, np.random.default_rng(5)
+    dx, dz = LX / nx, LZ / nz
+    lam = np.array([(4.0 / (dx * dx)) * math.sin(math.pi * kx / nx) ** 2
+                    + (4.0 / (dz * dz)) * math.sin(math.pi * kz / nz) ** 2 for kx, kz in MODES])
+    i, k = np.arange(nx), np.arange(nz)
+    ex = np.exp(-2j * np.pi * np.outer([m[0] for m in MODES], i) / nx).astype(np.clongdouble)
+    ez = np.exp(-2j * np.pi * np.outer([m[1] for m in MODES], k) / nz).astype(np.clongdouble)
+    lines = lambda f: np.stack([ex[m] @ (ez[m] @ f.reshape(nz, -1)).reshape(f.shape[1], nx).T
+                                for m in range(len(MODES))], 1)   # (k, j, i) -> (j, mode)
+    err, plain = [], []
+    for ny in range(17, 64, 2):
+        dy = LY / ny
+        us = np.zeros((nz + 2, ny + 2, nx + 2))
+        for m, (kx, kz) in enumerate(MODES):
+            us[1:-1, 1:-1, 1:-1] += (rng.standard_normal(ny)[None, :, None] * np.cos(2 * np.pi * kz * k / nz)[:, None, None]
+                                     * np.cos(2 * np.pi * kx * i / nx))
+        us[1:-1, 1:-1, nx + 1], us[1:-1, 1:-1, 0] = us[1:-1, 1:-1, 1], us[1:-1, 1:-1, nx]
+        ch = M.Channel(M.channel_config(nx, ny, nz, LX, LY, LZ, 1000.0, solver=M.SOLVER_FFT, p_neumann_y=False))
+        ch.upload(us=us)
+        ch.pressure_projection(dtg)
+        phi = ch.download(("pn",))["pn"][1:-1, 1:-1, 1:-1]
+        ch.close()
+        u = us.astype(np.longdouble)
+        rhs = (u[1:-1, 1:-1, 2:] - u[1:-1, 1:-1, 1:-1]) / np.longdouble(dx) / np.longdouble(dtg)
+        d = lines(rhs)
+        dyi2 = 1.0 / (dy * dy)
+        ref = _thomas(np.longdouble, dyi2, lam, d)
+        scale = np.abs(ref).max(0)
+        err.append(np.abs(lines(phi.astype(np.longdouble)) - ref).max(0) / scale)
+        plain.append(np.abs(_thomas(np.float64, dyi2, lam, d.astype(np.complex128)) - ref).max(0) / scale)
+    rms = [float(np.sqrt((np.array(e, np.float64) ** 2).mean())) for e in (err, plain)]
+    print(nz, rms, rms[0] / rms[1], flush=True)
+    assert rms[0] < 2.6 * rms[1], rms

@@ -1385,10 +1385,7 @@ static bool launch_tridiag_wave(hipStream_t st, const Dims &d, C *hat, const typ
     const size_t lds = (size_t)TW_LINES * (d.ny + 1) * sizeof(C);   // <= 66 KB (ny <= 256)
 #define TW_CASE(MM)                                                                                            \
     case MM: {                                                                                                 \
-        static const hipError_t attr = hipFuncSetAttribute(                                                    \
-            reinterpret_cast<const void *>(&tridiag_wave_kernel<C, MM, MEAN_ZERO>),                            \
-            hipFuncAttributeMaxDynamicSharedMemorySize, 16 * 257 * (int)sizeof(C));                            \
-        if (attr != hipSuccess) return false;                                                                  \
+        if (allow_lds<tridiag_wave_kernel<C, MM, MEAN_ZERO>>(lds) != hipSuccess) return false;                 \
         hipLaunchKernelGGL((tridiag_wave_kernel<C, MM, MEAN_ZERO>), grid, blk, lds, st, nlines, stride, nxh, d.ny, plane, \
                            hat, lamx, lamz, a, bd, c);                                                         \
         return true;                                                                                           \
@@ -1633,30 +1630,12 @@ static size_t fft_lds(int lines, int ls, int n) {
     return (2 * (size_t)lines * ls + (size_t)(n / 2)) * sizeof(C);
 }
 
-// allow a z-transform kernel more than the default 64 KB of dynamic LDS (once per kernel)
-template <typename C>
-static hipError_t zfft_allow(size_t bytes) {
-    static size_t allowed = 65536;
-    if (bytes <= allowed) return hipSuccess;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&zfft_kernel<C>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    if (e == hipSuccess) allowed = bytes;
-    return e;
-}
-
-// allow a kernel more than the default 64 KB of dynamic LDS (once per kernel)
-template <auto FN> static hipError_t rf_allow(size_t bytes) {
-    if (bytes <= 65536) return hipSuccess;
-    static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(FN),
-                                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    return e;
-}
 // a kernel of the register transforms on `blocks` workgroups
 template <typename C, int N, int TH, auto FN, int W = 1, typename... A>
 static hipError_t rf_launch(hipStream_t st, unsigned blocks, A... args) {
     using F = RFft<N, TH>;
     const size_t lds = ((size_t)F::LPW * F::LS + F::TW) * sizeof(C);
-    const hipError_t e = rf_allow<FN>(lds);
+    const hipError_t e = allow_lds<FN>(lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(FN, dim3(blocks), dim3(TH * W), lds, st, args...);
     return hipGetLastError();
@@ -1713,8 +1692,6 @@ static hipError_t launch_zfft(hipStream_t st, const Dims &d, C *hat, const C *tw
 #undef ZF
     const int tx = z_tile(d.nz), nxh = d.nx / 2 + 1;
     const size_t shz = fft_lds<C>(tx, d.nz + 1, d.nz);
-    hipError_t e = zfft_allow<C>(shz);
-    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(zfft_kernel<C>, dim3(d.ny * ((nxh + tx - 1) / tx)), dim3(FFT_THREADS), shz, st, d, hat, tw, tx,
                        INV ? 1 : 0, fft_stride_t<C>(d.nx));
     return hipGetLastError();
@@ -1790,7 +1767,7 @@ template <int N, int M> static hipError_t column_solve(mdx_handle *h) {
     constexpr size_t lds = column_lds<N, M>();
     auto launch = [&](auto refine) {
         constexpr auto FN = column_solve_kernel<N, M, decltype(refine)::value>;
-        const hipError_t e = rf_allow<FN>(lds);
+        const hipError_t e = allow_lds<FN>(lds);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(FN, dim3(d.nx / 2 + 1), dim3(CS_T), lds, h->stream, d.ny, (const double2 *)h->tw_z, h->lamx,
                            h->lamz, h->tw_a, h->bdrow, h->crow, (double2 *)h->hat);

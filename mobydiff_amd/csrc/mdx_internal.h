@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/mobydiff_hip.h"
+#include "mdx_once.h"
 
 namespace mdx {
 
@@ -382,6 +383,19 @@ struct mdx_handle {
 
 // kernel launchers (defined in the .hip files)
 namespace mdx {
+// Allow kernel FN more than the default 64 KB of dynamic LDS on the current device.  The attribute
+// belongs to a device: a handle on a second one needs it set there too.
+template <auto FN> inline hipError_t allow_lds(size_t bytes) {
+    if (bytes <= 65536) return hipSuccess;
+    int dev = 0;
+    const hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    static OncePerDevice once;
+    return once.run(dev, [] {
+        return hipFuncSetAttribute(reinterpret_cast<const void *>(FN), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   160 * 1024);
+    });
+}
 GridK grid_k(const mdx_handle *h);
 BcK bc_k(const mdx_handle *h);
 

@@ -1075,9 +1075,7 @@ static hipError_t conv3(mdx_net *n, int cin, int cout, bool relu, const bf16 *in
     if (n->tiled_conv && cin == CI && cout == CO && relu == R && W % CTX == 0 && H % CTY == 0 &&                   \
         D % ConvTile<CI>::TZ == 0) {                                                                               \
         const unsigned tiles = (unsigned)((W / CTX) * (H / CTY) * (D / ConvTile<CI>::TZ));                          \
-        static const hipError_t attr = ConvTile<CI>::BYTES <= 65536 ? hipSuccess :                                 \
-            hipFuncSetAttribute(reinterpret_cast<const void *>(&conv3_tiled_kernel<CI, CO, R>),                     \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)ConvTile<CI>::BYTES);              \
+        const hipError_t attr = allow_lds<conv3_tiled_kernel<CI, CO, R>>(ConvTile<CI>::BYTES);                     \
         if (attr != hipSuccess) return attr;                                                                       \
         hipLaunchKernelGGL((conv3_tiled_kernel<CI, CO, R>), dim3(tiles), dim3(256), ConvTile<CI>::BYTES,           \
                            n->stream, in, up, cu, reinterpret_cast<const bf16x8 *>(wp), bias, out, W, H, D);       \

@@ -1094,27 +1094,39 @@ static int rb_occupancy(bool fp32, bool ibm, int maxp, bool stretch, size_t lds)
 // sized by one shape, need equal even parts.  `why` receives the reason when nothing fits.
 bool rb_plan(const mdx_handle *h, bool fp32, RbPlanOut &out, std::string &why) {
     const int nx = h->d.nx, ny = h->d.ny, nz = h->d.nz;
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, h->device) != hipSuccess) { why = "no device properties"; return false; }
-    if (h->rb_coop && !prop.cooperativeLaunch) { why = "device reports no cooperative launch"; return false; }
+    // single attributes: reading all device properties takes longer than the search below
+    auto attr = [&](hipDeviceAttribute_t a) {
+        int v = -1;
+        if (hipDeviceGetAttribute(&v, a, h->device) != hipSuccess) (void)hipGetLastError();
+        return v;
+    };
+    const int all_cus = attr(hipDeviceAttributeMultiprocessorCount), lds_block = attr(hipDeviceAttributeMaxSharedMemoryPerBlock),
+              lds_cu = attr(hipDeviceAttributeMaxSharedMemoryPerMultiprocessor);
+    if (all_cus < 1 || lds_block < 1) { why = "no device properties"; return false; }
+    if (h->rb_coop && attr(hipDeviceAttributeCooperativeLaunch) != 1) {
+        why = "device reports no cooperative launch";
+        return false;
+    }
     if (h->cfg.periodic[1] && ny % 2) { why = "odd periodic y"; return false; }
-    const int cus = h->rb_cus > 0 ? std::min(h->rb_cus, prop.multiProcessorCount) : prop.multiProcessorCount;
-    const size_t lds_max = prop.maxSharedMemoryPerMultiProcessor > prop.sharedMemPerBlock
-                               ? prop.maxSharedMemoryPerMultiProcessor : prop.sharedMemPerBlock;
+    const int cus = h->rb_cus > 0 ? std::min(h->rb_cus, all_cus) : all_cus;
+    const size_t lds_max = (size_t)std::max(lds_cu, lds_block);
     const size_t ts = fp32 ? 4 : 8;
     bool found = false;
     double best_cells = 1e300, best_x = 1e300;
     std::map<std::pair<int, size_t>, int> occupancy;   // by form and LDS size
-    why = "no decomposition fits (cus=" + std::to_string(cus) + ", lds/block=" + std::to_string(prop.sharedMemPerBlock) +
-          ", lds/cu=" + std::to_string(prop.maxSharedMemoryPerMultiProcessor) + ")";
+    why = "no decomposition fits (cus=" + std::to_string(cus) + ", lds/block=" + std::to_string(lds_block) +
+          ", lds/cu=" + std::to_string(lds_cu) + ")";
+    const long max_wg = 4L * cus;
     for (int px = 1; px <= nx / 2; ++px) {
         const int bx = rb_part_max(nx, px);
         if (bx + 2 * RB_H > RB_BX) continue;   // the fixed LDS row
         for (int py = 1; py <= std::max(1, ny / 2); ++py) {
+            if ((long)px * py > max_wg) break;
             const int by = rb_part_max(ny, py);
             if (by + 2 * RB_H > RB_BY) continue;   // the fixed LDS plane
             for (int pz = 1; pz <= nz / 2; ++pz) {
                 const int bz = rb_part_max(nz, pz);
+                if ((long)px * py * pz > max_wg) break;
                 const int nwg = px * py * pz;
                 const bool equal = (nx / 2) % px == 0 && ny % 2 == 0 && (ny / 2) % py == 0 && (nz / 2) % pz == 0;
                 // the column form where a thread per column (subdomain and face ring) fits
@@ -1134,7 +1146,6 @@ bool rb_plan(const mdx_handle *h, bool fp32, RbPlanOut &out, std::string &why) {
                 if (rb_ring_total(bx, by, bz) > RB_MAXR * RB_THREADS) continue;
                 const int total = rb_xchg_total(bx, by, bz);
                 if (total > RB_HE * RB_THREADS) continue;
-                if (nwg > 4 * cus) continue;
                 const double rounds = std::ceil((double)nwg / cus);
                 const double cells = rounds * bx * by * bz;
                 // a column form where one fits: the pair form relaxes absent cells too (48 x 32 x 24:

@@ -237,9 +237,9 @@ static void free_all(mdx_handle *h) {
                     h->cu, h->cv, h->cw, h->d_ihc, h->d_ihv, h->d_yc, h->phi, h->phi2, h->rhs,
                     h->e32, h->r32, h->e32b, h->mu64[0], h->mu64[1], h->mu64[2], h->mu32[0], h->mu32[1],
                     h->mu32[2], h->fft_rhs, h->hat, h->cp, h->den_inv, h->arow, h->tw_x, h->tw_z,
-                    h->red_part, h->red_max, h->max_part, h->rb_faces, h->phi_hist, h->res64,
+                    h->red_part, h->red_max, h->max_part, h->rb_sets[0].mem, h->rb_sets[1].mem, h->phi_hist, h->res64,
                     h->fft_phi, h->fft_res, h->fft_mean, h->hat32, h->cp32, h->den32, h->arow32, h->tw_x32,
-                    h->tw_z32, h->rb_xl32, h->rb_xl64, h->cvel, h->lamx, h->lamz, h->tw_a, h->bdrow, h->crow, h->lamx32, h->lamz32,
+                    h->tw_z32, h->cvel, h->lamx, h->lamz, h->tw_a, h->bdrow, h->crow, h->lamx32, h->lamz32,
                     h->tw_a32, h->bdrow32, h->crow32, h->fr_part, h->sola_tmp};
     for (auto &s : h->graphs)
         if (s.exec) (void)hipGraphExecDestroy(s.exec);
@@ -570,7 +570,7 @@ static void invalidate_graphs(mdx_handle *h) {
         if (s.exec) (void)hipGraphExecDestroy(s.exec);
         s = mdx_handle::GraphSlot{};
     }
-    h->rb_state = 0;   // the LDS solver's plan depends on the IBM state too
+    for (auto &r : h->rb_sets) r.state = 0;   // the LDS solver's plans depend on the IBM state too
 }
 
 static int upload_ibm(mdx_handle *h) {
@@ -780,6 +780,16 @@ static constexpr int MDX_LDS_REFUSED = 101;
 // restarts after which the LDS-resident solver stays off for the handle
 static constexpr int LDS_TIMEOUT_MAX = 3;
 
+// Neighbour waits gave up LDS_TIMEOUT_MAX times: the handle keeps to the streaming sweeps, whatever
+// CUs it is stepped on.
+static void lds_off(mdx_handle *h) {
+    for (auto &r : h->rb_sets) {
+        r.state = -1;
+        r.note = "streaming sweeps: neighbour waits of the LDS-resident sweeps gave up " +
+                 std::to_string(h->lds_timeouts) + " times";
+    }
+}
+
 // The wait-timeout word has been seen set: clear it on the device (it is set again only by a later
 // wait that gives up) and report the timeout once.
 static int lds_timeout_seen(mdx_handle *h) {
@@ -837,55 +847,68 @@ public:
 };
 
 // Plan and allocate the LDS-resident solver once the IBM state is known (z-invariant or absent IBM
-// coefficients); rb_state = -1 leaves the streaming sweeps in charge.
+// coefficients); state -1 leaves the streaming sweeps in charge.  A handle keeps one set of plans for
+// steps of its own and one for its share of a batch, so that stepping it one way costs the other
+// nothing.
 static int rb_prepare(mdx_handle *h) {
-    if (h->rb_state != 0) return MDX_OK;
-    h->rb_state = -1;
+    RbSet &S = h->rb_sets[h->in_batch ? 1 : 0];
+    h->rb = &S;
+    if (h->in_batch && S.cus != h->batch_cus) {
+        S.cus = h->batch_cus;
+        S.state = 0;
+    }
+    if (S.state != 0) return MDX_OK;
+    S.state = -1;
     if (h->lds_sor_mode == 0) {
-        h->rb_note = "streaming sweeps: z-marching pairs, " + std::to_string(h->sweep_kz) + " planes per thread";
-        if (h->sweep_kz == 0) h->rb_note = "streaming sweeps: one cell per thread";
-        if (h->sweep_fused) h->rb_note = "fused red+black iterations: 32x8x8 tiles with a two-cell halo in LDS";
+        S.note = "streaming sweeps: z-marching pairs, " + std::to_string(h->sweep_kz) + " planes per thread";
+        if (h->sweep_kz == 0) S.note = "streaming sweeps: one cell per thread";
+        if (h->sweep_fused) S.note = "fused red+black iterations: 32x8x8 tiles with a two-cell halo in LDS";
         return MDX_OK;
     }
-    if (h->ibm_on && !h->coef_plane) { h->rb_note = "streaming sweeps: IBM coefficients vary in z"; return MDX_OK; }
+    if (h->lds_timeouts >= LDS_TIMEOUT_MAX) { lds_off(h); return MDX_OK; }
+    if (h->ibm_on && !h->coef_plane) { S.note = "streaming sweeps: IBM coefficients vary in z"; return MDX_OK; }
     RbPlanOut p64{}, p32{};
     std::string why;
-    if (!rb_plan(h, true, p32, why)) {
-        h->rb_note = "streaming sweeps: " + why;
+    if (!rb_plan(h, true, S.cus, p32, why)) {
+        S.note = "streaming sweeps: " + why;
         return MDX_OK;
     }
-    std::string note64;
-    if (h->lds_sor_mode == 2 && !rb_plan(h, false, p64, why)) {
-        h->lds_sor_mode = 1;   // FP64 batches stay on the streaming sweeps
-        note64 = "; fp64: streaming (" + why + ")";
-    }
+    // (without a plan FP64 batches stay on the streaming sweeps)
+    S.fp64 = h->lds_sor_mode == 2 && rb_plan(h, false, S.cus, p64, why);
     auto desc = [](const RbPlanOut &p) {
         return std::to_string(p.px) + "x" + std::to_string(p.py) + "x" + std::to_string(p.pz) + " workgroups of " +
                std::to_string(p.bx) + "x" + std::to_string(p.by) + "x" + std::to_string(p.bz) + " cells (" +
                (p.maxp == -1 ? "a z-column per thread" : (p.maxp == -2 ? "half a z-column per thread" : "x-pairs")) + "), LDS " + std::to_string(p.lds) + " B";
     };
-    h->rb_note = "LDS-resident sweeps (two-deep halo, one exchange per iteration): fp32 " + desc(p32);
-    if (h->lds_sor_mode == 2) h->rb_note += "; fp64 " + desc(p64);
-    else if (!note64.empty()) h->rb_note += note64;
-    else h->rb_note += "; fp64: streaming z-marching pairs, " + std::to_string(h->sweep_kz) + " planes per thread";
-    size_t need = rb_faces_bytes(p32, true);
-    if (h->lds_sor_mode == 2) need = std::max(need, rb_faces_bytes(p64, false));
-    if (h->rb_faces) { (void)hipFree(h->rb_faces); h->rb_faces = nullptr; }
-    MDX_HIP(hipMalloc(&h->rb_faces, need));
-    MDX_HIP(hipMemset(h->rb_faces, 0, need));   // tag 0 is never published
-    h->rb_faces_bytes = need;
-    for (int **xl : {&h->rb_xl32, &h->rb_xl64})
-        if (*xl) { (void)hipFree(*xl); *xl = nullptr; }
-    MDX_HIP(hipMalloc(&h->rb_xl32, rb_xlist_bytes(p32)));
-    MDX_HIP(rb_build_xlists(h, p32, true, h->rb_xl32));
-    if (h->lds_sor_mode == 2) {
-        MDX_HIP(hipMalloc(&h->rb_xl64, rb_xlist_bytes(p64)));
-        MDX_HIP(rb_build_xlists(h, p64, false, h->rb_xl64));
+    S.note = "LDS-resident sweeps (two-deep halo, one exchange per iteration): fp32 " + desc(p32);
+    if (S.fp64) S.note += "; fp64 " + desc(p64);
+    else if (h->lds_sor_mode == 2) S.note += "; fp64: streaming (" + why + ")";
+    else S.note += "; fp64: streaming z-marching pairs, " + std::to_string(h->sweep_kz) + " planes per thread";
+    S.faces_bytes = rb_faces_bytes(p32, true);
+    if (S.fp64) S.faces_bytes = std::max(S.faces_bytes, rb_faces_bytes(p64, false));
+    const size_t x32 = rb_xlist_bytes(p32), x64 = S.fp64 ? rb_xlist_bytes(p64) : 0, need = S.faces_bytes + x32 + x64;
+    if (S.mem_bytes < need) {
+        if (S.mem) { (void)hipFree(S.mem); S.mem = nullptr; }
+        S.mem_bytes = 0;
+        const hipError_t e = hipMalloc(&S.mem, need);
+        if (e == hipErrorOutOfMemory) {   // the streaming sweeps need none of it
+            (void)hipGetLastError();
+            S.mem = nullptr;
+            S.note = "streaming sweeps: no memory for the face buffers (" + std::to_string(need) + " B)";
+            return MDX_OK;
+        }
+        MDX_HIP(e);
+        S.mem_bytes = need;
     }
-    h->rb_tag = 0;
-    h->rb_plan64 = p64;
-    h->rb_plan32 = p32;
-    h->rb_state = 1;
+    MDX_HIP(hipMemsetAsync(S.mem, 0, S.faces_bytes, h->stream));   // tag 0 is never published
+    S.xl32 = reinterpret_cast<int *>(static_cast<char *>(S.mem) + S.faces_bytes);
+    S.xl64 = S.xl32 + x32 / sizeof(int);
+    MDX_HIP(rb_build_xlists(h, p32, true, S.xl32));
+    if (S.fp64) MDX_HIP(rb_build_xlists(h, p64, false, S.xl64));
+    S.tag = 0;
+    S.plan64 = p64;
+    S.plan32 = p32;
+    S.state = 1;
     return MDX_OK;
 }
 
@@ -971,7 +994,7 @@ static hipError_t sweep_launches(mdx_handle *h, bool fp32, int m) {
 
 // whether batches of this precision run on the LDS-resident solver
 static bool lds_for(const mdx_handle *h, bool fp32) {
-    return h->rb_state == 1 && !h->lds_suspended && (fp32 || h->lds_sor_mode == 2);
+    return h->rb->state == 1 && !h->lds_suspended && (fp32 || h->rb->fp64);
 }
 
 // sweep counters: account finished batches in order (end event complete; `wait`: block for them)
@@ -1010,8 +1033,8 @@ static int sweep_batch(mdx_handle *h, bool fp32, int m, const RbDefect *df = nul
             // the runtime refused the launch (nothing ran): use the streaming sweeps
             (void)hipGetLastError();
             launches = 0;
-            h->rb_state = -1;
-            h->rb_note = std::string("streaming sweeps: LDS-resident launch refused (") + hipGetErrorString(e) + ")";
+            h->rb->state = -1;
+            h->rb->note = std::string("streaming sweeps: LDS-resident launch refused (") + hipGetErrorString(e) + ")";
             if (fp32) MDX_HIP(launch_zero32(h, h->e32, h->ni));   // the streaming sweeps start from e = 0
             // the streaming FP64 sweeps change Phi whatever the pending check says
             else if (df && df->skip) return MDX_LDS_REFUSED;
@@ -1630,7 +1653,7 @@ extern "C" int mdx_pressure_projection(mdx_handle *h, double dtg, mdx_solve_stat
         if (rc) return rc;
         if ((rc = rb_prepare(h))) return rc;
         LdsTurn turn;   // held until this solve has read its last check
-        h->lds_suspended = h->rb_state == 1 && (h->in_batch ? !h->batch_lds : !turn.take(h->device));
+        h->lds_suspended = h->rb->state == 1 && (h->in_batch ? !h->batch_lds : !turn.take(h->device));
         double r_first = -1.0;
         const int stage = (int)(h->proj_count % 3);
         const auto t_plan = std::chrono::steady_clock::now();
@@ -1685,11 +1708,7 @@ extern "C" int mdx_pressure_projection(mdx_handle *h, double dtg, mdx_solve_stat
             // tries the LDS-resident sweeps again (for good off after LDS_TIMEOUT_MAX restarts)
             h->lds_timeouts += 1;
             h->lds_suspended = true;
-            if (h->lds_timeouts >= LDS_TIMEOUT_MAX) {
-                h->rb_state = -1;
-                h->rb_note = "streaming sweeps: neighbour waits of the LDS-resident sweeps gave up " +
-                             std::to_string(h->lds_timeouts) + " times";
-            }
+            if (h->lds_timeouts >= LDS_TIMEOUT_MAX) lds_off(h);
             const int learned_mode = c.guess == MDX_GUESS_LEARNED;
             st = mdx_solve_stats{};
             st.lds_restarts = 1;
@@ -1919,10 +1938,7 @@ extern "C" int mdx_step_batch(mdx_handle *const *hs, int32_t n, double dt, mdx_s
             cus = 0;   // no share: the streaming sweeps
         }
         const int share = cus / n;
-        if (h->rb_cus == 0 || h->rb_cus > std::max(1, share)) {
-            h->rb_cus = std::max(1, share);
-            h->rb_state = 0;   // planned again on its share
-        }
+        h->batch_cus = std::max(1, share);
         int first = q;   // the handle that took (or failed to take) the turn of this device
         for (int r = 0; r < q; ++r)
             if (hs[r]->device == h->device) { first = r; break; }
@@ -1980,7 +1996,7 @@ extern "C" int mdx_get_info(mdx_handle *h, char *buf, int32_t len) {
     MDX_CHECK(h && buf && len > 0, MDX_ERR_ARG, "mdx_get_info: bad argument");
     std::string s = h->cfg.solver == MDX_SOLVER_FFT ? "FFT/tridiagonal pressure solve"
                     : h->cfg.solver == MDX_SOLVER_SOLA ? "SOLA red-black sweeps (fixed niter)"
-                    : (h->rb_note.empty() ? "red-black SOR (not yet planned)" : h->rb_note);
+                    : (h->rb->note.empty() ? "red-black SOR (not yet planned)" : h->rb->note);
     std::snprintf(buf, (size_t)len, "%s", s.c_str());
     return MDX_OK;
 }

@@ -176,6 +176,21 @@ struct RbPlanOut {
     int px, py, pz, bx, by, bz, maxp;
     size_t lds;
     int total;   // halo values exchanged per workgroup and iteration
+    int groups() const { return px * py * pz; }
+};
+
+// The LDS-resident sweeps on a number of CUs: the plans of both precisions, their exchange lists and
+// the tagged face buffers (one allocation), kept until the body or the number of CUs changes.
+struct RbSet {
+    int cus = 0;                   // CUs the plans may hold (0: all of the device's)
+    int state = 0;                 // 0 not planned, 1 ready, -1 unavailable
+    bool fp64 = false;             // FP64 batches have a plan too
+    RbPlanOut plan64{}, plan32{};
+    void *mem = nullptr;           // the faces, then the exchange lists
+    size_t mem_bytes = 0, faces_bytes = 0;
+    int *xl32 = nullptr, *xl64 = nullptr;
+    unsigned long long tag = 0;    // half-sweeps published so far (the tag of the last one)
+    std::string note;              // why the streaming sweeps are in use, or the chosen plan
 };
 
 }  // namespace mdx
@@ -291,9 +306,8 @@ struct mdx_handle {
     bool sweep_fused = false;
 
     // LDS-resident red-black solver (MOBYDIFF_LDS_SOR): 0 off, 1 FP32 sweep batches, 2 FP32 and FP64
-    // batches (the default); plans per precision and the tagged face buffers
+    // batches (the default)
     int lds_sor_mode = 2;
-    int rb_cus = 0;                // CUs the plan may hold (0: all of the device's)
     // launch the LDS-resident kernel through hipLaunchCooperativeKernel (MOBYDIFF_LDS_COOP=1)
     // instead of an ordinary launch of a grid that the plan already sized to be co-resident
     bool rb_coop = false;
@@ -316,7 +330,9 @@ struct mdx_handle {
     // 12; MOBYDIFF_MOM_KZ)
     int mom_kz = 8;
     bool mom_fixed = false;   // MOBYDIFF_MOM_KZ: on every grid
-    int rb_state = 0;              // 0 not planned, 1 ready, -1 unavailable
+    // plans for the handle stepped alone ([0], all CUs) and for mdx_step_batch ([1], the share of
+    // its last batch), and the one in use
+    mdx::RbSet rb_sets[2], *rb = &rb_sets[0];
     // polls of a neighbour wait before it gives up (MOBYDIFF_LDS_SPIN_LIMIT; a test hook); a wait
     // that gives up sets the error word, the batch drains, and the solve restarts on the
     // streaming sweeps (lds_suspended for the rest of that solve; after LDS_TIMEOUT_MAX such
@@ -324,16 +340,11 @@ struct mdx_handle {
     int rb_spin_limit = 1 << 20;
     int lds_timeouts = 0;
     bool lds_suspended = false;
-    // the handle is being stepped by mdx_step_batch, which holds the device's LDS turn for all of
-    // its handles (or, with batch_lds false, could not take it)
+    // the handle is being stepped by mdx_step_batch on batch_cus CUs; the batch holds the device's
+    // LDS turn for all of its handles (or, with batch_lds false, could not take it)
     bool in_batch = false, batch_lds = false;
-    mdx::RbPlanOut rb_plan64{}, rb_plan32{};
-    void *rb_faces = nullptr;      // tagged face words of the LDS-resident sweeps
-    int *rb_xl32 = nullptr, *rb_xl64 = nullptr;   // exchange lists of the two plans
-    size_t rb_faces_bytes = 0;
+    int batch_cus = 0;
     int *rb_err = nullptr;         // points into red_max[1]
-    unsigned long long rb_tag = 0; // half-sweeps published so far (the tag of the last one)
-    std::string rb_note;           // why the streaming sweeps are in use, or the chosen plan
 
     // learned guess (attached network) and training-pair capture
     struct mdx_net *net = nullptr;
@@ -473,7 +484,8 @@ hipError_t launch_learned_input(mdx_handle *h, const double *prev, double fac, d
 // check in max_part, posted to rg_slot
 hipError_t launch_select_start(mdx_handle *h, double margin, unsigned nb, double *rg_slot, const double *other_slot,
                                const double *phi0, const double *res0, double *host_slot, unsigned long long seq);
-bool rb_plan(const mdx_handle *h, bool fp32, RbPlanOut &out, std::string &why);
+// the decomposition for `cus` of the device's CUs (0: all of them)
+bool rb_plan(const mdx_handle *h, bool fp32, int cus, RbPlanOut &out, std::string &why);
 // check epilogue of an LDS batch: FP32 phi_out = phi_in + e, r32 = defect; FP64 phi_out = the iterate
 // (phi_in unused); the maximum to the slot
 struct RbDefect {

@@ -1088,11 +1088,11 @@ static int rb_occupancy(bool fp32, bool ibm, int maxp, bool stretch, size_t lds)
     return nb;
 }
 
-// Choose the decomposition: every workgroup co-resident (runtime occupancy) on the handle's CUs,
+// Choose the decomposition: every workgroup co-resident (runtime occupancy) on `share` CUs (0: all),
 // the fewest cells per CU, then the smallest exchange.  The half-column form takes any cut of the
 // grid into parts of at least 4 cells (rb_part); the pair and whole-column forms, whose lists are
 // sized by one shape, need equal even parts.  `why` receives the reason when nothing fits.
-bool rb_plan(const mdx_handle *h, bool fp32, RbPlanOut &out, std::string &why) {
+bool rb_plan(const mdx_handle *h, bool fp32, int share, RbPlanOut &out, std::string &why) {
     const int nx = h->d.nx, ny = h->d.ny, nz = h->d.nz;
     // single attributes: reading all device properties takes longer than the search below
     auto attr = [&](hipDeviceAttribute_t a) {
@@ -1108,7 +1108,7 @@ bool rb_plan(const mdx_handle *h, bool fp32, RbPlanOut &out, std::string &why) {
         return false;
     }
     if (h->cfg.periodic[1] && ny % 2) { why = "odd periodic y"; return false; }
-    const int cus = h->rb_cus > 0 ? std::min(h->rb_cus, all_cus) : all_cus;
+    const int cus = share > 0 ? std::min(share, all_cus) : all_cus;
     const size_t lds_max = (size_t)std::max(lds_cu, lds_block);
     const size_t ts = fp32 ? 4 : 8;
     bool found = false;
@@ -1189,6 +1189,7 @@ size_t rb_faces_bytes(const RbPlanOut &p, bool fp32) {
 template <typename T>
 static hipError_t rb_launch_t(mdx_handle *h, const RbPlanOut &pl, T *x, const T *rhs, int zero_init, int iters,
                               T *const *mu, const RbDefect *df) {
+    RbSet &S = *h->rb;
     RbArgs<T> a;
     a.defect = df != nullptr;
     a.g = grid_k(h);
@@ -1232,18 +1233,18 @@ static hipError_t rb_launch_t(mdx_handle *h, const RbPlanOut &pl, T *x, const T 
                   dpz = pl.bz > 2 ? pl.bz - 2 : 0;
         a.md = (dpx * dpy * dpz / RB_THREADS) / RB_G * RB_G;   // whole relax groups only
     }
-    a.faces = reinterpret_cast<unsigned long long *>(h->rb_faces);
+    a.faces = reinterpret_cast<unsigned long long *>(S.mem);
     a.total = pl.total;
-    a.xl = sizeof(T) == 4 ? h->rb_xl32 : h->rb_xl64;
-    // tags of this launch: rb_tag + 1 .. rb_tag + iters + 1 (the last for the maxima); before the
+    a.xl = sizeof(T) == 4 ? S.xl32 : S.xl64;
+    // tags of this launch: tag + 1 .. tag + iters + 1 (the last for the maxima); before the
     // 32-bit tag would wrap to 0 the face buffer is cleared and the count restarts
-    if (h->rb_tag + (unsigned long long)iters + 2ull > 0xffffffffull) {
-        hipError_t e = hipMemsetAsync(h->rb_faces, 0, h->rb_faces_bytes, h->stream);
+    if (S.tag + (unsigned long long)iters + 2ull > 0xffffffffull) {
+        hipError_t e = hipMemsetAsync(S.mem, 0, S.faces_bytes, h->stream);
         if (e != hipSuccess) return e;
-        h->rb_tag = 0;
+        S.tag = 0;
     }
-    a.tag0 = (unsigned)h->rb_tag;
-    h->rb_tag += (unsigned long long)iters + 1ull;
+    a.tag0 = (unsigned)S.tag;
+    S.tag += (unsigned long long)iters + 1ull;
     a.err = h->rb_err;
     a.spin_limit = h->rb_spin_limit;
     const void *fn = h->ibm_on ? rb_fn_for<T, true>(pl.maxp, h->stretched) : rb_fn_for<T, false>(pl.maxp, h->stretched);
@@ -1263,7 +1264,7 @@ static hipError_t rb_launch_t(mdx_handle *h, const RbPlanOut &pl, T *x, const T 
 }
 
 hipError_t launch_rb_lds(mdx_handle *h, bool fp32, int iters, int zero_init, const RbDefect *df) {
-    const RbPlanOut &pl = fp32 ? h->rb_plan32 : h->rb_plan64;
+    const RbPlanOut &pl = fp32 ? h->rb->plan32 : h->rb->plan64;
     if (fp32) return rb_launch_t<float>(h, pl, h->e32, h->r32, zero_init, iters, h->mu32, df);
     return rb_launch_t<double>(h, pl, h->phi, h->rhs, zero_init, iters, h->mu64, df);
 }

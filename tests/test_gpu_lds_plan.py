@@ -33,3 +33,76 @@ def test_first_solve_is_not_slowed_by_the_search():
     extra = min(a - b for a, b in (_first_and_later((512, 256, 256)) for _ in range(2)))
     print("first solve: +%.2f ms" % extra, flush=True)
     assert extra < 2.0
+
+
+def _channels(shape, n, **kw):
+    kw = dict(dict(solver=M.SOLVER_SOR, omega=1.8, tol=1e-7, check_every=20, max_iter=40, inner_iters=20), **kw)
+    chs = []
+    for q in range(n):
+        ch = M.Channel(M.channel_config(*shape, 4.0, 2.0, 2.0, 2000.0, **kw))
+        ch.init_fields(seed=q, amp=0.05, dt=5e-4)
+        chs.append(ch)
+    return chs
+
+
+def _lds(stats):
+    return [stats.stage[q].lds_sweeps for q in range(3)]
+
+
+def test_a_batch_leaves_the_plan_of_single_steps():
+    """FP64 at 160 x 128 x 96: the sweeps fit the whole device's LDS, not half of it.  A batch of two
+    runs on the streaming sweeps, and each channel stepped alone before and after it on the same
+    whole-device plan; the same for a smaller grid, whose batch has plans of its own."""
+    dt = 5e-4
+    for shape, batched in (((160, 128, 96), 0), ((48, 32, 24), 1)):
+        chs = _channels(shape, 2)
+        assert _lds(chs[0].step(dt)) == [1, 1, 1], chs[0].info()
+        alone = chs[0].info()
+        for _ in range(2):
+            stats = M.step_batch(chs, dt)
+            assert [_lds(s) for s in stats] == [[batched] * 3] * 2, [ch.info() for ch in chs]
+            assert chs[0].info() != alone
+            assert _lds(chs[0].step(dt)) == [1, 1, 1], chs[0].info()
+            assert chs[0].info() == alone
+        for ch in chs:
+            ch.close()
+
+
+@pytest.mark.parametrize("precision", [M.PREC_FP64, M.PREC_MIXED])
+def test_single_and_batched_steps_give_the_same_bits(precision):
+    dt, shape = 5e-4, (48, 33, 26)
+    outs = []
+    for batched in ((0, 1, 0, 1, 1, 0), (0,) * 6):
+        chs = _channels(shape, 3, precision=precision, max_iter=100000)
+        for b in batched:
+            if b:
+                M.step_batch(chs, dt)
+            else:
+                for ch in chs:
+                    ch.step(dt)
+        outs.append([ch.download(("un", "vn", "wn", "pn")) for ch in chs])
+        for ch in chs:
+            ch.close()
+    for a, b in zip(*outs):
+        for k in a:
+            assert np.array_equal(a[k], b[k]), k
+
+
+def test_a_timed_out_handle_stays_off_in_a_batch(monkeypatch):
+    """After three solves whose neighbour waits gave up (a spin limit of 0 polls, set from the host) a
+    handle keeps to the streaming sweeps, in a batch too."""
+    monkeypatch.setenv("MOBYDIFF_LDS_SPIN_LIMIT", "0")
+    chs = _channels((96, 64, 48), 2)
+    off = lambda ch: "gave up 3 times" in ch.info()
+    for ch in chs:
+        for _ in range(10):
+            if not off(ch):
+                ch.step(5e-4)
+    if not all(off(ch) for ch in chs):
+        pytest.skip("the neighbours had always published")
+    for _ in range(2):
+        for s in M.step_batch(chs, 5e-4):
+            assert _lds(s) == [0, 0, 0] and all(s.stage[q].lds_restarts == 0 for q in range(3))
+    assert all(off(ch) for ch in chs)
+    for ch in chs:
+        ch.close()

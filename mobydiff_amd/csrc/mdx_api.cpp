@@ -851,9 +851,10 @@ public:
 // steps of its own and one for its share of a batch, so that stepping it one way costs the other
 // nothing.
 static int rb_prepare(mdx_handle *h) {
-    RbSet &S = h->rb_sets[h->in_batch ? 1 : 0];
+    const bool shared = h->in_batch && h->batch_cus > 0;
+    RbSet &S = h->rb_sets[shared ? 1 : 0];
     h->rb = &S;
-    if (h->in_batch && S.cus != h->batch_cus) {
+    if (shared && S.cus != h->batch_cus) {
         S.cus = h->batch_cus;
         S.state = 0;
     }
@@ -1937,8 +1938,14 @@ extern "C" int mdx_step_batch(mdx_handle *const *hs, int32_t n, double dt, mdx_s
             (void)hipGetLastError();
             cus = 0;   // no share: the streaming sweeps
         }
-        const int share = cus / n;
-        h->batch_cus = std::max(1, share);
+        // An equal share of the device's CUs for each of its channels that sweep, the same number on
+        // every XCD: workgroups are dealt to the XCDs in turn, so a share of 85 CUs (three channels)
+        // would want 11 places on some XCDs, 33 of their 32 CUs, and two channels could each hold
+        // the place the other's last workgroup waits for.
+        auto sweeps = [&](const mdx_handle *r) { return r->device == h->device && r->cfg.solver == MDX_SOLVER_SOR; };
+        const int on_device = (int)std::count_if(hs, hs + n, sweeps);
+        const int share = on_device > 0 ? cus / RB_XCDS / on_device * RB_XCDS : 0;
+        h->batch_cus = on_device > 1 ? share : 0;   // (one alone has them all)
         int first = q;   // the handle that took (or failed to take) the turn of this device
         for (int r = 0; r < q; ++r)
             if (hs[r]->device == h->device) { first = r; break; }

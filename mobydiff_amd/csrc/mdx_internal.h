@@ -179,6 +179,9 @@ struct RbPlanOut {
     int groups() const { return px * py * pz; }
 };
 
+// XCDs of the device, to which the workgroups of a launch are dealt in turn
+static constexpr int RB_XCDS = 8;
+
 // The LDS-resident sweeps on a number of CUs: the plans of both precisions, their exchange lists and
 // the tagged face buffers (one allocation), kept until the body or the number of CUs changes.
 struct RbSet {
@@ -340,7 +343,7 @@ struct mdx_handle {
     int rb_spin_limit = 1 << 20;
     int lds_timeouts = 0;
     bool lds_suspended = false;
-    // the handle is being stepped by mdx_step_batch on batch_cus CUs; the batch holds the device's
+    // the handle is being stepped by mdx_step_batch on batch_cus CUs (0: all); the batch holds the device's
     // LDS turn for all of its handles (or, with batch_lds false, could not take it)
     bool in_batch = false, batch_lds = false;
     int batch_cus = 0;

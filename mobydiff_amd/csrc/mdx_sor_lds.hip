@@ -235,9 +235,9 @@ __global__ __launch_bounds__(FORM == 2 ? 2 * RB_THREADS : RB_THREADS) void rb_ld
     const int nwg = a.px * a.py * a.pz;
     // XCD-aware placement: workgroups are dispatched round-robin over the 8 XCDs, so consecutive
     // subdomain ids (neighbours along x first) are given to workgroups on the same XCD.
-    const int per_xcd = nwg / 8;
+    const int per_xcd = nwg / RB_XCDS;
     const int b = blockIdx.x;
-    const int w = (nwg % 8 == 0) ? (b % 8) * per_xcd + b / 8 : b;
+    const int w = (nwg % RB_XCDS == 0) ? (b % RB_XCDS) * per_xcd + b / RB_XCDS : b;
     const int wx = w % a.px, wy = (w / a.px) % a.py, wz = w / (a.px * a.py);
     int ox, oy, oz, bx, by, bz;   // this workgroup's subdomain
     rb_part(d.nx, a.px, wx, ox, bx);
@@ -1088,7 +1088,8 @@ static int rb_occupancy(bool fp32, bool ibm, int maxp, bool stretch, size_t lds)
     return nb;
 }
 
-// Choose the decomposition: every workgroup co-resident (runtime occupancy) on `share` CUs (0: all),
+// Choose the decomposition: every workgroup co-resident (runtime occupancy) on `share` CUs (0: all
+// of them, several workgroups on a CU where they fit),
 // the fewest cells per CU, then the smallest exchange.  The half-column form takes any cut of the
 // grid into parts of at least 4 cells (rb_part); the pair and whole-column forms, whose lists are
 // sized by one shape, need equal even parts.  `why` receives the reason when nothing fits.
@@ -1128,6 +1129,9 @@ bool rb_plan(const mdx_handle *h, bool fp32, int share, RbPlanOut &out, std::str
                 const int bz = rb_part_max(nz, pz);
                 if ((long)px * py * pz > max_wg) break;
                 const int nwg = px * py * pz;
+                // a share: a CU for every workgroup, so that no other launch's workgroups, however
+                // they are spread, take the place one of these waits for
+                if (share > 0 && nwg > cus) break;
                 const bool equal = (nx / 2) % px == 0 && ny % 2 == 0 && (ny / 2) % py == 0 && (nz / 2) % pz == 0;
                 // the column form where a thread per column (subdomain and face ring) fits
                 const bool colfit = bx * by + 2 * (bx + by) <= RB_THREADS && rb_part_min(nx, px) >= 4 &&

@@ -106,3 +106,31 @@ def test_a_timed_out_handle_stays_off_in_a_batch(monkeypatch):
     assert all(off(ch) for ch in chs)
     for ch in chs:
         ch.close()
+
+
+@pytest.mark.parametrize("n", [2, 3, 5, 7])
+def test_shares_fit_every_xcd(n):
+    """The plans of a batch of n on the eight XCDs of 32 CUs, to which a launch's workgroups are dealt
+    in turn: all of them have a CU of their own at once.  For three of 20 x 18 x 28 cells the third of
+    256 CUs would hold 84 workgroups, 11 on an XCD and 33 for all three.  Same bits as alone, no
+    restart."""
+    shape, dt = (20, 18, 28), 5e-4
+    outs = []
+    for batched in (True, False):
+        chs = _channels(shape, n, max_iter=100000)
+        for _ in range(2):
+            stats = M.step_batch(chs, dt) if batched else [ch.step(dt) for ch in chs]
+            assert all(_lds(s) == [1, 1, 1] for s in stats), chs[0].info()
+            assert sum(s.stage[q].lds_restarts for s in stats for q in range(3)) == 0
+        if batched:
+            print(n, chs[0].info(), flush=True)
+            for ch in chs:
+                cuts = [int(np.prod([int(v) for v in part.split(" workgroups")[0].split()[-1].split("x")]))
+                        for part in ch.info().split("; ")]
+                assert len(cuts) == 2 and all(n * -(-c // 8) <= 32 for c in cuts), ch.info()
+        outs.append([ch.download(("un", "vn", "wn", "pn")) for ch in chs])
+        for ch in chs:
+            ch.close()
+    for a, b in zip(*outs):
+        for k in a:
+            assert np.array_equal(a[k], b[k]), k

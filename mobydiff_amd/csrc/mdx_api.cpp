@@ -821,28 +821,35 @@ static int read_norm(mdx_handle *h, double *out) {
 }
 
 // The LDS-resident solver's workgroups wait for each other, so two of its batches that share the
-// device's CUs could hold each other up until their waits give up.  A device has one turn: a solve
-// (or an mdx_step_batch call, for all of its handles, whose plans share the CUs out) that finds it
-// taken by another thread runs on the streaming sweeps, which give the same bits.  When a turn
-// ends no batch of it still waits: the last check has been read, and a batch queued behind it
-// finds it converged and returns.
+// device's CUs could hold each other up until their waits give up.  Solves therefore take the places
+// their plan needs, counted as CUs of one XCD (workgroups are dealt to the XCDs in turn), from a
+// budget per device: solves of several threads run side by side while a CU is left for every
+// workgroup of theirs, and one that finds too few places runs on the streaming sweeps, which give
+// the same bits.  When a turn ends no batch of it still waits: the last check has been read, and a
+// batch queued behind it finds it converged and returns.
 static constexpr int LDS_MAX_DEVICES = 64;
-static std::atomic<bool> g_lds_turn[LDS_MAX_DEVICES];
+static std::atomic<int> g_lds_places[LDS_MAX_DEVICES];   // taken
 
 class LdsTurn {
-    int dev_ = -1;
+    int dev_ = -1, places_ = 0;
 
 public:
     LdsTurn() = default;
     LdsTurn(const LdsTurn &) = delete;
     LdsTurn &operator=(const LdsTurn &) = delete;
-    bool take(int dev) {
-        if (dev < 0 || dev >= LDS_MAX_DEVICES || g_lds_turn[dev].exchange(true, std::memory_order_acquire)) return false;
+    bool take(int dev, int places, int all) {
+        if (dev < 0 || dev >= LDS_MAX_DEVICES) return false;
+        int used = g_lds_places[dev].load(std::memory_order_relaxed);
+        do {
+            if (used + places > all) return false;
+        } while (!g_lds_places[dev].compare_exchange_weak(used, used + places, std::memory_order_acquire,
+                                                          std::memory_order_relaxed));
         dev_ = dev;
+        places_ = places;
         return true;
     }
     ~LdsTurn() {
-        if (dev_ >= 0) g_lds_turn[dev_].store(false, std::memory_order_release);
+        if (dev_ >= 0) g_lds_places[dev_].fetch_sub(places_, std::memory_order_release);
     }
 };
 
@@ -851,7 +858,7 @@ public:
 // steps of its own and one for its share of a batch, so that stepping it one way costs the other
 // nothing.
 static int rb_prepare(mdx_handle *h) {
-    const bool shared = h->in_batch && h->batch_cus > 0;
+    const bool shared = h->batch_cus > 0;
     RbSet &S = h->rb_sets[shared ? 1 : 0];
     h->rb = &S;
     if (shared && S.cus != h->batch_cus) {
@@ -909,6 +916,12 @@ static int rb_prepare(mdx_handle *h) {
     S.tag = 0;
     S.plan64 = p64;
     S.plan32 = p32;
+    int cus = 0;
+    MDX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device));
+    // (several workgroups on a CU: the device to itself)
+    const int groups = (h->cfg.precision == MDX_PREC_MIXED ? p32 : p64).groups();
+    S.all_places = std::max(1, cus / RB_XCDS);
+    S.places = groups > cus ? S.all_places : std::min(S.all_places, (groups + RB_XCDS - 1) / RB_XCDS);
     S.state = 1;
     return MDX_OK;
 }
@@ -1654,7 +1667,9 @@ extern "C" int mdx_pressure_projection(mdx_handle *h, double dtg, mdx_solve_stat
         if (rc) return rc;
         if ((rc = rb_prepare(h))) return rc;
         LdsTurn turn;   // held until this solve has read its last check
-        h->lds_suspended = h->rb->state == 1 && (h->in_batch ? !h->batch_lds : !turn.take(h->device));
+        h->lds_suspended = false;
+        if (lds_for(h, c.precision == MDX_PREC_MIXED))
+            h->lds_suspended = !turn.take(h->device, h->rb->places, h->rb->all_places);
         double r_first = -1.0;
         const int stage = (int)(h->proj_count % 3);
         const auto t_plan = std::chrono::steady_clock::now();
@@ -1930,13 +1945,12 @@ extern "C" int mdx_step_batch(mdx_handle *const *hs, int32_t n, double dt, mdx_s
                       "mdx_step_batch: two handles share one attached network");
         }
     }
-    std::vector<LdsTurn> turns(n);
     for (int q = 0; q < n; ++q) {
         mdx_handle *h = hs[q];
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) {
             (void)hipGetLastError();
-            cus = 0;   // no share: the streaming sweeps
+            cus = 0;
         }
         // An equal share of the device's CUs for each of its channels that sweep, the same number on
         // every XCD: workgroups are dealt to the XCDs in turn, so a share of 85 CUs (three channels)
@@ -1944,13 +1958,8 @@ extern "C" int mdx_step_batch(mdx_handle *const *hs, int32_t n, double dt, mdx_s
         // the place the other's last workgroup waits for.
         auto sweeps = [&](const mdx_handle *r) { return r->device == h->device && r->cfg.solver == MDX_SOLVER_SOR; };
         const int on_device = (int)std::count_if(hs, hs + n, sweeps);
-        const int share = on_device > 0 ? cus / RB_XCDS / on_device * RB_XCDS : 0;
-        h->batch_cus = on_device > 1 ? share : 0;   // (one alone has them all)
-        int first = q;   // the handle that took (or failed to take) the turn of this device
-        for (int r = 0; r < q; ++r)
-            if (hs[r]->device == h->device) { first = r; break; }
-        h->in_batch = true;
-        h->batch_lds = share > 0 && (first < q ? hs[first]->batch_lds : turns[q].take(h->device));
+        // (more channels than CUs on an XCD take turns; one alone has all CUs)
+        h->batch_cus = on_device > 1 ? std::max(1, cus / RB_XCDS / on_device) * RB_XCDS : 0;
     }
     std::vector<int> rc(n, MDX_OK);
     std::vector<std::string> err(n);
@@ -1967,7 +1976,7 @@ extern "C" int mdx_step_batch(mdx_handle *const *hs, int32_t n, double dt, mdx_s
             if (rc[q]) err[q] = mdx_last_error();
         });
     for (auto &t : th) t.join();
-    for (int q = 0; q < n; ++q) hs[q]->in_batch = false;
+    for (int q = 0; q < n; ++q) hs[q]->batch_cus = 0;
     for (int q = 0; q < n; ++q)
         if (rc[q]) {
             mdx_set_error("mdx_step_batch: instance " + std::to_string(q) + ": " + err[q]);

@@ -188,6 +188,7 @@ struct RbSet {
     int cus = 0;                   // CUs the plans may hold (0: all of the device's)
     int state = 0;                 // 0 not planned, 1 ready, -1 unavailable
     bool fp64 = false;             // FP64 batches have a plan too
+    int places = 0, all_places = 0;   // CUs of an XCD that a solve's workgroups take, of how many
     RbPlanOut plan64{}, plan32{};
     void *mem = nullptr;           // the faces, then the exchange lists
     size_t mem_bytes = 0, faces_bytes = 0;
@@ -343,9 +344,7 @@ struct mdx_handle {
     int rb_spin_limit = 1 << 20;
     int lds_timeouts = 0;
     bool lds_suspended = false;
-    // the handle is being stepped by mdx_step_batch on batch_cus CUs (0: all); the batch holds the device's
-    // LDS turn for all of its handles (or, with batch_lds false, could not take it)
-    bool in_batch = false, batch_lds = false;
+    // while mdx_step_batch steps the handle: its share of the CUs (0: all of them)
     int batch_cus = 0;
     int *rb_err = nullptr;         // points into red_max[1]
 

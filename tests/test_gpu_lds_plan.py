@@ -1,5 +1,6 @@
 """Plans of the LDS-resident sweeps: what the first solve on a handle pays for its plan, and which plan
 a handle runs on when it is stepped alone and in batches in turn."""
+import threading
 import time
 
 import numpy as np
@@ -132,5 +133,40 @@ def test_shares_fit_every_xcd(n):
         for ch in chs:
             ch.close()
     for a, b in zip(*outs):
+        for k in a:
+            assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("precision", [M.PREC_FP64, M.PREC_MIXED])
+def test_threads_share_the_device_where_their_workgroups_fit(precision):
+    """Three channels of 64 workgroups (16^3 cells) stepped by three threads: a CU for each of their 192
+    workgroups, so every solve of each stays on the LDS-resident sweeps, with the bits it has alone."""
+    dt, steps = 5e-4, 12
+
+    def run(together):
+        chs = _channels((16, 16, 16), 3, precision=precision, max_iter=100000)
+        lds = [[] for _ in chs]
+
+        def work(q):
+            for _ in range(steps):
+                st = chs[q].step(dt)
+                lds[q] += _lds(st) + [1 - st.stage[s].lds_restarts for s in range(3)]
+
+        th = [threading.Thread(target=work, args=(q,)) for q in range(3)]
+        for t in th:
+            t.start()
+            if not together:
+                t.join()
+        for t in th:
+            t.join()
+        out = [ch.download(("un", "vn", "wn", "pn")) for ch in chs]
+        print(precision, chs[0].info(), [sum(v) for v in lds], flush=True)
+        for ch in chs:
+            ch.close()
+        return lds, out
+
+    (lds, out), (_, alone) = run(True), run(False)
+    assert all(v == [1] * (6 * steps) for v in lds)
+    for a, b in zip(out, alone):
         for k in a:
             assert np.array_equal(a[k], b[k]), k

@@ -1695,8 +1695,10 @@ extern "C" int mdx_pressure_projection(mdx_handle *h, double dtg, mdx_solve_stat
                 // again: the solve queues its first batch (inner_iters, the network start's first
                 // batch) behind the choice and learns which start ran from the first check.  Else
                 // the choice is read first, so the batches are those of the start that runs (a
-                // fallback solve is then the other mode's solve exactly).
-                defer = rc == MDX_OK && h->defer_choice && h->net_prev_started[stage] && lds_for(h, true);
+                // fallback solve is then the other mode's solve exactly).  The schedule does not
+                // depend on the sweeps: a solve that streams (its places taken, no plan) has the
+                // same batches.
+                defer = rc == MDX_OK && h->defer_choice && h->net_prev_started[stage];
                 double r0 = 0.0;
                 if (rc == MDX_OK && !defer) rc = wait_check(h, CHECK_PIN, first_seq, &r0);
                 if (rc == MDX_OK && !defer) rc = resolve_learned_start(h, stage, gp, &st, &r_first);

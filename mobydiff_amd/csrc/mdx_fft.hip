@@ -1758,10 +1758,6 @@ static hipError_t launch_ixfft(mdx_handle *h, double *phi) {
 
 // the LDS a column may take
 static constexpr size_t COLUMN_LDS = 160 * 1024 - 1024;
-// Whether (2.) to (4.) go column by column in one launch: FP64 grids whose x-transforms take the
-// small workgroups, with a kx column in LDS.  A step against the three launches: 149 and 163 us at
-// 64^3, 227 and 250 at 128 x 97 x 64, 224 and 264 at 256 x 60 x 64, 110 and 129 at 32 x 24 x 32, 154 and
-// 160 at 16 x 96 x 64 (nine columns).
 template <int N, int M> static hipError_t column_solve(mdx_handle *h) {
     const Dims d = h->d;
     constexpr size_t lds = column_lds<N, M>();
@@ -1777,52 +1773,41 @@ template <int N, int M> static hipError_t column_solve(mdx_handle *h) {
     else if constexpr (CS_SEGS * (M - 1) >= 63) return launch(std::false_type{});
     else return d.ny < 64 ? launch(std::true_type{}) : launch(std::false_type{});
 }
-#define CS_ROWS(N, CALL)                                  \
-    do {                                                  \
-        const int m = (d.ny + CS_SEGS - 1) / CS_SEGS;     \
-        if (m <= 4) CALL(N, 4);                           \
-        if (m <= 8) CALL(N, 8);                           \
-        if (m <= 12) CALL(N, 12);                         \
-        if (m <= 13) CALL(N, 13);                         \
-        if (m <= 16) CALL(N, 16);                         \
-    } while (0)
+// Rows per segment: the fewest that reach ny (every further one is a step of all chains and a line of
+// LDS), from 4 to 16, what a thread's registers hold; the larger ones only where the column fits.
+template <int N, int M = 4> static bool column_fits(int m) {
+    if constexpr (M > 16 || column_lds<N, M>() > COLUMN_LDS) return false;
+    else return m <= M || column_fits<N, M + 1>(m);
+}
+template <int N, int M = 4> static hipError_t column_solve_rows(mdx_handle *h, int m) {
+    if constexpr (M > 16 || column_lds<N, M>() > COLUMN_LDS) return hipErrorInvalidValue;
+    else return m <= M ? column_solve<N, M>(h) : column_solve_rows<N, M + 1>(h, m);
+}
+// Whether (2.) to (4.) go column by column in one launch: FP64 grids whose x-transforms take the
+// small workgroups, with a kx column in LDS.  A step against the three launches: 128 and 163 us at
+// 64^3, 204 and 250 at 128 x 97 x 64, 219 and 246 at 128 x 120 x 64, 224 and 264 at 256 x 60 x 64, 110 and 129 at
+// 32 x 24 x 32, 154 and 160 at 16 x 96 x 64 (nine columns).
 static bool columns_fit(const mdx_handle *h) {
     const Dims d = h->d;
     if (!h->wave_tridiag || !h->part_tridiag || d.nx < 16 || d.nx > 256) return false;
-    bool small = false;
-#define CALL(N) { small = rf_small(rf_row_blocks<N, 256>(d)); break; }
-    switch (d.nx) {
-    case 16: CALL(16)
-    case 32: CALL(32)
-    case 64: CALL(64)
-    case 128: CALL(128)
-    default: CALL(256)
-    }
-#undef CALL
-    if (!small) return false;
-#define CALL(N, M) return column_lds<N, M>() <= COLUMN_LDS
+    const int lines = 256 * 16 / d.nx;   // RFft<nx, 256>::LPW
+    if (!rf_small((unsigned)((d.ny * d.nz / 2 + lines - 1) / lines))) return false;
+    const int m = (d.ny + CS_SEGS - 1) / CS_SEGS;
     switch (d.nz) {
-    case 32: CS_ROWS(32, CALL); break;
-    case 64: CS_ROWS(64, CALL); break;
-    case 128: CS_ROWS(128, CALL); break;
-    default: break;
+    case 32: return column_fits<32>(m);
+    case 64: return column_fits<64>(m);
+    case 128: return column_fits<128>(m);
+    default: return false;
     }
-#undef CALL
-    return false;
 }
 static hipError_t launch_columns(mdx_handle *h) {
-    const Dims d = h->d;
-#define CALL(N, M)                                                                       \
-    if constexpr (column_lds<N, M>() <= COLUMN_LDS) return column_solve<N, M>(h); \
-    else return hipErrorInvalidValue
-    switch (d.nz) {
-    case 32: CS_ROWS(32, CALL); break;
-    case 64: CS_ROWS(64, CALL); break;
-    case 128: CS_ROWS(128, CALL); break;
-    default: break;
+    const int m = (h->d.ny + CS_SEGS - 1) / CS_SEGS;
+    switch (h->d.nz) {
+    case 32: return column_solve_rows<32>(h, m);
+    case 64: return column_solve_rows<64>(h, m);
+    case 128: return column_solve_rows<128>(h, m);
+    default: return hipErrorInvalidValue;
     }
-#undef CALL
-    return hipErrorInvalidValue;
 }
 
 static hipError_t launch_ixfft_columns(mdx_handle *h, double *phi) {

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import mobydiff_amd as M
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +70,26 @@ def test_slow_modes_keep_their_digits(nz):
     rms = [float(np.sqrt((np.array(e, np.float64) ** 2).mean())) for e in (err, plain)]
     print(nz, rms, rms[0] / rms[1], flush=True)
     assert rms[0] < 2.6 * rms[1], rms
+
+
+@pytest.mark.parametrize("nz,rows", [(32, range(4, 18)), (64, range(4, 17)), (128, range(4, 9))])
+def test_every_segment_length_matches_the_oracle(nz, rows):
+    """ny at both edges of every number of rows per segment of the column solves, and past the last one
+    that fits (16 rows at nz = 32, 15 at 64, 7 at 128), against the oracle's projection."""
+    for m in rows:
+        for ny in (8 * m - 7, 8 * m):
+            print(nz, ny, flush=True)
+            g = O.Grid(16, ny, nz, lx=2.0, ly=2.0, lz=1.0, periodic=(1, 0, 1), beta=1.5 if m % 2 else None)
+            f = O.random_fields(g, np.random.default_rng(ny))
+            ch = M.Channel(M.channel_config(g.nx, ny, nz, g.lx, g.ly, g.lz, g.re, solver=M.SOLVER_FFT, p_neumann_y=False,
+                                            stretch_beta=g.beta or 0.0))
+            ch.upload(**f)
+            ch.apply_bc()
+            ch.pressure_projection(0.07)
+            out = ch.download(("un", "vn", "wn", "pn"))
+            ch.close()
+            O.apply_bc_fft(g, f)
+            O.projection_fft(g, f, None, 0.07)
+            for k in out:
+                a, b = out[k][1:-1, 1:-1, 1:-1], f[k][1:-1, 1:-1, 1:-1]
+                assert np.linalg.norm(a - b) < 1e-12 * np.linalg.norm(b), (k, ny)

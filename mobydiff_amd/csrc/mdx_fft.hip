@@ -1697,6 +1697,10 @@ static hipError_t launch_zfft(hipStream_t st, const Dims &d, C *hat, const C *tw
     return hipGetLastError();
 }
 
+// the x points of a column-solved grid
+static constexpr int COLUMN_NX = 256;
+
+// (TRK: into the transposed spectrum of the column solves)
 template <bool TRK> static hipError_t launch_rhs_xfft(mdx_handle *h, double dtg) {
     GridK g = grid_k(h);
     const Dims d = h->d;
@@ -1711,15 +1715,21 @@ template <bool TRK> static hipError_t launch_rhs_xfft(mdx_handle *h, double dtg)
             (double2 *)h->hat);                                                                                       \
     } while (0)
 #define XF(N)                                                  \
-    if (rf_small(rf_row_blocks<N, 256>(d))) {                  \
-        if (h->stretched) XF_(N, 64, 4, true);                 \
-        XF_(N, 64, 4, false);                                  \
+    if constexpr (!TRK || N <= COLUMN_NX) {                    \
+        if (TRK || rf_small(rf_row_blocks<N, 256>(d))) {       \
+            if (h->stretched) XF_(N, 64, 4, true);             \
+            XF_(N, 64, 4, false);                              \
+        }                                                      \
     }                                                          \
-    if (h->stretched) XF_(N, 256, 1, true);                    \
-    XF_(N, 256, 1, false)
+    if constexpr (!TRK) {                                      \
+        if (h->stretched) XF_(N, 256, 1, true);                \
+        XF_(N, 256, 1, false);                                 \
+    }                                                          \
+    break
     RF_SIZES(d.nx, XF)
 #undef XF
 #undef XF_
+    if (TRK) return hipErrorInvalidValue;   // (columns_fit)
     const int lines = rows_per_block(d.nx);
     const int nrows = d.ny * d.nz;
     const size_t shx = fft_lds<double2>(lines, d.nx, d.nx);
@@ -1789,7 +1799,7 @@ template <int N, int M = 4> static hipError_t column_solve_rows(mdx_handle *h, i
 // 32 x 24 x 32, 154 and 160 at 16 x 96 x 64 (nine columns).
 static bool columns_fit(const mdx_handle *h) {
     const Dims d = h->d;
-    if (!h->wave_tridiag || !h->part_tridiag || d.nx < 16 || d.nx > 256) return false;
+    if (!h->wave_tridiag || !h->part_tridiag || d.nx < 16 || d.nx > COLUMN_NX) return false;
     const int lines = 256 * 16 / d.nx;   // RFft<nx, 256>::LPW
     if (!rf_small((unsigned)((d.ny * d.nz / 2 + lines - 1) / lines))) return false;
     const int m = (d.ny + CS_SEGS - 1) / CS_SEGS;
@@ -1814,10 +1824,12 @@ static hipError_t launch_ixfft_columns(mdx_handle *h, double *phi) {
     const Dims d = h->d;
     const double scale = 1.0 / (double)(d.nx * d.nz);
 #define IX(N)                                                                                                       \
-    return rf_launch<double2, N, 64, ixfft_columns_kernel<N, 64, 4>, 4>(h->stream, rf_row_blocks<N, 64>(d), d,      \
-                                                                        (const double2 *)h->hat,                    \
-                                                                        (const double2 *)h->tw_x, d.ny * d.nz,      \
-                                                                        scale, phi)
+    if constexpr (N <= COLUMN_NX)                                                                                   \
+        return rf_launch<double2, N, 64, ixfft_columns_kernel<N, 64, 4>, 4>(h->stream, rf_row_blocks<N, 64>(d), d,  \
+                                                                            (const double2 *)h->hat,                \
+                                                                            (const double2 *)h->tw_x, d.ny * d.nz,  \
+                                                                            scale, phi);                            \
+    break
     RF_SIZES(d.nx, IX)
 #undef IX
     return hipErrorInvalidValue;

@@ -226,9 +226,10 @@ __global__ __launch_bounds__(FORM == 2 ? 2 * RB_THREADS : RB_THREADS) void rb_ld
     constexpr int TXP = rb_stride(sizeof(T) == 4, FORM == 2).row, PLANE = rb_stride(sizeof(T) == 4, FORM == 2).plane;
     constexpr int cw = TXP, cpl = PLANE;   // coefficient table: local i, j in [0, b+1]
     T *X = reinterpret_cast<T *>(smem_raw);
-    // unused slots of the per-thread cell lists point at a dummy cell past the tile, whose stencil
-    // reads and writes stay inside a padding of 2 planes + 3 values: the relax loops need no branches
-    // (the same cell in every workgroup, past the largest tile)
+    // Unused slots of the pair form's cell lists point at a dummy cell past the tile, whose stencil
+    // reads and writes stay inside a padding of 2 planes + 3 values, so its relax loops need no
+    // branches; the column forms mask absent cells off (colour()) and only mark them by it.  The
+    // same cell in every workgroup, past the largest tile.
     const int dummy = rb_dummy(PLANE, a.bz);
     T *C = X + dummy + PLANE + 2;   // IBM pair form: 6 planes of cpl values
                                        // (planes: threads read at pair stride)
@@ -426,8 +427,9 @@ __global__ __launch_bounds__(FORM == 2 ? 2 * RB_THREADS : RB_THREADS) void rb_ld
     // a wavefront of interior columns only (csplit), the rest of each colour reads no halo value
     // and sends none (colour 0 is at least 2 cells from every face, colour 1 at least 3), so it
     // relaxes while the halo exchange is in flight: colour 1's after the publish, the next
-    // iteration's colour 0 after that.  Cells past a range's end, and every cell of a thread
-    // without a column, go to the dummy cell.
+    // iteration's colour 0 after that.  A thread without a column has the dummy cell as its end
+    // cell and no rest; cells that are not there are masked off, and a wave without any skips the
+    // pass.
     int cb0 = dummy, cr0 = dummy, nr0 = 0;   // colour 0: end cell, first of the rest, their count
     int cb1 = dummy, cr1 = dummy, nr1 = 0;   // colour 1
     bool csplit = false;
@@ -539,13 +541,12 @@ __global__ __launch_bounds__(FORM == 2 ? 2 * RB_THREADS : RB_THREADS) void rb_ld
         }
     }
     // ---- exchange lists (built once per plan by rb_xlist_kernel): entry e = t + jj * NT
-    __shared__ int nbr_from[19];   // the workgroup that sends direction q's region to this one
+    __shared__ int nbr_from[18];   // the workgroup that sends direction q's region to this one
     if (t < 18) {
         int dx, dy, dz;
         rb_dir(t, dx, dy, dz);
         nbr_from[t] = neighbour(-dx, -dy, -dz);
     }
-    if (t == 18) nbr_from[18] = w;
     int xpub[HE], xdst[HE];
 #pragma unroll
     for (int jj = 0; jj < HE; ++jj) {
@@ -555,7 +556,8 @@ __global__ __launch_bounds__(FORM == 2 ? 2 * RB_THREADS : RB_THREADS) void rb_ld
     }
     bool failed = false;
     __syncthreads();
-    // per entry: whether it waits for a sender, the sender's word (of the even buffer) and the cell
+    // per entry: whether it waits for a sender, the sender's word (of the even buffer; of no use to an
+    // entry that does not wait) and the cell
     bool xwait[HE];
     unsigned xsrc[HE];
 #pragma unroll
@@ -971,9 +973,9 @@ __global__ __launch_bounds__(FORM == 2 ? 2 * RB_THREADS : RB_THREADS) void rb_ld
 // coordinate sum; cells 2k and 2k+1 of a region's natural order are neighbours along its first
 // extent above one, of opposite colours, and entry k of the region is the one of the two of
 // colour 1, on both sides alike.
-// Unused entries publish the dummy cell; an entry with no sender (beyond a wall, or past the end
-// of the list) does not wait, reads this workgroup's own slot (direction 18) and lands in the
-// dummy cell.  Built once per plan; the batch kernel only loads it.
+// An entry of the list without a cell to send publishes the dummy cell, one past the list's end is
+// not sent; an entry with no sender (beyond a wall, or past the end) neither loads nor stores.
+// Built once per plan; the batch kernel only loads it.
 struct RbGeom {
     int nx, ny, nz, px, py, pz, bx, by, bz, per_y, total, dummy;
     RbStride st;
@@ -995,7 +997,7 @@ __global__ __launch_bounds__(256) void rb_xlist_kernel(RbGeom g, int *xl) {
         const int ny_ = wy - dy;
         return g.per_y || (ny_ >= 0 && ny_ < g.py);
     };
-    int xpub = g.dummy, xdst = g.dummy | (18 << 20);
+    int xpub = g.dummy, xdst = g.dummy;
     if (e < g.total) {
         int q = 0, off = 0, ex = 0, ey = 0, ez = 0;
         for (; q < 18; ++q) {   // the regions start at the offsets of the largest subdomain

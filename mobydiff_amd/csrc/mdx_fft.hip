@@ -109,9 +109,10 @@ __device__ inline void stage_twiddles(C *dst, const C *__restrict__ tw, int n) {
 // loads and last stores are its own points, so no staging either.  LDS addresses are padded by one
 // element in 16, which keeps the radix-16 scatter (16 elements apart) and the gather (consecutive)
 // free of bank conflicts.  At 256 x 192 x 256 in FP64 the LDS kernels took 129 us (x, with the
-// right-hand side), 94 us (z, either way) and 89 us (x inverse); these take 99 (116 with u* not in a
-// cache), 41 (38 inverse) and 35 us, 4 to 5 TB/s of the fields and the spectrum read and written once.  In FP32: 49 us
-// (x), 62 (z) and 62 (x inverse, adding to phi) before, 25, 31 (24 inverse) and 40 now.
+// right-hand side), 94 us (z, either way) and 89 us (x inverse); these take 105, 43 (37 inverse) and
+// 36 us in a step: 3.9, 4.9 (5.7) and 5.8 TB/s by the counters, which see 1.02 to 1.04 times the fields
+// and the spectrum read and written once.  In FP32: 49 us (x), 62 (z) and 62 (x inverse, adding to phi)
+// before, 26, 32 (26 inverse) and 26 (to zero; 40 adding) now.
 template <typename C, bool INV> __device__ inline C ctw(C a, C w) {   // a w (forward) or a conj(w)
     const typename Cx<C>::R wi = INV ? -w.y : w.y;
     return Cx<C>::mk(a.x * w.x - a.y * wi, a.x * wi + a.y * w.x);

@@ -375,9 +375,9 @@ static constexpr unsigned PROJ_GHOST_BLOCKS = 256;
 // rows below, the pair to the east and the row above, two planes below and one above are recomputed
 // by every workgroup that needs them, from the same inputs: bit-identical to the one-colour sweeps.
 // x and z periodic, Dirichlet v on the y walls (or periodic y, ny even), z-invariant coefficients
-// or none.  200^3, three iterations: 1314 us of sweeps and 77 us of copies -> 480 us (3.1 TB/s of the
-// 64 B per cell and iteration; a plane's two barriers and FP64 chain leave the CUs' one or two
-// workgroups waiting, and 200 VGPRs allow no more).  32 x 24 x 16: 42 -> 21 us.
+// or none.  200^3, three iterations: 1314 us of sweeps and 77 us of copies -> 480 us (3.2 TB/s of the
+// 64 B per cell and iteration, 3.6 of the 585 MB that the counters see; a plane's two barriers and
+// FP64 chain leave the CUs' one or two workgroups waiting, and 200 VGPRs allow no more).  32 x 24 x 16: 42 -> 21 us.
 // last: 0 an iteration whose result another one reads, 1 the last one (its ghost blocks fill the
 // ghost shell of un, vn, wn with u*'s values), 2 the last one inside a step: it also writes the
 // boundary conditions (as sor_apply_kernel with BC).
